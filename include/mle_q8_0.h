@@ -68,11 +68,12 @@ int mle_q8_0_abi_version(void);
  *
  * Paths: M == 1, M <= 4 with K <= 1024 and N <= 32768, and M == 2 with
  * 2048 <= K <= 4096 and N <= 32768, run the FP32 decode GEMV; other
- * M < 64 run the MFMA decode kernel in chunks of up to 16 tokens (FP32
- * activations split exactly into three bf16 parts, so it matches FP32 to about
+ * M < 64 run MFMA decode kernels (up to 16 tokens, and 17-63 in one launch; FP32
+ * activations split exactly into three bf16 parts, so they match FP32 to about
  * 1e-7 relative L2);
- * M >= 64 runs the bf16-MFMA prefill GEMM (relative L2 error vs FP32 about
- * 2e-3).  Both MFMA paths may split K over workgroups and reduce the partials
+ * M >= 64 rounds both operands to bf16 (relative L2 error vs FP32 about 2e-3):
+ * the batch kernel of 17-63 tokens up to 128 on fewer rows, else the prefill GEMM.
+ * The MFMA paths may split K over workgroups and reduce the partials
  * in a fixed order, so results are deterministic run to run.
  * Errors: NULL x/w/y -> InvalidArgument; M, N or K <= 0 -> InvalidArgument;
  * K % 32 != 0 -> Unsupported ("... requires K to be a multiple of 32").
@@ -121,7 +122,7 @@ int mle_q8_0_linear_swiglu(const float* x, const uint8_t* w_gate, const uint8_t*
  * (src/model/transformer_graph_builder.cpp:214-221).  `bias` may be NULL (no
  * bias anywhere) or hold NULL entries.  For M < 64 each output is bit-identical
  * to mle_q8_0_linear on the same operands (same kernel arithmetic); M >= 64
- * takes the bf16 MFMA GEMM with a tile choice of its own.
+ * takes the bf16 paths with a tile choice of its own.
  * Errors: count outside 1..3 or NULL w / y / N arrays -> InvalidArgument; each
  * output is validated as mle_q8_0_linear validates its operands.
  */

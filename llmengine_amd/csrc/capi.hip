@@ -276,6 +276,47 @@ struct Tune {
   mle::GemmConfig gemm{0, 0, 0};  // 0 fields = automatic
 };
 
+// Whether the graph workspace of (current device, stream) holds `need`.
+bool graph_workspace_holds(const mle::SplitKNeed& need, hipStream_t stream) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return false;
+  std::lock_guard<std::mutex> lock(g_ws_mu);
+  const auto it = g_ws.find({dev, stream, true});
+  return it != g_ws.end() && it->second.buf_cap >= need_bytes(need) &&
+         it->second.counter_cap >= need.counters;
+}
+
+// The launches of linear_mid.hip (mle::linear_mid_pick).  Returns whether the call
+// was one, with its status in *rc.  `general` is what the general path's launches
+// need: a plan names the larger of both, so a workspace sized for a batch serves the
+// smaller steps that take the general path.  Where the K splits' partials do not fit
+// (a caller-fixed workspace, or a captured stream's reservation made for the general
+// path) the launch runs unsplit, which needs no workspace.
+bool run_mid(const char* what, const float* x, const mle::LinearSegs& s, int M, int K,
+             const mle::SplitKNeed& general, const Exec& ex, int* rc) {
+  mle::MidConfig c = mle::linear_mid_pick(M, s, K);
+  if (c.tt == 0 || !mle::linear_mid_fits(M, K)) return false;
+  mle::SplitKNeed need = mle::linear_mid_workspace(c, s, K);
+  const bool short_of_space =
+      need.partial_floats != 0 &&
+      (ex.fixed ? need_bytes(need) > ex.fixed_bytes || need.counters > ex.fixed_counter_count
+                : !ex.planning() && stream_capturing(ex.stream) &&
+                      !graph_workspace_holds(need, ex.stream));
+  if (short_of_space) {
+    c.splits = 1;
+    need = mle::linear_mid_workspace(c, s, K);
+  }
+  mle::SplitKWorkspace ws;
+  std::unique_lock<std::mutex> hold;  // released after the launch is enqueued
+  if (ex.planning()) (void)workspace_for(general, ex, &ws, &hold);
+  *rc = workspace_for(need, ex, &ws, &hold);
+  if (*rc == MLE_OK)
+    *rc = check_launch(ex.planning() ? hipSuccess
+                                     : mle::launch_linear_mid(c, x, s, M, K, ws, ex.stream),
+                       what);
+  return true;
+}
+
 // Tiled weights (mle::WeightLayout::kTiled): the tiled FP32 GEMV where
 // mle::gemv_tiled_wins (one token; two below vocabulary-sized outputs; up to
 // four on short rows), else the MFMA decode below 64 tokens and the MFMA GEMM
@@ -284,6 +325,7 @@ int run_linear(const float* x, const uint8_t* w, const void* bias, float* y, int
                int N, int K, int path, const Tune& tune, const Exec& ex,
                mle::WeightLayout layout = mle::WeightLayout::kRaw, bool bias_bf16 = false) {
   const bool tiled = layout == mle::WeightLayout::kTiled;
+  const bool automatic = path == 0;
   if (path == 0) {
     path = tiled ? (M >= 64 ? 2 : 3) : pick_path(M, N, K);
     const int mc = M < 16 ? M : 16;
@@ -297,6 +339,12 @@ int run_linear(const float* x, const uint8_t* w, const void* bias, float* y, int
   one.seg[0] = mle::LinearSeg{w, bias, y, N};
   one.seg[0].bias_bf16 = bias_bf16 ? 1 : 0;
   one.layout = layout;
+  const char* const what = "hip sgemm_nt Q8_0 launch failed";
+  int rc = MLE_OK;
+  if (automatic && path == 3) {
+    const mle::DecodeMfmaConfig c = mle::decode_mfma_pick(M < 16 ? M : 16, N, K, layout);
+    if (run_mid(what, x, one, M, K, mle::decode_mfma_workspace_segs(c, one, K), ex, &rc)) return rc;
+  }
   if (tiled && path == 3 && tune.dec.mt == 0 && M <= 4 && mle::gemv_tiled_wins(M, N, K)) {
     const mle::TiledGemvConfig c = mle::gemv_tiled_pick(M, N, K, false);
     return check_launch((ex.planning() ? hipSuccess : mle::launch_gemv_tiled_segs(c, x, one, M, K, ex.stream)),
@@ -316,6 +364,8 @@ int run_linear(const float* x, const uint8_t* w, const void* bias, float* y, int
                                             std::to_string(c.bn) + ")");
     if (!mle::gemm_mfma_fits(c, M, N, K))
       return fail(MLE_UNSUPPORTED, "hip sgemm_nt Q8_0: K too large for the MFMA GEMM");
+    if (automatic && run_mid(what, x, one, M, K, mle::gemm_mfma_workspace(c, M, N, K), ex, &rc))
+      return rc;
     mle::SplitKWorkspace ws;
     std::unique_lock<std::mutex> hold;  // released after the launch is enqueued
     MLE_TRY(workspace_for(mle::gemm_mfma_workspace(c, M, N, K), ex, &ws, &hold));
@@ -375,10 +425,13 @@ int run_segs(const char* ctx, const float* x, const mle::LinearSegs& s, int M, i
   const bool swi = s.mode == mle::Epilogue::kSwiGLU;
   int total_n = 0;
   for (int i = 0; i < s.count; ++i) total_n += s.seg[i].N;
+  const char* const what = "hip Q8_0 fused Linear launch failed";
+  int rc = MLE_OK;
   if (M >= 64) {
     const mle::GemmConfig c = mle::gemm_mfma_pick_segs(M, s, K);
     if (!mle::gemm_mfma_fits(c, M, 0, K))
       return fail(MLE_UNSUPPORTED, std::string("hip ") + ctx + ": K too large for the MFMA GEMM");
+    if (run_mid(what, x, s, M, K, mle::gemm_mfma_workspace_segs(c, M, s, K), ex, &rc)) return rc;
     mle::SplitKWorkspace ws;
     std::unique_lock<std::mutex> hold;  // released after the launch is enqueued
     MLE_TRY(workspace_for(mle::gemm_mfma_workspace_segs(c, M, s, K), ex, &ws, &hold));
@@ -398,6 +451,11 @@ int run_segs(const char* ctx, const float* x, const mle::LinearSegs& s, int M, i
     return check_launch((ex.planning() ? hipSuccess : mle::launch_gemv_segs(c, x, s, M, K, ex.stream)),
                         "hip Q8_0 fused Linear launch failed");
   }
+  const int m16 = M < 16 ? M : 16;
+  const mle::DecodeMfmaConfig c16 = mle::decode_mfma_pick_segs(m16, s, K);
+  if (mle::decode_mfma_fits(c16, m16, 1, K) &&
+      run_mid(what, x, s, M, K, mle::decode_mfma_workspace_segs(c16, s, K), ex, &rc))
+    return rc;
   for (int m0 = 0; m0 < M; m0 += 16) {
     const int mc = M - m0 < 16 ? M - m0 : 16;
     const mle::DecodeMfmaConfig c = mle::decode_mfma_pick_segs(mc, s, K);
@@ -689,6 +747,9 @@ int mle_q8_0_linear_noalloc(const float* x, const uint8_t* w_q8_0, const float* 
     Exec plan;
     plan.plan_bytes = &bytes;
     plan.plan_counters = &counters;
+    plan.fixed = true;  // the launches' choices as on the scratch below
+    plan.fixed_bytes = kNoAllocBytes;
+    plan.fixed_counter_count = kNoAllocCounters;
     MLE_TRY(run_linear(x, w_q8_0, bias, y, M, N, K, 0, Tune{}, plan));
   }
   if (bytes > kNoAllocBytes || counters > kNoAllocCounters)
@@ -701,13 +762,13 @@ int mle_q8_0_linear_noalloc(const float* x, const uint8_t* w_q8_0, const float* 
   Exec ex;
   ex.stream = stream;
   ex.fixed = true;  // launches needing no workspace get none
+  ex.fixed_bytes = kNoAllocBytes;
+  ex.fixed_counter_count = kNoAllocCounters;
   if (bytes != 0 || counters != 0) {
     uint8_t* base = nullptr;
     MLE_TRY(noalloc_scratch(stream, &base));
     ex.fixed_buf = base;
-    ex.fixed_bytes = kNoAllocBytes;
     ex.fixed_counters = reinterpret_cast<uint32_t*>(base + kNoAllocBytes);
-    ex.fixed_counter_count = kNoAllocCounters;
   }
   return run_linear(x, w_q8_0, bias, y, M, N, K, 0, Tune{}, ex);
 }

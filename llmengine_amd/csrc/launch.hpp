@@ -138,6 +138,20 @@ hipError_t launch_gemv_mfma_segs(const DecodeMfmaConfig& c, const float* x,
                                  const LinearSegs& s, int M, int K, const SplitKWorkspace& ws,
                                  hipStream_t stream);
 
+// Linear of a serving batch or a short prompt (9-128 tokens): 64 rg weight rows per
+// workgroup, all tokens (tt tiles of 16), `splits` K splits.
+struct MidConfig {
+  int tt = 0;      // token tiles of 16 (16 tt >= M); 0: the launch is not this kernel's
+  int parts = 3;   // bf16 parts per activation: 3 (FP32-exact) or 1 (rounded once)
+  int rg = 1;      // 16-row groups per wave (SwiGLU: even, half of each weight)
+  int splits = 1;  // K splits asked for
+};
+MidConfig linear_mid_pick(int M, const LinearSegs& s, int K);
+bool linear_mid_fits(int M, int K);
+SplitKNeed linear_mid_workspace(const MidConfig& c, const LinearSegs& s, int K);
+hipError_t launch_linear_mid(const MidConfig& c, const float* x, const LinearSegs& s, int M, int K,
+                             const SplitKWorkspace& ws, hipStream_t stream);
+
 // Linear GEMM on bf16 MFMA (prefill): same contract as launch_gemv, any M.
 // X is first converted to bf16 into the workspace scratch; `splits` K splits
 // (1 = none) meet in the split-K partials.

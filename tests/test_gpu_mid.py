@@ -1,0 +1,179 @@
+"""GPU parity of the Linear for 9-128 tokens (linear_mid.hip).
+
+Raw and tiled weights (the same bits: same products, same order) against the CPU oracle
+(cpu_kernels.cpp:208-218), against the general paths that the tuning hook forces (the
+16-token MFMA decode below 64 tokens, the bf16 GEMM from 64), and against themselves.
+Shapes: token tiles and their remainders, single rows, ragged row groups, one block, an
+odd number of blocks, phases of 1-4 blocks, 1 / 2 / 4 / 8 K splits.  Bars: 1e-5 (fp32
+sums) below 64 tokens and 1e-6 against the decode (the same exact block products grouped
+differently); 1e-2 from 64 tokens (both operands rounded once to bf16).
+"""
+import numpy as np
+import pytest
+
+from helpers import assert_bitexact, empty_f32, note, rel_l2, to_dev, to_host
+from llmengine_amd import capi
+from llmengine_amd import synthetic as S
+
+pytestmark = pytest.mark.gpu
+
+
+def weight(seed, N, K):
+    return S.q8_0_weight(seed, N, K)[0]
+
+
+def tiled_dev(dw, N, K, dev):
+    import torch
+    t = torch.empty(capi.tiled_bytes(N, K), dtype=torch.uint8, device=dev)
+    capi.tile(dw, t, N, K)
+    return t
+
+
+def tol(M):
+    return 1e-5 if M < 64 else 1e-2
+
+
+@pytest.mark.parametrize("M,N,K,bias", [
+    (9, 100, 32, "f32"), (16, 65, 1024, None), (12, 300, 992, None),
+    (17, 1, 96, "bf16"), (31, 63, 256, None), (32, 64, 288, "f32"), (33, 257, 512, "bf16"),
+    (48, 129, 544, None), (49, 1000, 4096, "f32"), (63, 640, 4128, None),
+    (63, 16384 + 5, 256, None), (40, 50000, 96, None),
+    (64, 100, 32, "bf16"), (65, 513, 1056, None), (80, 300, 4160, "f32"), (81, 77, 288, None),
+    (96, 4864, 224, "bf16"), (97, 1024, 2048, None), (128, 4096, 160, "f32"),
+    (128, 96, 8192, None)])
+def test_mid_linear(dev, orc, M, N, K, bias):
+    import torch
+    note(f"mid linear M={M} N={N} K={K} bias={bias}")
+    raw = weight(900 + N % 97, N, K)
+    x = S.activations(901 + M, (M, K))
+    b32 = S.activations(902, (N,), tag=S.TAG_BIAS)
+    b16 = (b32.view(np.uint32) >> 16).astype(np.uint16)
+    if bias == "bf16":
+        b32 = (b16.astype(np.uint32) << 16).view(np.float32)
+    dx, dw = to_dev(x, dev), to_dev(raw, dev)
+    dt = tiled_dev(dw, N, K, dev)
+    db = {None: None, "f32": to_dev(b32, dev), "bf16": to_dev(b16.view(np.int16), dev)}[bias]
+    y = [empty_f32((M, N), dev) for _ in range(4)]
+    for out, w, tiled in ((y[0], dw, False), (y[1], dt, True), (y[2], dt, True)):
+        if bias == "bf16":
+            capi.linear_bias_bf16(dx, w, db, out, M, N, K, tiled=tiled)
+        else:
+            (capi.linear_tiled if tiled else capi.linear)(dx, w, db, out, M, N, K)
+    general = to_dev(b32, dev) if bias else None
+    capi.linear_ex(dx, dw, general, y[3], M, N, K, path=3 if M < 64 else 2)
+    torch.cuda.synchronize()
+    got = to_host(y[0])
+    assert_bitexact(to_host(y[1]), got, "tiled vs raw")
+    assert torch.equal(y[1], y[2])
+    assert rel_l2(got, to_host(y[3])) <= (1e-6 if M < 64 else 1e-2)
+    rows = np.unique(np.linspace(0, N - 1, min(N, 200)).astype(int))
+    w_rows = np.ascontiguousarray(raw.reshape(N, -1)[rows]).reshape(-1)
+    want = orc.linear(x, w_rows, b32[rows] if bias else None, M, rows.size, K)
+    assert rel_l2(got[:, rows], want) <= tol(M)
+
+
+@pytest.mark.parametrize("M,Ns,K", [(20, (70, 33, 1), 512), (63, (4096, 128, 128), 896),
+                                    (13, (500, 20, 20), 736), (77, (1024, 40, 300), 2080)])
+def test_mid_multi(dev, orc, M, Ns, K):
+    """Segment boundaries inside a wave's row groups; below 64 tokens each output has the
+    single Linear's bits."""
+    note(f"mid multi M={M} Ns={Ns} K={K}")
+    ws = [weight(910 + i, n, K) for i, n in enumerate(Ns)]
+    bs = [S.activations(911, (Ns[0],), tag=S.TAG_BIAS), None,
+          S.activations(912, (Ns[2],), tag=S.TAG_BIAS)]
+    x = S.activations(913, (M, K))
+    dx, dws = to_dev(x, dev), [to_dev(w, dev) for w in ws]
+    dbs = [None if b is None else to_dev(b, dev) for b in bs]
+    dts = [tiled_dev(w, n, K, dev) for w, n in zip(dws, Ns)]
+    yr, yt = ([empty_f32((M, n), dev) for n in Ns] for _ in range(2))
+    capi.linear_multi(dx, dws, dbs, yr, Ns, M, K)
+    capi.linear_multi_tiled(dx, dts, dbs, yt, Ns, M, K)
+    for i, n in enumerate(Ns):
+        got = to_host(yr[i])
+        assert_bitexact(to_host(yt[i]), got, f"tiled vs raw {i}")
+        assert rel_l2(got, orc.linear(x, ws[i], bs[i], M, n, K)) <= tol(M)
+        if M < 64:
+            single = empty_f32((M, n), dev)
+            capi.linear(dx, dws[i], dbs[i], single, M, n, K)
+            assert_bitexact(to_host(single), got, f"single vs fused {i}")
+
+
+@pytest.mark.parametrize("M,N,K", [(17, 50, 64), (40, 1111, 4096), (63, 8000, 544),
+                                   (48, 11008, 1056), (10, 300, 992)])
+def test_mid_swiglu(dev, orc, M, N, K):
+    note(f"mid swiglu M={M} N={N} K={K}")
+    wg, wu = weight(920, N, K), weight(921, N, K)
+    x = S.activations(922, (M, K))
+    dx, dg, du = to_dev(x, dev), to_dev(wg, dev), to_dev(wu, dev)
+    yr, yt = empty_f32((M, N), dev), empty_f32((M, N), dev)
+    capi.linear_swiglu(dx, dg, du, yr, M, N, K)
+    capi.linear_swiglu_tiled(dx, tiled_dev(dg, N, K, dev), tiled_dev(du, N, K, dev), yt, M, N, K)
+    got = to_host(yr)
+    assert_bitexact(to_host(yt), got, "tiled vs raw")
+    rows = np.unique(np.linspace(0, N - 1, min(N, 200)).astype(int))
+    cut = [np.ascontiguousarray(w.reshape(N, -1)[rows]).reshape(-1) for w in (wg, wu)]
+    g, u = (orc.sgemm_nt(x, w, M, rows.size, K).astype(np.float64) for w in cut)
+    assert rel_l2(got[:, rows], g / (1.0 + np.exp(-g)) * u) <= tol(M)
+
+
+@pytest.mark.parametrize("M", [24, 70])
+def test_mid_special_values(dev, M):
+    """Inf, NaN, zero rows and the largest magnitudes give the general path's non-finite
+    entries and its finite values, on both layouts; other tokens are untouched."""
+    N, K = 96, 1056
+    raw = weight(930, N, K)
+    x = S.activations(931, (M, K))
+    x[1, 5], x[2, 100], x[3, 7], x[4, :], x[5, 3] = np.inf, -np.inf, np.nan, 0.0, 3.0e38
+    note(f"mid special values M={M}")
+    dx, dw = to_dev(x, dev), to_dev(raw, dev)
+    y, yt, yg = (empty_f32((M, N), dev) for _ in range(3))
+    capi.linear(dx, dw, None, y, M, N, K)
+    capi.linear_tiled(dx, tiled_dev(dw, N, K, dev), None, yt, M, N, K)
+    capi.linear_ex(dx, dw, None, yg, M, N, K, path=3 if M < 64 else 2)
+    got, want = to_host(y), to_host(yg)
+    assert_bitexact(to_host(yt), got, "tiled vs raw")
+    fin = np.isfinite(want)
+    assert np.array_equal(np.isfinite(got), fin) and not fin[1:4].all() and fin[6:].all()
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    inf = np.isinf(want)
+    assert np.array_equal(got[inf], want[inf])
+    ok = fin.copy()
+    ok[5] = False  # 3e38 products: the sum's order decides what overflows
+    assert rel_l2(got[ok], want[ok]) <= (1e-6 if M < 64 else 1e-2)
+
+
+def test_mid_split_counters_and_noalloc(dev):
+    """Launches of different split counts back to back on one stream leave the counters
+    clean, and the no-allocation entry point gives the same bits."""
+    import torch
+    note("mid split counters")
+    x = to_dev(S.activations(940, (63, 8256)), dev)
+    for N, K in ((200, 8256), (700, 512), (64, 4096), (200, 8256)):
+        dw = to_dev(weight(941, N, K), dev)
+        y, y2 = empty_f32((63, N), dev), empty_f32((63, N), dev)
+        capi.linear(x, dw, None, y, 63, N, K)
+        capi.linear_noalloc(x, dw, None, y2, 63, N, K)
+        torch.cuda.synchronize()
+        assert torch.equal(y, y2) and bool(torch.isfinite(y).all())
+
+
+def test_mid_capture_on_a_smaller_reservation(dev):
+    """A stream whose graph workspace was reserved for 16 tokens still captures 40: the
+    launch runs unsplit there, with fp32 rounding between it and the eager call."""
+    import torch
+    M, N, K = 40, 4096, 8192  # 5.5 MB of partials; a reservation holds at least 4 MiB
+    note("mid capture on a smaller reservation")
+    x, dw = to_dev(S.activations(950, (M, K)), dev), to_dev(weight(951, N, K), dev)
+    y, eager = empty_f32((M, N), dev), empty_f32((M, N), dev)
+    st = torch.cuda.Stream()
+    capi.workspace_reserve(1, 1, stream=st)
+    capi.linear(x, dw, None, eager, M, N, K, stream=st)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=st):
+        capi.linear(x, dw, None, y, M, N, K, stream=st)
+    for _ in range(3):
+        y.fill_(float("nan"))
+        g.replay()
+        torch.cuda.synchronize()
+        assert rel_l2(to_host(y), to_host(eager)) <= 1e-6
