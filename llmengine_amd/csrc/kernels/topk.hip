@@ -13,31 +13,52 @@
 // the reference leaves the order of equal probabilities to std::partial_sort,
 // the order here is the logit, then the index.
 //
-// Two launches.  Pass 1 (grid chunks x rows, 256 threads): a workgroup reads a
-// 2048-value chunk once, forms 64-bit keys (order(value) << 32 | ~index: the
-// largest key is the largest value with the smallest index) and keeps its
-// top_n keys, plus the chunk's maximum, its sum of exp(value - maximum) and a
-// NaN flag.  Pass 2 (one 1024-thread workgroup per row): merges the chunk
-// statistics in a fixed order (max, then the sum of sum_c * exp(max_c - max)),
-// selects the top_n of the chunks' candidate keys and writes ids and
-// probabilities.
+// Two launches.  Pass 1 (grid chunks x rows, 256 threads) streams a 2048-value chunk:
+// its maximum, its sum of exp(value - maximum), a NaN flag, and the maxima of its
+// groups of 64 values (1024 / top_n for fewer than 16 tokens, so that the workspace
+// stays within 2 top_n floats a chunk).  Pass 2 (one 1024-thread workgroup per row)
+// merges the chunk statistics in a fixed order (max, then the sum of sum_c *
+// exp(max_c - max)) and works on whole groups: the top_n tokens lie in the top_n
+// groups of largest maximum (ties to the lower group), so it picks groups, re-reads
+// only their values and picks among those.
+//   * Groups: one histogram over the distance of the group maxima from the row's
+//     maximum, in floating-point bins (5 mantissa bits), gives a distance within which
+//     at least top_n groups lie; usually a few more do, all of them are taken.  Where
+//     that is too many values (massive ties), the exact top_n groups are selected.
+//   * Values within that distance are ranked by counting the larger keys (64-bit:
+//     order(value) << 32 | ~index, all distinct); more than 256 go through the
+//     radix select.
+// Selection (exact): a radix select over the keys' upper 32 bits (four 8-bit digit
+// histograms in LDS, most significant first) finds the top_n-th largest value T; the
+// keys >= T (T's ties included) are gathered and sorted by one wave in registers
+// (bitonic network, lane shuffles, no barriers), and the first top_n are the result.
+// If more than 256 keys reach T the whole set is sorted in LDS instead.  Results are
+// deterministic: the keys are distinct, so neither the ranks nor the sorted order
+// depend on the order of gathering.
 //
-// Selection (both passes): a radix select over the keys' upper 32 bits (four
-// 8-bit digit histograms in LDS, most significant first) finds the top_n-th
-// largest value T; the keys >= T (T's ties included) are gathered and sorted by
-// one wave in registers (bitonic network, lane shuffles, no barriers), and the
-// first top_n are the result.  If more than 256 keys reach T (massive ties) the
-// whole set is sorted in LDS instead.  Results are deterministic: the keys are
-// distinct, so the sorted order does not depend on the order of gathering.
+// Latency bounds it, not bytes (8 rows x 152k logits are 4.9 MB).  Selecting top_n keys
+// in every chunk instead (a radix select per chunk, then one over 75 x top_n
+// candidates) took 31.7 us for 8 rows at top_n 40 and 28.5 for one (MI355X); this
+// takes 13.5 and 12.8.
 #include "../launch.hpp"
 
 namespace mle {
 namespace {
 
 constexpr int kChunk = 2048;           // values per pass-1 workgroup
+constexpr int kGroup = 64;             // values per group (top_n >= 16)
 constexpr int kP1Threads = 256;
 constexpr int kP2Threads = 1024;
-constexpr int kP2Keys = 16384;         // candidate keys a row can merge (128 KB of LDS)
+constexpr int kP2Keys = 16384;         // values of the picked groups (128 KB of LDS)
+constexpr int kP2Groups = 8192;        // groups of a row that pass 2 picks from
+constexpr int kBins = 8192;            // distance bins: 8 exponent and 5 mantissa bits
+
+// Group maxima a pass-1 chunk writes for top k: at most 2 k, whole powers of two.
+__host__ __device__ constexpr int chunk_groups(int k) {
+  int c = kChunk / kGroup;
+  while (c > 2 * k) c >>= 1;
+  return c;
+}
 
 __device__ __forceinline__ uint64_t topk_key(float v, uint32_t i) {
   if (v != v) return 0;      // NaN (the row becomes uniform anyway)
@@ -215,112 +236,244 @@ __device__ void select_top(const uint64_t (&key)[E], int k, uint64_t* __restrict
   __syncthreads();
 }
 
+// Distance bin of a value below the row's finite maximum (0: at it).
+__device__ __forceinline__ uint32_t dist_bin(float mx, float v) {
+  return __builtin_bit_cast(uint32_t, mx - v) >> 18;  // mx >= v: sign clear, +Inf bin 8160
+}
+
 // Pass 1: workgroup (c, r) over logits[r, c * kChunk : (c + 1) * kChunk).
-// keys: [row][chunk][k]; stats: [row][chunk] x {max, sum, nan, 0}.
+// maxima: [row][chunk][gpc] group maxima; stats: [row][chunk] x {max, sum, nan, rest of
+// the sum}.
 __global__ __launch_bounds__(kP1Threads) void topk_chunks_kernel(
-    const float* __restrict__ x, int64_t n, int k, float inv_temp, int scale,
-    uint64_t* __restrict__ keys, float* __restrict__ stats) {
-  __shared__ uint64_t s[kChunk];  // only for massive ties
-  __shared__ SelectLds sm;
-  __shared__ uint64_t top[kTopTokensMax];
+    const float* __restrict__ x, int64_t n, int gpc, float inv_temp, int scale,
+    float* __restrict__ maxima, float* __restrict__ stats) {
+  __shared__ float gmax[kChunk / kGroup];
   __shared__ float fpart[kP1Threads / 64];
+  __shared__ double dpart[kP1Threads / 64];
   __shared__ int ipart[kP1Threads / 64];
+  typedef float f4 __attribute__((ext_vector_type(4), aligned(4)));  // rows are 4-byte aligned
   const int64_t r = blockIdx.y;
   const int64_t b = (int64_t)blockIdx.x * kChunk;
   const float* row = x + r * n;
-  constexpr int PER = kChunk / kP1Threads;
+  constexpr int PER = kChunk / kP1Threads, Q = PER / 4;
+  static_assert(kGroup == 64, "16 lanes x 4 values are a group");
   float v[PER];
-  uint64_t key[PER];
   float mx = -__builtin_inff();
   int nan = 0;
 #pragma unroll
-  for (int j = 0; j < PER; ++j) {
-    const int64_t i = b + threadIdx.x + kP1Threads * j;
-    float t = -__builtin_inff();
-    key[j] = 0;
-    if (i < n) {
-      t = row[i];
-      if (scale) t *= inv_temp;
-      key[j] = topk_key(t, (uint32_t)i);
-      nan |= t != t;
-      mx = fmaxf(mx, t);  // ignores NaN
+  for (int j = 0; j < Q; ++j) {
+    const int64_t i = b + 4 * ((int)threadIdx.x + kP1Threads * j);
+    f4 t = {-__builtin_inff(), -__builtin_inff(), -__builtin_inff(), -__builtin_inff()};
+    if (i + 4 <= n) {
+      t = *reinterpret_cast<const f4*>(row + i);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (i + e < n) t[e] = row[i + e];
     }
-    v[j] = t;
+    float g = -__builtin_inff();
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float u = scale && i + e < n ? t[e] * inv_temp : t[e];
+      v[4 * j + e] = u;
+      nan |= u != u;
+      g = fmaxf(g, u);  // ignores NaN
+    }
+#pragma unroll
+    for (int off = 8; off > 0; off >>= 1) g = fmaxf(g, __shfl_xor(g, off, 64));
+    if ((threadIdx.x & 15) == 0) gmax[threadIdx.x / 16 + kP1Threads / 16 * j] = g;
+    mx = fmaxf(mx, g);
   }
   mx = block_reduce<kP1Threads>(mx, [](float a, float c) { return fmaxf(a, c); }, fpart);
   nan = block_reduce<kP1Threads>(nan, [](int a, int c) { return a | c; }, ipart);
-  float sum = 0.0f;
+  double sum = 0.0;  // one chunk can hold most of the row's sum: its rounding is the row's
   if (mx > -__builtin_inff() && mx < __builtin_inff()) {
 #pragma unroll
     for (int j = 0; j < PER; ++j)
       if (v[j] == v[j]) sum += expf(v[j] - mx);
   }
-  sum = block_reduce<kP1Threads>(sum, [](float a, float c) { return a + c; }, fpart);
-  select_top<kP1Threads, PER>(key, k, top, sm, s);
+  sum = block_reduce<kP1Threads>(sum, [](double a, double c) { return a + c; }, dpart);
   const int64_t slot = r * gridDim.x + blockIdx.x;
-  for (int j = threadIdx.x; j < k; j += kP1Threads) keys[slot * k + j] = top[j];
+  if ((int)threadIdx.x < gpc) {
+    const int f = kChunk / kGroup / gpc;  // 64-value groups per written maximum
+    float g = gmax[threadIdx.x * f];
+    for (int i = 1; i < f; ++i) g = fmaxf(g, gmax[threadIdx.x * f + i]);
+    maxima[slot * gpc + threadIdx.x] = g;
+  }
   if (threadIdx.x == 0) {
     stats[slot * 4 + 0] = mx;
-    stats[slot * 4 + 1] = sum;
+    stats[slot * 4 + 1] = (float)sum;
     stats[slot * 4 + 2] = nan ? 1.0f : 0.0f;
-    stats[slot * 4 + 3] = 0.0f;
+    stats[slot * 4 + 3] = (float)(sum - (float)sum);
   }
 }
 
-// Pass 2: one workgroup per row over its chunks' statistics and candidates.
+// Pass 2: one workgroup per row over its chunks' statistics and group maxima.  A group
+// here is `gm` consecutive written maxima (a power of two; 1 up to kP2Groups maxima),
+// 2^gshift values; the kk groups' values fit kP2Keys for every accepted n.
 __global__ __launch_bounds__(kP2Threads) void topk_final_kernel(
-    const uint64_t* __restrict__ keys, const float* __restrict__ stats, int chunks, int k,
-    int64_t n, int kk, int32_t* __restrict__ ids, float* __restrict__ probs) {
-  __shared__ uint64_t s[kP2Keys];  // only for massive ties
+    const float* __restrict__ x, const float* __restrict__ maxima,
+    const float* __restrict__ stats, int chunks, int gpc, int gm, int gshift, int64_t n, int kk,
+    float inv_temp, int scale, int32_t* __restrict__ ids, float* __restrict__ probs) {
+  __shared__ __attribute__((aligned(16))) uint64_t s[kP2Keys];  // bins, then massive ties
   __shared__ SelectLds sm;
   __shared__ uint64_t top[kTopTokensMax];
+  __shared__ int list[kP2Keys / kGroup];
   __shared__ float fpart[kP2Threads / 64];
+  __shared__ double dpart[kP2Threads / 64];
   __shared__ int ipart[kP2Threads / 64];
+  __shared__ uint32_t wsum[kP2Threads / 64];
+  __shared__ uint32_t bin_at, groups_in, nlist;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int64_t r = blockIdx.x;
   const float* st = stats + r * chunks * 4;
+  uint32_t* const hist = reinterpret_cast<uint32_t*>(s);
+  // The group maxima first: nothing below waits for more than they do.
+  constexpr int GPT = kP2Groups / kP2Threads;
+  const int total_max = chunks * gpc;  // per row
+  const int groups = (int)((n + ((int64_t)1 << gshift) - 1) >> gshift);
+  const float* mrow = maxima + r * (int64_t)total_max;
+  float gv[GPT];
+#pragma unroll
+  for (int e = 0; e < GPT; ++e) {
+    const int gi = tid + kP2Threads * e;
+    float g = -__builtin_inff();
+    if (gi < groups)
+      for (int j = 0; j < gm && gi * gm + j < total_max; ++j) g = fmaxf(g, mrow[gi * gm + j]);
+    gv[e] = g;
+  }
   float mx = -__builtin_inff();
   int bad = 0;
-  for (int c = threadIdx.x; c < chunks; c += kP2Threads) {
+  for (int c = tid; c < chunks; c += kP2Threads) {
     mx = fmaxf(mx, st[c * 4 + 0]);
     bad |= st[c * 4 + 2] != 0.0f;
   }
+  for (int i = tid; i < kBins / 4; i += kP2Threads)
+    reinterpret_cast<uint4*>(hist)[i] = uint4{0u, 0u, 0u, 0u};
+  if (tid == 0) {
+    bin_at = kBins - 1;
+    groups_in = (uint32_t)groups;
+    nlist = 0;
+    sm.ncand = 0;
+  }
   mx = block_reduce<kP2Threads>(mx, [](float a, float c) { return fmaxf(a, c); }, fpart);
   bad = block_reduce<kP2Threads>(bad, [](int a, int c) { return a | c; }, ipart);
-  float sum = 0.0f;
+  double sum = 0.0;
   const bool finite_max = mx > -__builtin_inff() && mx < __builtin_inff();
   if (finite_max) {
-    for (int c = threadIdx.x; c < chunks; c += kP2Threads) {
+    for (int c = tid; c < chunks; c += kP2Threads) {
       const float mc = st[c * 4 + 0];
-      if (mc > -__builtin_inff()) sum += st[c * 4 + 1] * expf(mc - mx);
+      if (mc > -__builtin_inff()) sum += ((double)st[c * 4 + 1] + st[c * 4 + 3]) * exp((double)mc - (double)mx);
     }
   }
-  sum = block_reduce<kP2Threads>(sum, [](float a, float c) { return a + c; }, fpart);
-  const bool uniform = bad || !finite_max || !(sum > 0.0f) || !(sum < __builtin_inff());
+  sum = block_reduce<kP2Threads>(sum, [](double a, double c) { return a + c; }, dpart);
+  const bool uniform = bad || !finite_max || !(sum > 0.0) || !(sum < __builtin_inf());
   int32_t* oid = ids + r * kk;
   float* opr = probs + r * kk;
   if (uniform) {
     const float u = 1.0f / (float)n;
-    for (int j = threadIdx.x; j < kk; j += kP2Threads) {
+    for (int j = tid; j < kk; j += kP2Threads) {
       oid[j] = j;
       opr[j] = u;
     }
     return;
   }
-  const int total = chunks * k;
-  const uint64_t* kr = keys + r * (int64_t)total;
+  // The first bin B at which kk groups have a maximum within it.
+#pragma unroll
+  for (int e = 0; e < GPT; ++e)
+    if (tid + kP2Threads * e < groups) atomicAdd(&hist[dist_bin(mx, gv[e])], 1u);
+  __syncthreads();
+  {
+    constexpr int BPT = kBins / kP2Threads;
+    uint32_t h[BPT], local = 0;
+#pragma unroll
+    for (int t = 0; t < BPT; ++t) local += h[t] = hist[tid * BPT + t];
+    uint32_t incl = local;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const uint32_t o = (uint32_t)__shfl_up((int)incl, off, 64);
+      if (lane >= off) incl += o;
+    }
+    if (lane == 63) wsum[wave] = incl;
+    __syncthreads();
+    uint32_t before = 0;
+    for (int w = 0; w < wave; ++w) before += wsum[w];
+    uint32_t run = before + incl - local;
+#pragma unroll
+    for (int t = 0; t < BPT; ++t) {
+      if (run < (uint32_t)kk && (uint32_t)kk <= run + h[t]) {
+        bin_at = (uint32_t)(tid * BPT + t);
+        groups_in = run + h[t];
+      }
+      run += h[t];
+    }
+  }
+  __syncthreads();
+  uint32_t bin = bin_at;
+  uint32_t ngroups = groups_in;
+  if (((int64_t)ngroups << gshift) <= kP2Keys) {
+#pragma unroll
+    for (int e = 0; e < GPT; ++e) {
+      const int gi = tid + kP2Threads * e;
+      if (gi < groups && dist_bin(mx, gv[e]) <= bin) list[atomicAdd(&nlist, 1u)] = gi;
+    }
+    __syncthreads();
+  } else {
+    // Massive ties: the kk groups of largest maximum, ties to the lower group.
+    uint64_t gk[GPT];
+#pragma unroll
+    for (int e = 0; e < GPT; ++e) {
+      const int gi = tid + kP2Threads * e;
+      gk[e] = gi < groups ? topk_key(gv[e], (uint32_t)gi) : 0;
+    }
+    select_top<kP2Threads, GPT>(gk, kk, top, sm, s);
+    ngroups = (uint32_t)(kk < groups ? kk : groups);
+    for (int j = tid; j < (int)ngroups; j += kP2Threads) list[j] = (int)~(uint32_t)top[j];
+    if (tid == 0) sm.ncand = 0;
+    __syncthreads();
+  }
+  // Their values; those within the bin are candidates (all kk winners are).
   constexpr int PER = kP2Keys / kP2Threads;
+  const int total = (int)(ngroups << gshift);
+  const float* row = x + r * n;
   uint64_t key[PER];
 #pragma unroll
   for (int e = 0; e < PER; ++e) {
-    const int j = threadIdx.x + kP2Threads * e;
-    key[e] = j < total ? kr[j] : 0;
+    const int j = tid + kP2Threads * e;
+    key[e] = 0;
+    if (j < total) {
+      const int64_t i = ((int64_t)list[j >> gshift] << gshift) + (j & ((1 << gshift) - 1));
+      if (i < n) {
+        float t = row[i];
+        if (scale) t *= inv_temp;
+        if (dist_bin(mx, t) <= bin) {
+          key[e] = topk_key(t, (uint32_t)i);
+          const uint32_t slot = atomicAdd(&sm.ncand, 1u);
+          if (slot < 256u) sm.cand[slot] = key[e];
+        }
+      }
+    }
   }
-  select_top<kP2Threads, PER>(key, kk, top, sm, s);
-  const float inv_sum = 1.0f / sum;
-  for (int j = threadIdx.x; j < kk; j += kP2Threads) {
+  __syncthreads();
+  const uint32_t ncand = sm.ncand;
+  if (ncand <= 256u) {
+    // 4 threads a candidate count the larger keys: its rank.
+    const int c = tid >> 2;
+    const uint64_t mine = c < (int)ncand ? sm.cand[c] : 0;
+    int rank = 0;
+    if (mine != 0)
+      for (int j = tid & 3; j < (int)ncand; j += 4) rank += sm.cand[j] > mine;
+    rank += __shfl_xor(rank, 1, 64);
+    rank += __shfl_xor(rank, 2, 64);
+    if (mine != 0 && (tid & 3) == 0 && rank < kk) top[rank] = mine;
+    __syncthreads();
+  } else {
+    select_top<kP2Threads, PER>(key, kk, top, sm, s);
+  }
+  for (int j = tid; j < kk; j += kP2Threads) {
     const uint64_t kv = top[j];
     oid[j] = (int32_t)~(uint32_t)kv;
-    opr[j] = expf(key_value(kv) - mx) * inv_sum;
+    opr[j] = (float)(exp((double)key_value(kv) - (double)mx) / sum);
   }
 }
 
@@ -329,7 +482,7 @@ __global__ __launch_bounds__(kP2Threads) void topk_final_kernel(
 int topk_chunks(int64_t n) { return (int)((n + kChunk - 1) / kChunk); }
 
 int topk_max_n(int k) {
-  // Candidate keys of a row must fit pass 2's LDS: chunks * k <= kP2Keys.
+  // The values of k groups must fit pass 2's LDS; kept at chunks * k <= kP2Keys.
   return k <= 0 ? 0 : (kP2Keys / k) * kChunk;
 }
 
@@ -340,23 +493,30 @@ hipError_t launch_top_tokens(const float* x, int rows, int64_t n, int top_n, flo
       n > topk_max_n(kk))
     return hipErrorInvalidValue;
   const int chunks = topk_chunks(n);
-  uint64_t* keys = reinterpret_cast<uint64_t*>(workspace);
-  float* stats = workspace + (size_t)rows * chunks * kk * 2;
+  const int gpc = chunk_groups(kk);
+  // Pass 2 groups: gm written maxima each, at most kP2Groups (n / (2048 / gpc) is at
+  // most 4 kP2Groups for an accepted n, so kk groups hold at most kP2Keys values).
+  int gm = 1, gshift = 0;
+  while ((int64_t)chunks * gpc > (int64_t)gm * kP2Groups) gm <<= 1;
+  while ((1 << gshift) < kChunk / gpc * gm) ++gshift;
+  if (((int64_t)kk << gshift) > kP2Keys) return hipErrorInvalidValue;
+  float* maxima = workspace;
+  float* stats = workspace + (size_t)rows * chunks * gpc;
   const bool scale = temperature > 0.0f && temperature != 1.0f;
   const float inv_temp = scale ? 1.0f / temperature : 1.0f;
   hipLaunchKernelGGL(topk_chunks_kernel, dim3((unsigned)chunks, (unsigned)rows), dim3(kP1Threads),
-                     0, stream, x, n, kk, inv_temp, scale ? 1 : 0, keys, stats);
+                     0, stream, x, n, gpc, inv_temp, scale ? 1 : 0, maxima, stats);
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) return err;
-  hipLaunchKernelGGL(topk_final_kernel, dim3((unsigned)rows), dim3(kP2Threads), 0, stream, keys,
-                     stats, chunks, kk, n, kk, ids, probs);
+  hipLaunchKernelGGL(topk_final_kernel, dim3((unsigned)rows), dim3(kP2Threads), 0, stream, x,
+                     maxima, stats, chunks, gpc, gm, gshift, n, kk, inv_temp, scale ? 1 : 0, ids,
+                     probs);
   return hipGetLastError();
 }
 
 size_t top_tokens_workspace_floats(int rows, int64_t n, int top_n) {
   const int kk = (int)(top_n < n ? top_n : n);
-  const size_t chunks = (size_t)topk_chunks(n);
-  return (size_t)rows * chunks * ((size_t)kk * 2 + 4);
+  return (size_t)rows * topk_chunks(n) * (size_t)(chunk_groups(kk) + 4);
 }
 
 }  // namespace mle

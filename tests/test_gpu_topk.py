@@ -113,3 +113,37 @@ def test_top_tokens_lm_head_pipeline(dev, orc):
         if clear:
             assert np.array_equal(ids[r], wi), r
             np.testing.assert_allclose(probs[r], wp, rtol=2e-4)
+
+
+@pytest.mark.parametrize("kind,n,top_n", [
+    ("sorted", 151936, 40), ("sorted", 5000, 128), ("equal", 151936, 128), ("masked", 151936, 40),
+    ("masked", 60000, 3), ("steps", 151936, 100), ("normal", 600_000, 9),
+    ("normal", 2_500_000, 2), ("normal", 1_000_000, 31), ("wide", 70_001, 64),
+    ("normal", 65, 64)])
+def test_top_tokens_group_selection(dev, kind, n, top_n):
+    """Rows that press on the selection by groups of values: winners side by side in few
+    groups, ties over all groups, logits masked with the lowest fp32 value, few distinct
+    values, a range of magnitudes, coarser groups for few tokens and long rows; unaligned
+    second row."""
+    rows = 2
+    rng = np.random.default_rng(n + top_n)
+    x = (S.activations(430, (rows, n)) * np.float32(3)).astype(np.float32)
+    if kind == "sorted":
+        x = np.sort(x, axis=1)
+    elif kind == "equal":
+        x[:] = 0.5
+    elif kind == "masked":
+        keep = rng.integers(0, n, size=(rows, 50))
+        m = np.full_like(x, np.finfo(np.float32).min)
+        np.put_along_axis(m, keep, np.take_along_axis(x, keep, 1), 1)
+        x = m
+    elif kind == "steps":
+        x = np.round(x).astype(np.float32)
+    elif kind == "wide":
+        x = (x * np.float32(10) ** rng.integers(-30, 2, size=(rows, n))).astype(np.float32)
+    note(f"top_tokens {kind} n={n} top_n={top_n}")
+    ids, probs = run(x, rows, n, top_n, 0.8, dev)
+    for r in range(rows):
+        want_ids, want_p = ref_top_tokens(x[r], top_n, 0.8)
+        assert np.array_equal(ids[r], want_ids), r
+        np.testing.assert_allclose(probs[r], want_p, rtol=1e-5, atol=1e-37)
