@@ -138,7 +138,8 @@ int mle_q8_0_linear_multi(const float* x, int count, const uint8_t* const* w,
  * int M, int N, int K)  (reference cuda_kernels.h:13, cuda_kernels.cu:852-868).
  * Elements as the reference CPU kernel cpu::sgemm(q8_0) forms them
  * (src/runtime/kernels/cpu_kernels.cpp:116-130), v = d*q in fp32.
- *   M < 64 (or A not 16-byte aligned): FP32 FMAs; the K sum is split into
+ *   M < 64 (or A not 16-byte aligned): FP32 FMAs for one or two rows of A, else
+ *   bf16 MFMA on a * d split exactly into three bf16 parts; the K sum is split into
  *   fixed pieces added in a fixed order (as the reference's device kernel
  *   splits K over warps), so results are deterministic and within fp32
  *   rounding of the CPU kernel (relative L2 <= 1e-5; small exact cases match it

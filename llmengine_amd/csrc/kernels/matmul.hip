@@ -9,128 +9,355 @@
 // sequential sum (relative L2 ~1e-7), as the reference's own device kernel is
 // (it splits K over 8 warps and adds their partials).
 //
-// Two kernels (from 64 rows of A the MatMul runs the bf16 MFMA GEMM instead):
-//   * M <= 8: the half-block kernel below, lanes reading 16-byte pieces of whole
-//     blocks along a B row;
-//   * 9 <= M < 64: the column-quad kernel.  A workgroup owns a tile of 256 output
-//     columns (8 blocks of a B row: lane l of every wave takes columns 4l .. 4l+3)
-//     for MR token rows, and a run of 256-row K slices.  Its 16 waves take 16
-//     consecutive rows of each slice each, issue all 16 rows' loads (the block
-//     scale and the lane's 4 quants, as 2-byte loads) before using any, and fold
-//     them into fp32 accumulators in row order; the activations of a row are
-//     wave-uniform (scalar loads).  The 16 waves' sums are then added in LDS in
-//     wave order.  When the column and token tiles alone leave the GPU's 256 CUs
-//     short of work, the K slices are spread over S workgroups per tile: each
-//     writes its partial tile to a workspace [S][M][N], and a second launch adds
-//     the S partials of every output in fixed runs of slices.  B is read once per
-//     MR token rows (MR = 8 at most).
+// Kernels (from 64 rows of A, 16-byte aligned, the MatMul runs the bf16 MFMA GEMM
+// instead):
+//   * one or two rows of A: the half-block kernel below, lanes
+//     reading 16-byte pieces of whole blocks along a B row, fp32 FMAs;
+//   * more: the MFMA kernel below, up to 64 rows a launch, B read once.
+// Where column tiles alone leave the GPU's 256 CUs short of work, K is spread over S
+// workgroups per tile.  Up to 8 rows of A they meet through a tile counter (a second
+// launch costs the host as much as such a call takes: 4 x 1632 x 2272 10.6 us a call with
+// it, 7.8 without); for more rows the MFMA kernel writes [S][M][N] partials, which a second
+// launch adds in fixed runs of splits.
 #include "../launch.hpp"
 #include "../q8_0_device.hpp"
 
 namespace mle {
 namespace {
 
-constexpr int kMmCols = 256;                 // output columns per workgroup
-constexpr int kMmWaves = 16;                 // waves per workgroup
-constexpr int kMmRun = 16;                   // B rows per wave per slice
-constexpr int kMmSlice = kMmWaves * kMmRun;  // B rows per slice
-constexpr int kMmTargetGroups = 512;         // workgroups wanted per launch (2 per CU)
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef int v2i __attribute__((ext_vector_type(2)));
 
-struct MmGrid {
-  unsigned col_tiles, row_tiles, splits;
-  int slices_per_split;
+__device__ __forceinline__ uint32_t top_halves(uint32_t lo_word, uint32_t hi_word) {
+  return __builtin_amdgcn_perm(hi_word, lo_word, 0x07060302u);
+}
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t mm_rsrc(const void* base, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes,
+                                           0x00020000);
+}
+
+// MFMA kernel (3 to 64 rows of A), fp32-exact operands.
+//
+// A block of B holds 32 columns of one k, so its scale cannot leave the K sum; it goes
+// into the activations instead: for one 32-column block, c[m, n] = sum_k (a[m, k]
+// d[k]) q[k, n].  The fp32 product a * d (one rounding, as the FMA chain rounds each
+// sum) is split exactly into three bf16 parts by truncation, the quants are exact in
+// bf16, and v_mfma_f32_16x16x32_bf16 forms the products exactly with fp32 sums.  K
+// steps that hold a non-finite scale or an activation past 2^100 (whose product could
+// leave the range where d * q would not) are summed by fp32 FMAs instead, v = d * q
+// first, as the reference does.
+//
+// A workgroup owns NBW 32-column blocks and one K split; its 8 waves take 32-row K
+// steps in turn and add their sums in LDS.  Per step a wave reads its 32 B rows as
+// whole half blocks (2 NBW lanes a row, 34 NBW contiguous bytes) and its 16 TT x 32
+// activations (8 lanes a row), passes both through wave-private LDS, and takes the
+// quants back transposed, 8 consecutive k of one column a lane, with ds_read_b64_tr_b8.
+// The next step's loads are in flight while one is multiplied.
+//
+// Bound by the vector ALUs (8 products, the split of 8 values and 16 int8 -> bf16
+// conversions a lane for 6 TT MFMAs).  Measured (MI355X, rotated B, us, against fp32
+// FMAs on up to 8 rows at a time): 4096 x 4096 at M = 4 / 8 / 16 / 63 14.5 / 28.0 /
+// 43.4 / 127 -> 11.9 / 12.0 / 13.3 / 23.6; 11008 x 4096 21.4 / 38.0 / 102 / 370 -> 21.4
+// / 21.7 / 22.6 / 52.5; [896, 151936] 48.7 / 87.1 / 288 / 1028 -> 43.4 / 44.5 / 47.8 /
+// 146.  256-column wave tiles (one workgroup a CU) were 1.1-1.5x slower.
+constexpr int kMfWaves = 8;
+constexpr int kMfNT = 64 * kMfWaves;
+
+struct MfGrid {
+  unsigned tiles, splits;
+  int tt, nbw, steps_per_split;
 };
 
-MmGrid mm_grid(int M, int N, int K, int mr) {
-  MmGrid g;
-  g.col_tiles = (unsigned)((N + kMmCols - 1) / kMmCols);
-  g.row_tiles = (unsigned)((M + mr - 1) / mr);
-  const int slices = (K + kMmSlice - 1) / kMmSlice;
-  const int64_t tiles = (int64_t)g.col_tiles * g.row_tiles;
-  int s = (int)((kMmTargetGroups + tiles - 1) / tiles);
-  if (s > slices) s = slices;
+MfGrid mf_grid(int M, int N, int K) {
+  MfGrid g;
+  g.tt = (M + 15) / 16;
+  if (g.tt > 4) g.tt = 4;
+  g.nbw = g.tt <= 2 ? 4 : 2;
+  g.tiles = (unsigned)((N / kBlockElems + g.nbw - 1) / g.nbw);
+  const int steps = K / kBlockElems;
+  // At most two workgroups a CU at one token tile (126 registers), else one; each wave
+  // at least one K step.  Rounded down: a third round for a few workgroups costs more
+  // (11008 x 4096 at 16 rows: 22.6 us with 5 splits, 25.7 with 6).
+  int s = (int)((g.tt == 1 ? 512 : 256) / g.tiles);
+  if (s > steps / kMfWaves) s = steps / kMfWaves;
   if (s < 1) s = 1;
-  g.slices_per_split = (slices + s - 1) / s;
-  g.splits = (unsigned)((slices + g.slices_per_split - 1) / g.slices_per_split);
+  g.steps_per_split = (steps + s - 1) / s;
+  g.splits = (unsigned)((steps + g.steps_per_split - 1) / g.steps_per_split);
   return g;
 }
 
-int mm_rows_per_tile(int M) { return M >= 8 ? 8 : M >= 4 ? 4 : M >= 2 ? 2 : 1; }
+// Whether the K splits meet inside the launch (else in a second one).
+bool mf_handoff(int M) { return M <= 8; }
 
-template <int MR>
-__global__ __launch_bounds__(64 * kMmWaves) void matmul_q8_0_kernel(
-    const float* __restrict__ a, const uint8_t* __restrict__ b, float* __restrict__ out,
-    int M, int N, int K, int slices_per_split) {
-  __shared__ float red[kMmWaves][MR][kMmCols];
+template <int TT, int NBW>
+__global__ __launch_bounds__(kMfNT, 2) void matmul_q8_0_mfma_kernel(
+    const float* __restrict__ a, const uint8_t* __restrict__ b, float* __restrict__ out, int M,
+    int N, int K, int steps_per_split, float* __restrict__ partials,
+    uint32_t* __restrict__ counters) {
+  constexpr int QS = NBW * 32 + 16;    // LDS bytes of a B row (16-byte pieces, banks spread)
+  constexpr int AS = 36;               // LDS floats of an activation row
+  constexpr int LPR = 2 * NBW;         // lanes a B row
+  constexpr int RPI = 64 / LPR;        // B rows per load instruction
+  constexpr int BL = 32 / RPI;         // B load instructions per step
+  constexpr int Q_BYTES = 32 * QS, S_BYTES = NBW * 64, A_BYTES = 16 * TT * AS * 4;
+  constexpr int WAVE_BYTES = Q_BYTES + S_BYTES + A_BYTES;
+  constexpr int SLOTS = 2 * NBW * TT;  // 16 x 16 output tiles
+  constexpr int RED_BYTES = 4 * SLOTS * 1024;
+  constexpr int LDS = kMfWaves * WAVE_BYTES > RED_BYTES ? kMfWaves * WAVE_BYTES : RED_BYTES;
+  static_assert(WAVE_BYTES % 16 == 0, "16-byte wave areas");
+  __shared__ __attribute__((aligned(16))) uint8_t lds[LDS];
+  __shared__ uint32_t arrived;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int n0 = blockIdx.x * kMmCols;
-  const int n = n0 + 4 * lane;  // this lane's 4 columns
-  const bool live_n = n < N;    // N % 32 == 0: the 4 columns are all inside or all outside
-  const int m0 = blockIdx.z * MR;
+  const int g = lane >> 4, r16 = lane & 15;
   const int64_t NB = N / kBlockElems;
-  const int blk = n / kBlockElems, o = n % kBlockElems;  // o: 0, 4, .., 28
-  const int s_begin = blockIdx.y * slices_per_split;
-  const int nslices = (K + kMmSlice - 1) / kMmSlice;
-  const int s_end = min(s_begin + slices_per_split, nslices);
-  // Activation rows of the tile (rows past M read row M - 1 and are never stored).
-  const float* arow[MR];
-#pragma unroll
-  for (int r = 0; r < MR; ++r) arow[r] = a + (int64_t)min(m0 + r, M - 1) * K;
+  // Workgroup i runs on XCD i % 8: each XCD takes a contiguous run of (split, column
+  // tile) pairs, so the 128-byte lines that neighbouring tiles share are fetched into
+  // one L2 (0.93-0.97x).
+  const unsigned total = gridDim.x * gridDim.y, lin = blockIdx.y * gridDim.x + blockIdx.x;
+  const unsigned q8 = total / 8, r8 = total % 8, xcd = lin % 8, ix = lin / 8;
+  const unsigned nid = xcd * q8 + min(xcd, r8) + ix;
+  const unsigned by = nid / gridDim.x, bx = nid % gridDim.x;
+  const int64_t blk0 = (int64_t)bx * NBW;
+  const int s0 = by * steps_per_split;
+  const int s1 = min(s0 + steps_per_split, K / kBlockElems);
+  uint8_t* const qs = lds + wave * WAVE_BYTES;
+  uint16_t* const ss = reinterpret_cast<uint16_t*>(qs + Q_BYTES);
+  float* const as = reinterpret_cast<float*>(qs + Q_BYTES + S_BYTES);
 
-  float acc[MR][4];
+  // This lane's half block of a B row (columns past N re-read the last block) and its
+  // 4 activations of a row (rows past M re-read row M - 1); neither is ever stored.
+  const int brow = lane / LPR, bcol = lane % LPR;
+  const uint8_t* const bp = b + ((int64_t)brow * NB + min(blk0 + (bcol >> 1), NB - 1)) * kBlockBytes;
+  const int arow = lane >> 3, acol = lane & 7;
+  const float* ap[2 * TT];
 #pragma unroll
-  for (int r = 0; r < MR; ++r)
+  for (int i = 0; i < 2 * TT; ++i) ap[i] = a + (int64_t)min(arow + 8 * i, M - 1) * K + 4 * acol;
+  struct Stage {
+    u32x4 q[BL];
+    uint16_t s[BL];
+    f32x4 x[2 * TT];
+  };
+  auto load = [&](int step, Stage& st) {
+    const uint8_t* p = bp + (int64_t)step * kBlockElems * NB * kBlockBytes;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[r][j] = 0.0f;
-  for (int sl = s_begin; sl < s_end; ++sl) {
-    const int k0 = sl * kMmSlice + wave * kMmRun;  // this wave's rows k0 .. k0 + 15
-    uint16_t sc[kMmRun], q01[kMmRun], q23[kMmRun];
+    for (int i = 0; i < BL; ++i) {
+      const uint8_t* r = p + (int64_t)(i * RPI) * NB * kBlockBytes;
+      __builtin_memcpy(&st.q[i], __builtin_assume_aligned(r + 2 + 16 * (bcol & 1), 2), 16);
+      st.s[i] = *reinterpret_cast<const uint16_t*>(r);
+    }
 #pragma unroll
-    for (int j = 0; j < kMmRun; ++j) {
-      const int k = k0 + j;
-      if (live_n && k < K) {
-        const uint16_t* hp =
-            reinterpret_cast<const uint16_t*>(b + ((int64_t)k * NB + blk) * kBlockBytes);
-        sc[j] = hp[0];
-        q01[j] = hp[1 + o / 2];
-        q23[j] = hp[2 + o / 2];
-      } else {
-        sc[j] = 0;  // scale +0: the row adds nothing
-        q01[j] = q23[j] = 0;
+    for (int i = 0; i < 2 * TT; ++i)
+      __builtin_memcpy(&st.x[i], __builtin_assume_aligned(ap[i] + (int64_t)step * kBlockElems, 4), 16);
+  };
+
+  f32x4 acc[NBW][2][TT];
+#pragma unroll
+  for (int n = 0; n < NBW; ++n)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int t = 0; t < TT; ++t) acc[n][j][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  auto wave_sync = [] {
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+  // Registers -> wave-private LDS; whether the step is all finite and small.
+  auto stage = [&](const Stage& st) {
+    bool fine = true;
+#pragma unroll
+    for (int i = 0; i < BL; ++i) {
+      const int row = i * RPI + brow;
+      *reinterpret_cast<u32x4*>(qs + row * QS + bcol * 16) = st.q[i];
+      ss[(bcol >> 1) * 32 + row] = st.s[i];
+      fine &= (st.s[i] & 0x7c00u) != 0x7c00u;
+    }
+#pragma unroll
+    for (int i = 0; i < 2 * TT; ++i) {
+      *reinterpret_cast<f32x4*>(as + (arow + 8 * i) * AS + 4 * acol) = st.x[i];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) fine &= __builtin_fabsf(st.x[i][e]) < 0x1p100f;  // false on NaN
+    }
+    return __builtin_amdgcn_ballot_w64(!fine) == 0;
+  };
+  auto multiply = [&] {
+    float x[TT][8];
+#pragma unroll
+    for (int t = 0; t < TT; ++t) {
+      const f32x4 lo = *reinterpret_cast<const f32x4*>(as + (16 * t + r16) * AS + 8 * g);
+      const f32x4 hi = *reinterpret_cast<const f32x4*>(as + (16 * t + r16) * AS + 8 * g + 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        x[t][e] = lo[e];
+        x[t][4 + e] = hi[e];
       }
     }
 #pragma unroll
-    for (int j = 0; j < kMmRun; ++j) {
-      const int k = k0 + j;
-      const float d = scale_to_f32(sc[j]);
-      const uint32_t q = (uint32_t)q01[j] | ((uint32_t)q23[j] << 16);
-      const float v[4] = {d * q_at(q, 0), d * q_at(q, 1), d * q_at(q, 2), d * q_at(q, 3)};
+    for (int n = 0; n < NBW; ++n) {
+      const u32x4 sc = *reinterpret_cast<const u32x4*>(ss + n * 32 + 8 * g);
+      float d[8];
 #pragma unroll
-      for (int r = 0; r < MR; ++r) {
-        const float av = k < K ? arow[r][k] : 0.0f;  // wave-uniform
+      for (int e = 0; e < 8; ++e)
+        d[e] = scale_to_f32_fast(e & 1 ? sc[e >> 1] >> 16 : sc[e >> 1] & 0xffffu);
+      bf16x8 wf[2];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) acc[r][i] = __builtin_fmaf(av, v[i], acc[r][i]);
+      for (int j = 0; j < 2; ++j) {
+        typedef __attribute__((address_space(3))) v2i lds_v2i;
+        const v2i q = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
+            (lds_v2i*)(qs + (8 * g + (r16 >> 1)) * QS + n * 32 + j * 16 + (r16 & 1) * 8));
+        u32x4 o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const uint32_t w = (uint32_t)(e < 2 ? q.x : q.y);
+          o[e] = top_halves(__builtin_bit_cast(uint32_t, q_at(w, 2 * (e & 1))),
+                            __builtin_bit_cast(uint32_t, q_at(w, 2 * (e & 1) + 1)));
+        }
+        wf[j] = __builtin_bit_cast(bf16x8, o);
       }
+#pragma unroll
+      for (int t = 0; t < TT; ++t) {
+        u32x4 part[3];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          uint32_t hb[2], rb[2], lb[2];
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            const float v = x[t][2 * e + u] * d[2 * e + u];
+            hb[u] = __builtin_bit_cast(uint32_t, v);
+            const float r = v - __builtin_bit_cast(float, hb[u] & 0xffff0000u);
+            rb[u] = __builtin_bit_cast(uint32_t, r);
+            lb[u] = __builtin_bit_cast(uint32_t, r - __builtin_bit_cast(float, rb[u] & 0xffff0000u));
+          }
+          part[0][e] = top_halves(hb[0], hb[1]);
+          part[1][e] = top_halves(rb[0], rb[1]);
+          part[2][e] = top_halves(lb[0], lb[1]);
+        }
+#pragma unroll
+        for (int p = 0; p < 3; ++p)
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+            acc[n][j][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                __builtin_bit_cast(bf16x8, part[p]), wf[j], acc[n][j][t], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  };
+  // The same sums by fp32 FMAs, v = d * q first (rare: see above).
+  auto multiply_fp32 = [&] {
+    for (int k = 0; k < 32; ++k)
+#pragma unroll
+      for (int n = 0; n < NBW; ++n)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const float v = scale_to_f32(ss[n * 32 + k]) *
+                          (float)(int8_t)qs[k * QS + n * 32 + j * 16 + r16];
+#pragma unroll
+          for (int t = 0; t < TT; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              acc[n][j][t][e] =
+                  __builtin_fmaf(as[(16 * t + 4 * g + e) * AS + k], v, acc[n][j][t][e]);
+        }
+  };
+
+  Stage st;
+  int step = s0 + wave;
+  if (step < s1) {
+    load(step, st);
+    for (; step < s1; step += kMfWaves) {
+      const bool fine = stage(st);
+      wave_sync();
+      if (step + kMfWaves < s1) load(step + kMfWaves, st);
+      if (fine)
+        multiply();
+      else
+        multiply_fp32();
+      wave_sync();  // the step's LDS reads come before the next one's writes
     }
   }
-#pragma unroll
-  for (int r = 0; r < MR; ++r)
-    *reinterpret_cast<f32x4*>(&red[wave][r][4 * lane]) =
-        f32x4{acc[r][0], acc[r][1], acc[r][2], acc[r][3]};
+
+  // Waves w and w + 4 add first, then the four pairs' sums in order.
   __syncthreads();
-  // The 16 waves' sums of each output, in wave order; outputs (r, column).
-  for (int idx = tid; idx < MR * kMmCols; idx += 64 * kMmWaves) {
-    const int r = idx / kMmCols, col = idx % kMmCols;
-    float s = red[0][r][col];
+  f32x4* const red = reinterpret_cast<f32x4*>(lds);
+  if (wave >= 4) {
 #pragma unroll
-    for (int w = 1; w < kMmWaves; ++w) s += red[w][r][col];
-    const int m = m0 + r, nn = n0 + col;
-    if (m < M && nn < N) out[((int64_t)blockIdx.y * M + m) * N + nn] = s;
+    for (int i = 0; i < SLOTS; ++i)
+      red[((wave - 4) * SLOTS + i) * 64 + lane] = acc[i / (2 * TT)][i / TT % 2][i % TT];
+  }
+  __syncthreads();
+  if (wave < 4) {
+#pragma unroll
+    for (int i = 0; i < SLOTS; ++i) {
+      f32x4& slot = red[(wave * SLOTS + i) * 64 + lane];
+      slot = acc[i / (2 * TT)][i / TT % 2][i % TT] + slot;
+    }
+  }
+  __syncthreads();
+  // Output tile i of the workgroup: rows 4 g .. + 3 of its token tile, column r16.
+  auto store = [&](float* dst, int i, const f32x4 v) {
+    const int n = i / (2 * TT), j = i / TT % 2, t = i % TT;
+    const int m = 16 * t + 4 * g;
+    const int64_t col = (blk0 + n) * kBlockElems + j * 16 + r16;
+    if (blk0 + n >= NB) return;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (m + e < M) dst[(int64_t)(m + e) * N + col] = v[e];
+  };
+  auto sum_of = [&](int i) {
+    f32x4 v = red[i * 64 + lane];
+#pragma unroll
+    for (int w = 1; w < 4; ++w) v += red[(w * SLOTS + i) * 64 + lane];
+    return v;
+  };
+  if (counters == nullptr) {
+    float* const dst = out + (int64_t)by * M * N;
+#pragma unroll
+    for (int u = 0; u < (SLOTS + kMfWaves - 1) / kMfWaves; ++u) {
+      const int i = u * kMfWaves + wave;
+      if (SLOTS % kMfWaves == 0 || i < SLOTS) store(dst, i, sum_of(i));
+    }
+    return;
+  }
+  if constexpr (SLOTS == kMfWaves) {  // one output tile a wave
+    // The splits of a tile meet: partials by device-scope stores, their completion,
+    // the tile's counter; the last workgroup resets it and adds them in split order.
+    constexpr int SC1 = 16;  // cache-policy bit: device scope
+    constexpr uint32_t REGION = SLOTS * 1024;
+    const unsigned nspl = gridDim.y;
+    const uint32_t mine = (uint32_t)(wave * 64 + lane) * 16;
+    const __amdgpu_buffer_rsrc_t prs =
+        mm_rsrc(reinterpret_cast<uint8_t*>(partials) + (int64_t)bx * nspl * REGION, nspl * REGION);
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, sum_of(wave)), prs,
+                                           by * REGION + mine, 0, SC1);
+    uint32_t* const counter = counters + (size_t)bx * kCounterStride;
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_s_waitcnt(0);  // every partial has reached the coherence point
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __syncthreads();
+    if (tid == 0)
+      arrived = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    if (arrived != nspl - 1) return;
+    if (tid == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    for (unsigned sp = 0; sp < nspl; sp += 8) {
+      f32x4 p[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        p[j] = __builtin_bit_cast(
+            f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                       prs, sp + j < nspl ? (sp + j) * REGION + mine : 0x80000000u, 0, SC1));
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v += p[j];
+    }
+    store(out, wave, v);
   }
 }
 
-// Half-block kernel (M <= 8).  A workgroup owns a tile of 256 output columns (8
+// Half-block kernel (M <= 2).  A workgroup owns a tile of 256 output columns (8
 // blocks of a B row) for MR token rows and a run of K.  Lane c of a 16-lane group
 // takes 16 columns, half h = c % 2 of block c / 2 of the tile, of one B row per
 // step, so a group reads the tile's 272 contiguous bytes of a row and a wave four
@@ -167,8 +394,8 @@ struct LnGrid {
 LnGrid ln_grid(int M, int N, int K) {
   LnGrid g;
   const int NB = N / kBlockElems;
-  g.mr = M >= 8 ? 8 : M >= 4 ? 4 : M >= 2 ? 2 : 1;
-  g.unroll = g.mr >= 4 ? 4 : 8;  // 16 MR accumulators + 5 U load registers per lane
+  g.mr = M >= 2 ? 2 : 1;
+  g.unroll = 8;
   g.col_tiles = (unsigned)((NB + kLnLanes / 2 - 1) / (kLnLanes / 2));
   g.row_tiles = (unsigned)((M + g.mr - 1) / g.mr);
   const int batch = g.unroll * kLnWaves * kLnRows;
@@ -181,11 +408,6 @@ LnGrid ln_grid(int M, int N, int K) {
   g.batches_per_split = (batches + s - 1) / s;
   g.splits = (unsigned)((batches + g.batches_per_split - 1) / g.batches_per_split);
   return g;
-}
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t mm_rsrc(const void* base, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes,
-                                           0x00020000);
 }
 
 template <int MR, int U>
@@ -331,7 +553,7 @@ __global__ __launch_bounds__(kLnNT) void matmul_q8_0_half_kernel(
   // thread sums its run in split order with the loads of 8 splits issued together,
   // then the runs' sums of a piece are added in run order in LDS.
   constexpr int PIECES = MR * kLnCols / 4;
-  constexpr int RUNS = kLnNT / PIECES;  // 8, 4, 2 or 1 for MR = 1, 2, 4, 8
+  constexpr int RUNS = kLnNT / PIECES;  // 8 or 4 for MR = 1, 2
   const unsigned nspl = gridDim.y, per = (nspl + RUNS - 1) / RUNS;
   const int pc = tid % PIECES, run = tid / PIECES;
   f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -392,11 +614,11 @@ __global__ __launch_bounds__(256) void matmul_splits_kernel(const float* __restr
   }
 }
 
-template <int MR>
-void launch_mm(const MmGrid& g, const float* a, const uint8_t* b, float* dst, int M, int N,
-               int K, hipStream_t stream) {
-  hipLaunchKernelGGL(matmul_q8_0_kernel<MR>, dim3(g.col_tiles, g.splits, g.row_tiles),
-                     dim3(64 * kMmWaves), 0, stream, a, b, dst, M, N, K, g.slices_per_split);
+template <int TT, int NBW>
+void launch_mf(const MfGrid& g, const float* a, const uint8_t* b, float* dst, int M, int N, int K,
+               float* partials, uint32_t* counters, hipStream_t stream) {
+  hipLaunchKernelGGL((matmul_q8_0_mfma_kernel<TT, NBW>), dim3(g.tiles, g.splits), dim3(kMfNT), 0,
+                     stream, a, b, dst, M, N, K, g.steps_per_split, partials, counters);
 }
 
 template <int MR, int U>
@@ -407,11 +629,11 @@ void launch_ln(const LnGrid& g, const float* a, const uint8_t* b, float* c, int 
                      counters);
 }
 
-// The half-block kernel takes M <= 8 (larger M keeps the column-quad kernel,
-// which reads B once per 8 token rows as well) and B below 2 GiB (32-bit buffer
-// offsets).
+// The half-block kernel's calls: up to two rows of A (MI355X, two rows: 4096 x 4096
+// 10.6 us vs 11.2 on the MFMA kernel, 11008 x 4096 20.3 vs 21.3; three and four rows
+// 13.9-14.5 vs 11.8, 21-28 vs 21.4) and B below 2 GiB (32-bit buffer offsets).
 bool use_half(int M, int N, int K) {
-  return M <= 8 && (int64_t)K * (N / kBlockElems) * kBlockBytes < (int64_t(1) << 31) &&
+  return M <= 2 && (int64_t)K * (N / kBlockElems) * kBlockBytes < (int64_t(1) << 31) &&
          (int64_t)M * K * 4 < (int64_t(1) << 31);
 }
 
@@ -429,8 +651,13 @@ MatmulNeed matmul_workspace(int M, int N, int K) {
     }
     return need;
   }
-  const MmGrid g = mm_grid(M, N, K, mm_rows_per_tile(M));
-  if (g.splits > 1) need.partial_floats = (size_t)g.splits * M * N;
+  const MfGrid g = mf_grid(M, N, K);
+  const int rows = M < 16 * g.tt ? M : 16 * g.tt;  // of one launch
+  if (g.splits > 1) need.partial_floats = (size_t)g.splits * rows * N;
+  if (g.splits > 1 && mf_handoff(M)) {
+    need.partial_floats = (size_t)g.tiles * g.splits * kMfWaves * 256;
+    need.counters = (size_t)g.tiles * kCounterStride;
+  }
   return need;
 }
 
@@ -448,29 +675,37 @@ hipError_t launch_matmul(const float* a, const uint8_t* b, float* c, int M, int 
     }
     switch (g.mr) {
       case 1: launch_ln<1, 8>(g, a, b, c, M, N, K, partials, counters, stream); break;
-      case 2: launch_ln<2, 8>(g, a, b, c, M, N, K, partials, counters, stream); break;
-      case 4: launch_ln<4, 4>(g, a, b, c, M, N, K, partials, counters, stream); break;
-      default: launch_ln<8, 4>(g, a, b, c, M, N, K, partials, counters, stream); break;
+      default: launch_ln<2, 8>(g, a, b, c, M, N, K, partials, counters, stream); break;
     }
     return hipGetLastError();
   }
-  const int mr = mm_rows_per_tile(M);
-  const MmGrid g = mm_grid(M, N, K, mr);
-  if (g.row_tiles > 65535 || g.splits > 65535) return hipErrorInvalidValue;
+  // Up to 64 rows of A a launch (more only where the GEMM does not take the call).
+  const MfGrid g = mf_grid(M, N, K);
   if (g.splits > 1 && partials == nullptr) return hipErrorInvalidValue;
-  float* dst = g.splits > 1 ? partials : c;
-  switch (mr) {
-    case 1: launch_mm<1>(g, a, b, dst, M, N, K, stream); break;
-    case 2: launch_mm<2>(g, a, b, dst, M, N, K, stream); break;
-    case 4: launch_mm<4>(g, a, b, dst, M, N, K, stream); break;
-    default: launch_mm<8>(g, a, b, dst, M, N, K, stream); break;
+  const bool handoff = g.splits > 1 && mf_handoff(M);
+  if (handoff && counters == nullptr) return hipErrorInvalidValue;
+  if (!handoff) counters = nullptr;
+  for (int m0 = 0; m0 < M; m0 += 16 * g.tt) {
+    const int mc = M - m0 < 16 * g.tt ? M - m0 : 16 * g.tt;
+    const float* am = a + (int64_t)m0 * K;
+    float* cm = c + (int64_t)m0 * N;
+    float* dst = g.splits > 1 && !handoff ? partials : cm;
+    switch (g.tt) {
+      case 1: launch_mf<1, 4>(g, am, b, dst, mc, N, K, partials, counters, stream); break;
+      case 2: launch_mf<2, 4>(g, am, b, dst, mc, N, K, partials, counters, stream); break;
+      case 3: launch_mf<3, 2>(g, am, b, dst, mc, N, K, partials, counters, stream); break;
+      default: launch_mf<4, 2>(g, am, b, dst, mc, N, K, partials, counters, stream); break;
+    }
+    hipError_t err = hipGetLastError();
+    if (err != hipSuccess) return err;
+    if (g.splits == 1 || handoff) continue;
+    const int64_t mn4 = (int64_t)mc * N / 4;
+    hipLaunchKernelGGL(matmul_splits_kernel, dim3((unsigned)((mn4 + kSpCols - 1) / kSpCols)),
+                       dim3(256), 0, stream, partials, cm, mn4, (int)g.splits);
+    err = hipGetLastError();
+    if (err != hipSuccess) return err;
   }
-  hipError_t err = hipGetLastError();
-  if (err != hipSuccess || g.splits == 1) return err;
-  const int64_t mn4 = (int64_t)M * N / 4;
-  hipLaunchKernelGGL(matmul_splits_kernel, dim3((unsigned)((mn4 + kSpCols - 1) / kSpCols)),
-                     dim3(256), 0, stream, partials, c, mn4, (int)g.splits);
-  return hipGetLastError();
+  return hipSuccess;
 }
 
 }  // namespace mle

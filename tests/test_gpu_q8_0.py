@@ -785,6 +785,53 @@ def test_matmul_gemm_path(dev, orc, M, N, K):
     assert rel_l2(got, fp32) <= 1e-2, (M, N, K)
 
 
+@pytest.mark.parametrize("M,N,K", [(3, 32, 32), (16, 160, 352), (17, 4096, 64), (33, 96, 288),
+                                   (49, 224, 4128), (64, 64, 96), (130, 352, 96)])
+def test_matmul_mfma_remainders(dev, orc, M, N, K):
+    """The MFMA MatMul at the edges of its tiles: token tiles and their remainders, one
+    column block, ragged column tiles, one K step, more waves than steps; rows of A at a
+    4-byte offset (which also keeps 64 and more rows off the bf16 GEMM), with B's."""
+    import torch
+    note(f"matmul mfma M={M} N={N} K={K}")
+    b, a = weight(500 + N, K, N), acts(501 + K, M, K)
+    da, db = to_dev(a, dev), to_dev(b, dev)
+    abuf = torch.zeros(M * K + 4, dtype=torch.float32, device=dev)
+    bbuf = torch.zeros(db.numel() + 2, dtype=torch.uint8, device=dev)
+    abuf[1:1 + M * K], bbuf[2:] = da.view(-1), db
+    out, out2 = empty_f32((M, N), dev), empty_f32((M, N), dev)
+    capi.matmul(abuf[1:], db, out, M, N, K)
+    capi.matmul(abuf[1:], bbuf[2:], out2, M, N, K)
+    torch.cuda.synchronize()
+    assert torch.equal(out, out2)
+    assert rel_l2(to_host(out), orc.sgemm(a, b, M, N, K)) <= 1e-5
+
+
+@pytest.mark.parametrize("M", [5, 40])
+def test_matmul_mfma_special_values(dev, orc, M):
+    """Non-finite scales and activations, and activations whose product with a scale
+    leaves the fp32 range while d * q (q = 0) does not, give the reference chain's
+    non-finite entries; the other entries its values."""
+    N, K = 96, 512
+    b = weight(510, K, N).reshape(K, N // 32, 34).copy()
+    b[7, 0, :2] = np.array([0x00, 0x7c], np.uint8)      # +Inf scale
+    b[40, 1, :2] = np.array([0x01, 0x7e], np.uint8)     # NaN scale
+    b[100, 2, :2] = np.array([0xff, 0x7b], np.uint8)    # 65504
+    b[100, 2, 2::2] = 0                                 # zero quants under it
+    a = acts(511, M, K)
+    a[0, 100], a[1, 3], a[2, 450], a[3, 9] = 1e37, np.inf, np.nan, -np.inf
+    note(f"matmul special values M={M}")
+    out = empty_f32((M, N), dev)
+    capi.matmul(to_dev(a, dev), to_dev(b.reshape(-1), dev), out, M, N, K)
+    with np.errstate(all="ignore"):
+        want = orc.sgemm(a, b.reshape(-1), M, N, K)
+    got = to_host(out)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    inf = np.isinf(want)
+    assert np.array_equal(np.isinf(got), inf) and np.array_equal(got[inf], want[inf])
+    fin = np.isfinite(want)
+    assert fin.any() and rel_l2(got[fin], want[fin]) <= 1e-5
+
+
 # ----------------------------------------------------------------------------- errors
 
 def test_device_error_paths(dev):
