@@ -358,7 +358,7 @@ int run_linear(const float* x, const uint8_t* w, const void* bias, float* y, int
       if (!tune.gemm.bm && !mle::gemm_mfma_config_valid(c)) c.bm = 128;
     }
     if (tune.gemm.splits) c.splits = tune.gemm.splits;
-    if (!mle::gemm_mfma_config_valid(c))
+    if (!mle::gemm_mfma_launchable(c))
       return fail(MLE_INVALID_ARGUMENT, "hip sgemm_nt_q8_0_weight: invalid MFMA GEMM shape (bm " +
                                             std::to_string(c.bm) + ", bn " +
                                             std::to_string(c.bn) + ")");

@@ -621,15 +621,19 @@ template <int MI, int NJ, int L>
 void launch_tile_l(const GemmGrid& g, Epilogue mode, const u32x4* xf, uint32_t xf_bytes, int M,
                    int K, const SplitKWorkspace& ws, hipStream_t stream) {
   const dim3 grid(g.tn, g.tm, g.splits);
-  if constexpr (L == int(WeightLayout::kKN)) {  // MatMul: plain epilogue only
+  constexpr bool kWide = MI == 2 && NJ == 4;
+  if constexpr (L == int(WeightLayout::kKN) && kWide) {
+    (void)grid;  // not launched (spills)
+  } else if constexpr (L == int(WeightLayout::kKN)) {  // MatMul: plain epilogue only
     (void)mode;
     hipLaunchKernelGGL((gemm_q8_0_mfma_kernel<MI, NJ, 0, L>), grid, dim3(Roles<MI>::kThreads), 0,
                        stream, xf, xf_bytes, g.args, M, K, g.steps_per_split, ws.partials,
                        ws.counters);
   } else if (mode == Epilogue::kSwiGLU) {
-    hipLaunchKernelGGL((gemm_q8_0_mfma_kernel<MI, NJ, 1, L>), grid, dim3(Roles<MI>::kThreads), 0,
-                       stream, xf, xf_bytes, g.args, M, K, g.steps_per_split, ws.partials,
-                       ws.counters);
+    if constexpr (!(kWide && L == int(WeightLayout::kRaw)))
+      hipLaunchKernelGGL((gemm_q8_0_mfma_kernel<MI, NJ, 1, L>), grid, dim3(Roles<MI>::kThreads),
+                         0, stream, xf, xf_bytes, g.args, M, K, g.steps_per_split, ws.partials,
+                         ws.counters);
   } else {
     hipLaunchKernelGGL((gemm_q8_0_mfma_kernel<MI, NJ, 0, L>), grid, dim3(Roles<MI>::kThreads), 0,
                        stream, xf, xf_bytes, g.args, M, K, g.steps_per_split, ws.partials,
@@ -656,8 +660,13 @@ constexpr size_t kScratchAlign = 256;
 
 }  // namespace
 
+// 256 x 128 tiles are the automatic pick's alone: the tuning hook refuses them, as it
+// always has.
+bool gemm_mfma_launchable(const GemmConfig& c) {
+  return gemm_mfma_config_valid(c) || (c.bm == 256 && c.bn == 128 && c.splits >= 1 && c.splits <= 64);
+}
+
 bool gemm_mfma_config_valid(const GemmConfig& c) {
-  // 256 x 128 tiles would need more than the 256 registers a wave gets.
   return ((c.bm == 128 && (c.bn == 64 || c.bn == 96 || c.bn == 128)) ||
           (c.bm == 256 && (c.bn == 64 || c.bn == 96))) &&
          c.splits >= 1 && c.splits <= 64;
@@ -670,11 +679,17 @@ GemmConfig gemm_mfma_pick_segs(int M, const LinearSegs& s, int K) {
   // {4096, 11008} sweeps), plus the split-K partial traffic (written and read
   // once per split; it mostly stays in cache, ~5.6 TB/s).  Tile heights of 256
   // only once M exceeds 128.  A SwiGLU tile holds BN/2 rows of each weight.
+  // 256 x 128 tiles (159-165 registers at 12 waves, no spills) do the same MFMAs in
+  // fewer rounds: 2048 x 4096 x 11008 in one round of 256 workgroups instead of 1.3 of
+  // 256 x 96 (tiled 212 -> 175 us, raw 220 -> 181), 2048 x 4096 x 4096 82 -> 74, 2048 x
+  // 11008 x 4096 191 -> 182, three 4096 x 4096 outputs at 512 tokens (258 tiles of 96
+  // columns) 76 -> 58; where both take the same rounds the narrower tile is faster
+  // (512 x 11008 x 4096 53 vs 60).
   struct Shape {
     int bm, bn;
     double step_us;
   };
-  static const Shape shapes[] = {{256, 96, 0.90}, {256, 64, 0.75}, {128, 128, 0.85},
+  static const Shape shapes[] = {{256, 128, 1.00}, {256, 96, 0.90}, {256, 64, 0.75}, {128, 128, 0.85},
                                  {128, 96, 0.62}, {128, 64, 0.52}};
   const bool swi = s.mode == Epilogue::kSwiGLU;
   const int count = swi ? 1 : s.count;
@@ -683,6 +698,8 @@ GemmConfig gemm_mfma_pick_segs(int M, const LinearSegs& s, int K) {
   double best_us = 1e300;
   for (const Shape& sh : shapes) {
     if (sh.bm == 256 && (M <= 128 || s.layout == WeightLayout::kKN)) continue;  // KN: below
+    // The raw SwiGLU producers (two weights) spill beside 128-column tiles.
+    if (sh.bm == 256 && sh.bn == 128 && swi && s.layout == WeightLayout::kRaw) continue;
     const int cols = swi ? sh.bn / 2 : sh.bn;
     int64_t col_tiles = 0, out_cols = 0;
     for (int i = 0; i < count; ++i) {
@@ -768,7 +785,7 @@ GemmConfig gemm_mfma_pick_kn(int M, int N, int K) {
 hipError_t launch_gemm_mfma_segs(const GemmConfig& c, const float* x, const LinearSegs& s,
                                  int M, int K, const SplitKWorkspace& ws, hipStream_t stream) {
   const bool swi = s.mode == Epilogue::kSwiGLU;
-  if (!gemm_mfma_config_valid(c) || !gemm_mfma_fits(c, M, 0, K) || ws.scratch == nullptr)
+  if (!gemm_mfma_launchable(c) || !gemm_mfma_fits(c, M, 0, K) || ws.scratch == nullptr)
     return hipErrorInvalidValue;
   if (s.count < 1 || s.count > 3 || (swi && s.count != 2))
     return hipErrorInvalidValue;
@@ -792,6 +809,11 @@ hipError_t launch_gemm_mfma_segs(const GemmConfig& c, const float* x, const Line
     case 1096: launch_tile<1, 3>(g, s.mode, s.layout, xf, (uint32_t)xfb, M, K, ws, stream); break;
     case 1128: launch_tile<1, 4>(g, s.mode, s.layout, xf, (uint32_t)xfb, M, K, ws, stream); break;
     case 2064: launch_tile<2, 2>(g, s.mode, s.layout, xf, (uint32_t)xfb, M, K, ws, stream); break;
+    case 2128:
+      if (s.layout == WeightLayout::kKN || (swi && s.layout == WeightLayout::kRaw))
+        return hipErrorInvalidValue;
+      launch_tile<2, 4>(g, s.mode, s.layout, xf, (uint32_t)xfb, M, K, ws, stream);
+      break;
     case 2096: launch_tile<2, 3>(g, s.mode, s.layout, xf, (uint32_t)xfb, M, K, ws, stream); break;
     default: return hipErrorInvalidValue;
   }

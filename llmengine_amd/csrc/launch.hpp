@@ -162,6 +162,8 @@ struct GemmConfig {
 };
 GemmConfig gemm_mfma_pick(int M, int N, int K);
 bool gemm_mfma_config_valid(const GemmConfig& c);
+// Shapes the launcher takes: the valid ones and 256 x 128 (automatic pick only).
+bool gemm_mfma_launchable(const GemmConfig& c);
 SplitKNeed gemm_mfma_workspace(const GemmConfig& c, int M, int N, int K);
 bool gemm_mfma_fits(const GemmConfig& c, int M, int N, int K);
 hipError_t launch_gemm_mfma(const GemmConfig& c, const float* x, const uint8_t* w,

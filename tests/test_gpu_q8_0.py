@@ -678,6 +678,32 @@ def test_linear_c3_prefill_full(dev, orc, N, K):
     assert torch.equal(y_again, y_mfma)
 
 
+@pytest.mark.parametrize("M,N,K", [(300, 12300, 160), (257, 16384, 96), (512, 16321, 64)])
+def test_linear_gemm_wide_tiles(dev, orc, M, N, K):
+    """256 x 128 tiles, taken where they need fewer rounds of workgroups than 256 x 96:
+    ragged rows, columns and last K step, raw and tiled the same bits, a bias, and a
+    tiled SwiGLU on them (its column tiles hold 64 rows of each weight); against the
+    oracle on sampled rows (both operands rounded to bf16: 1e-2)."""
+    note(f"gemm wide tiles M={M} N={N} K={K}")
+    w, x = weight(520, N, K), acts(521, M, K)
+    bias = S.activations(522, (N,), tag=S.TAG_BIAS)
+    dx, dw, db = to_dev(x, dev), to_dev(w, dev), to_dev(bias, dev)
+    import torch
+    dt = torch.empty(capi.tiled_bytes(N, K), dtype=torch.uint8, device=dev)
+    capi.tile(dw, dt, N, K)
+    y, yt, ys = (empty_f32((M, N), dev) for _ in range(3))
+    capi.linear(dx, dw, db, y, M, N, K)
+    capi.linear_tiled(dx, dt, db, yt, M, N, K)
+    capi.linear_swiglu_tiled(dx, dt, dt, ys, M, N, K)
+    got = to_host(y)
+    assert_bitexact(to_host(yt), got, "tiled vs raw")
+    rows = np.unique(np.r_[0, M - 1, np.linspace(0, M - 1, 12).astype(int)])
+    want = orc.linear(np.ascontiguousarray(x[rows]), w, bias, rows.size, N, K)
+    assert rel_l2(got[rows], want) <= 1e-2
+    g = (want - bias).astype(np.float64)
+    assert rel_l2(to_host(ys)[rows], g / (1.0 + np.exp(-g)) * g) <= 1e-2
+
+
 # ----------------------------------------------------------------------------- matmul
 
 def test_matmul_known_answers(dev, golden):
