@@ -709,6 +709,9 @@ GemmConfig gemm_mfma_pick_segs(int M, const LinearSegs& s, int K) {
     const int64_t tiles = col_tiles * ((M + sh.bm - 1) / sh.bm);
     for (int splits = 1; splits <= 4; splits *= 2) {
       if (splits > n_steps) break;
+      // 256 x 128 tiles unsplit only: their partials would outgrow the workspace that
+      // the narrower tiles' calls fit.
+      if (splits > 1 && sh.bm == 256 && sh.bn == 128) break;
       const int64_t rounds = (tiles * splits + 255) / 256;
       const int steps = (n_steps + splits - 1) / splits;
       const double split_us =
