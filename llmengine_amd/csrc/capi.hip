@@ -276,14 +276,16 @@ struct Tune {
   mle::GemmConfig gemm{0, 0, 0};  // 0 fields = automatic
 };
 
-// Whether the graph workspace of (current device, stream) holds `need`.
-bool graph_workspace_holds(const mle::SplitKNeed& need, hipStream_t stream) {
+// What the graph workspace of (current device, stream) holds.
+void graph_workspace_capacity(hipStream_t stream, size_t* bytes, size_t* counters) {
   int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return false;
+  *bytes = *counters = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return;
   std::lock_guard<std::mutex> lock(g_ws_mu);
   const auto it = g_ws.find({dev, stream, true});
-  return it != g_ws.end() && it->second.buf_cap >= need_bytes(need) &&
-         it->second.counter_cap >= need.counters;
+  if (it == g_ws.end()) return;
+  *bytes = it->second.buf_cap;
+  *counters = it->second.counter_cap;
 }
 
 // The launches of linear_mid.hip (mle::linear_mid_pick).  Returns whether the call
@@ -291,20 +293,42 @@ bool graph_workspace_holds(const mle::SplitKNeed& need, hipStream_t stream) {
 // need: a plan names the larger of both, so a workspace sized for a batch serves the
 // smaller steps that take the general path.  Where the K splits' partials do not fit
 // (a caller-fixed workspace, or a captured stream's reservation made for the general
-// path) the launch runs unsplit, which needs no workspace.
+// path) the row tiles go in several launches that reuse it: the same bits.  Where the
+// outputs of a fused launch alone would take another number of K splits, each gets a
+// launch of its own, so that it keeps the single Linear's bits.
 bool run_mid(const char* what, const float* x, const mle::LinearSegs& s, int M, int K,
              const mle::SplitKNeed& general, const Exec& ex, int* rc) {
   mle::MidConfig c = mle::linear_mid_pick(M, s, K);
   if (c.tt == 0 || !mle::linear_mid_fits(M, K)) return false;
+  if (s.mode == mle::Epilogue::kPlain && s.count > 1 && M < 64) {
+    mle::LinearSegs one[3];
+    bool same = true;
+    for (int i = 0; i < s.count; ++i) {
+      one[i] = s;
+      one[i].count = 1;
+      one[i].seg[0] = s.seg[i];
+      same &= mle::linear_mid_pick(M, one[i], K).splits == c.splits;
+    }
+    if (!same) {
+      *rc = MLE_OK;
+      for (int i = 0; i < s.count && *rc == MLE_OK; ++i)
+        (void)run_mid(what, x, one[i], M, K, general, ex, rc);
+      return true;
+    }
+  }
   mle::SplitKNeed need = mle::linear_mid_workspace(c, s, K);
-  const bool short_of_space =
-      need.partial_floats != 0 &&
-      (ex.fixed ? need_bytes(need) > ex.fixed_bytes || need.counters > ex.fixed_counter_count
-                : !ex.planning() && stream_capturing(ex.stream) &&
-                      !graph_workspace_holds(need, ex.stream));
-  if (short_of_space) {
-    c.splits = 1;
-    need = mle::linear_mid_workspace(c, s, K);
+  if (ex.fixed || (!ex.planning() && stream_capturing(ex.stream))) {
+    size_t bytes = ex.fixed_bytes, counters = ex.fixed_counter_count;
+    if (!ex.fixed) graph_workspace_capacity(ex.stream, &bytes, &counters);
+    if (need_bytes(general) > bytes || general.counters > counters) {
+      need = general;  // refused, as on the general path
+    } else if (need_bytes(need) > bytes || need.counters > counters) {
+      c.tiles_per_launch = 1;
+      const mle::SplitKNeed tile = mle::linear_mid_workspace(c, s, K);
+      const size_t tiles = std::min(bytes / need_bytes(tile), counters / tile.counters);
+      if (tiles > 1) c.tiles_per_launch = (int)tiles;  // none: refused below
+      need = mle::linear_mid_workspace(c, s, K);
+    }
   }
   mle::SplitKWorkspace ws;
   std::unique_lock<std::mutex> hold;  // released after the launch is enqueued
@@ -351,14 +375,16 @@ int run_linear(const float* x, const uint8_t* w, const void* bias, float* y, int
                         "hip sgemm_nt Q8_0 launch failed");
   }
   if (path == 2) {
-    mle::GemmConfig c = mle::gemm_mfma_pick(M, N, K);
+    const mle::GemmConfig pick = mle::gemm_mfma_pick(M, N, K);
+    mle::GemmConfig c = pick;
     if (tune.gemm.bm) c.bm = tune.gemm.bm;
     if (tune.gemm.bn) {
       c.bn = tune.gemm.bn;
       if (!tune.gemm.bm && !mle::gemm_mfma_config_valid(c)) c.bm = 128;
     }
     if (tune.gemm.splits) c.splits = tune.gemm.splits;
-    if (!mle::gemm_mfma_launchable(c))
+    const bool own = c.bm == pick.bm && c.bn == pick.bn;
+    if (!(own ? mle::gemm_mfma_launchable(c) : mle::gemm_mfma_config_valid(c)))
       return fail(MLE_INVALID_ARGUMENT, "hip sgemm_nt_q8_0_weight: invalid MFMA GEMM shape (bm " +
                                             std::to_string(c.bm) + ", bn " +
                                             std::to_string(c.bn) + ")");

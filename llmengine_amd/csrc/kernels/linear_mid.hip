@@ -39,6 +39,8 @@
 //   raw                       12288 x 4096  41.6 / 79.8 / 29.9 -> 26.4 / 34.7 / GEMM
 //                              4096 x 4096  21.3 / 41.5 / 18.8 -> 12.9 / 17.8 / 14.1
 //   SwiGLU 2 x 11008 x 4096, tiled, M = 32 / 63:  61.6 / 122.8 -> 33.9 / 51.0
+#include <algorithm>
+
 #include "../launch.hpp"
 #include "../q8_0_device.hpp"
 
@@ -123,6 +125,7 @@ struct MidArgs {
   unsigned grp_end[3];
   int count;
   int swiglu;
+  unsigned tile0;  // first tile of this launch
 };
 
 constexpr int kPhaseBlocks = 4;  // K blocks per phase
@@ -161,7 +164,7 @@ __global__ __launch_bounds__(kNT, 2) void linear_mid_kernel(const float* __restr
                              : args.count == 2 ? args.grp_end[1]
                                                : args.grp_end[2];
   const int RGO = swi ? RG / 2 : RG;  // output groups per wave
-  const unsigned wgrp0 = (blockIdx.x * kWN + wn) * RGO;
+  const unsigned wgrp0 = ((args.tile0 + blockIdx.x) * kWN + wn) * RGO;
   auto group_of = [&](int rg) {  // output group of this wave's row group rg
     return wgrp0 + (unsigned)(swi ? (rg >= RG / 2 ? rg - RG / 2 : rg) : rg);
   };
@@ -595,6 +598,7 @@ constexpr int max_rg(int tt, int parts) { return parts == 3 ? 4 : tt <= 5 ? 3 : 
 
 struct MidGrid {
   unsigned tiles, splits;
+  unsigned tiles_per_launch;
   int phases_per_split;
   MidArgs args;
 };
@@ -604,6 +608,8 @@ MidGrid mid_grid(const MidConfig& c, const LinearSegs& s, int K) {
   const unsigned groups = gr.args.grp_end[gr.args.count - 1];
   const unsigned per = kWN * (gr.args.swiglu ? c.rg / 2 : c.rg);
   gr.tiles = (groups + per - 1) / per;
+  gr.tiles_per_launch = c.tiles_per_launch > 0 ? std::min(gr.tiles, (unsigned)c.tiles_per_launch)
+                                               : gr.tiles;
   const int phases = (K / kBlockElems + kPhaseBlocks - 1) / kPhaseBlocks;
   gr.phases_per_split = (phases + c.splits - 1) / c.splits;
   gr.splits = (unsigned)((phases + gr.phases_per_split - 1) / gr.phases_per_split);
@@ -611,16 +617,24 @@ MidGrid mid_grid(const MidConfig& c, const LinearSegs& s, int K) {
 }
 
 template <int TT, int PARTS, int RG>
-hipError_t launch_mid_k(const MidGrid& gr, WeightLayout layout, const float* x, int M, int K,
+hipError_t launch_mid_k(MidGrid gr, WeightLayout layout, const float* x, int M, int K,
                         const SplitKWorkspace& ws, hipStream_t stream) {
-  const dim3 grid(gr.tiles, gr.splits), block(kNT);
-  if (layout == WeightLayout::kTiled)
-    hipLaunchKernelGGL((linear_mid_kernel<TT, PARTS, RG, int(WeightLayout::kTiled)>), grid, block,
-                       0, stream, x, gr.args, M, K, gr.phases_per_split, ws.partials, ws.counters);
-  else
-    hipLaunchKernelGGL((linear_mid_kernel<TT, PARTS, RG, int(WeightLayout::kRaw)>), grid, block, 0,
-                       stream, x, gr.args, M, K, gr.phases_per_split, ws.partials, ws.counters);
-  return hipGetLastError();
+  const dim3 block(kNT);
+  for (unsigned t0 = 0; t0 < gr.tiles; t0 += gr.tiles_per_launch) {
+    const dim3 grid(std::min(gr.tiles - t0, gr.tiles_per_launch), gr.splits);
+    gr.args.tile0 = t0;
+    if (layout == WeightLayout::kTiled)
+      hipLaunchKernelGGL((linear_mid_kernel<TT, PARTS, RG, int(WeightLayout::kTiled)>), grid,
+                         block, 0, stream, x, gr.args, M, K, gr.phases_per_split, ws.partials,
+                         ws.counters);
+    else
+      hipLaunchKernelGGL((linear_mid_kernel<TT, PARTS, RG, int(WeightLayout::kRaw)>), grid, block,
+                         0, stream, x, gr.args, M, K, gr.phases_per_split, ws.partials,
+                         ws.counters);
+    const hipError_t err = hipGetLastError();
+    if (err != hipSuccess) return err;
+  }
+  return hipSuccess;
 }
 
 template <int TT, int PARTS>
@@ -655,7 +669,8 @@ hipError_t launch_mid_rg(const MidConfig& c, const MidGrid& gr, WeightLayout lay
 // more than 64: 4096 x 11008 at 128 34.9 vs 31.6), and SwiGLU pairs (11008 x 4096 at
 // 64: 40.5 vs 39.8).
 //
-// K splits: by K alone, about 32 blocks each (8 splits past 4096 elements: 896 x 4864
+// K splits: by K alone, about 32 blocks each, none up to 16 blocks, where the 16-token
+// decode needs no workspace either (8 splits past 4096 elements: 896 x 4864
 // at 32 tokens 9.1 us vs 12.0 with 4; 7 at three token tiles, as fast as 8, whose
 // partials stay within the 16-token decode's); one split for weights whose rows alone
 // fill the GPU several times over (3072 groups).  A SwiGLU pair,
@@ -676,7 +691,7 @@ MidConfig linear_mid_pick(int M, const LinearSegs& s, int K) {
   }
   c.parts = M < 64 ? 3 : 1;
   c.tt = M < 64 ? (M + 15) / 16 : M <= 64 ? 4 : M <= 80 ? 5 : M <= 96 ? 6 : 8;
-  c.splits = G >= 3072 || KB <= 8 ? 1 : KB <= 16 ? 2 : KB <= 128 ? 4 : c.tt == 3 ? 7 : 8;
+  c.splits = G >= 3072 || KB <= 16 ? 1 : KB <= 128 ? 4 : c.tt == 3 ? 7 : 8;
   const int rg_max = max_rg(c.tt, c.parts);
   auto grid = [&](int rg) { return (G + kWN * rg - 1) / (kWN * rg) * c.splits; };
   if (swi) {
@@ -697,8 +712,8 @@ SplitKNeed linear_mid_workspace(const MidConfig& c, const LinearSegs& s, int K) 
   SplitKNeed need;
   need.splits = (int)gr.splits;
   if (gr.splits > 1) {
-    need.partial_floats = (size_t)gr.tiles * gr.splits * kWN * c.rg * c.tt * 256;
-    need.counters = (size_t)gr.tiles * kCounterStride;
+    need.partial_floats = (size_t)gr.tiles_per_launch * gr.splits * kWN * c.rg * c.tt * 256;
+    need.counters = (size_t)gr.tiles_per_launch * kCounterStride;
   }
   return need;
 }

@@ -145,6 +145,7 @@ struct MidConfig {
   int parts = 3;   // bf16 parts per activation: 3 (FP32-exact) or 1 (rounded once)
   int rg = 1;      // 16-row groups per wave (SwiGLU: even, half of each weight)
   int splits = 1;  // K splits asked for
+  int tiles_per_launch = 0;  // row tiles a launch, the workspace reused; 0: all in one
 };
 MidConfig linear_mid_pick(int M, const LinearSegs& s, int K);
 bool linear_mid_fits(int M, int K);

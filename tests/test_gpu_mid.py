@@ -159,7 +159,7 @@ def test_mid_split_counters_and_noalloc(dev):
 
 def test_mid_capture_on_a_smaller_reservation(dev):
     """A stream whose graph workspace was reserved for 16 tokens still captures 40: the
-    launch runs unsplit there, with fp32 rounding between it and the eager call."""
+    row tiles share it in several launches, with the eager call's bits."""
     import torch
     M, N, K = 40, 4096, 8192  # 5.5 MB of partials; a reservation holds at least 4 MiB
     note("mid capture on a smaller reservation")
@@ -176,4 +176,30 @@ def test_mid_capture_on_a_smaller_reservation(dev):
         y.fill_(float("nan"))
         g.replay()
         torch.cuda.synchronize()
-        assert rel_l2(to_host(y), to_host(eager)) <= 1e-6
+        assert_bitexact(to_host(y), to_host(eager), "replay vs eager")
+
+
+def test_mid_noalloc_scratch_limit(dev):
+    """K splits whose partials outgrow the no-allocation scratch (33.6 MB at 16400 rows)
+    give mle_q8_0_linear's bits there too."""
+    M, N, K = 63, 16400, 4128
+    note("mid noalloc scratch limit")
+    x, dw = to_dev(S.activations(960, (M, K)), dev), to_dev(weight(961, N, K), dev)
+    y, y2 = empty_f32((M, N), dev), empty_f32((M, N), dev)
+    capi.linear(x, dw, None, y, M, N, K)
+    capi.linear_noalloc(x, dw, None, y2, M, N, K)
+    assert_bitexact(to_host(y2), to_host(y), "noalloc vs linear")
+
+
+def test_mid_multi_past_the_split_bound(dev):
+    """Three outputs of 49152 rows together, each below the bound from which a launch
+    takes no K splits, keep their single Linears' bits."""
+    M, N, K = 20, 16384, 544
+    note("mid multi past the split bound")
+    x = to_dev(S.activations(970, (M, K)), dev)
+    ws = [to_dev(weight(971 + i, N, K), dev) for i in range(3)]
+    ys, one = [empty_f32((M, N), dev) for _ in ws], empty_f32((M, N), dev)
+    capi.linear_multi(x, ws, [None] * 3, ys, [N] * 3, M, K)
+    for w, y in zip(ws, ys):
+        capi.linear(x, w, None, one, M, N, K)
+        assert_bitexact(to_host(y), to_host(one), "fused vs single")
