@@ -944,11 +944,18 @@ int mle_argmax_f32(const float* logits, int rows, int n, int32_t* idx, float* va
   MLE_TRY(check_align(ctx, val, 4, "val"));
   mle::SplitKNeed need;
   need.partial_floats = (size_t)rows * mle::argmax_chunks(n) * 2;  // 64-bit keys
+  need.counters = mle::argmax_counters(rows);
+  if (need.counters != 0 && stream_capturing(stream)) {  // a reservation of bytes alone serves
+    size_t bytes = 0, counters = 0;
+    graph_workspace_capacity(stream, &bytes, &counters);
+    if (need.counters > counters) need.counters = 0;
+  }
   mle::SplitKWorkspace ws;
   std::unique_lock<std::mutex> hold;  // released after the launch is enqueued
   MLE_TRY(get_workspace(need, stream, &ws, &hold));
   return check_launch(mle::launch_argmax(logits, rows, n, idx, val,
-                                         reinterpret_cast<uint64_t*>(ws.partials), stream),
+                                         reinterpret_cast<uint64_t*>(ws.partials),
+                                         need.counters != 0 ? ws.counters : nullptr, stream),
                       "hip argmax launch failed");
 }
 

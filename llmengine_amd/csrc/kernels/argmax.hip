@@ -9,17 +9,27 @@
 // CUDA generator makes before sampling on the host
 // (examples/generate_cuda.cpp:81-94, 305-314).
 //
-// Two launches: pass 1 (grid chunks x rows) reduces a contiguous chunk of a row
-// per workgroup to one 64-bit key; pass 2 reduces a row's chunk keys and
-// decodes the winner.  key = (order(v) << 32) | ~index, where order() maps float
-// bits to unsigned integers in value order, so the largest key is the largest
-// value with the smallest index.  Deterministic; no atomics.
+// A workgroup (grid chunks x rows) reduces a chunk of a row to one 64-bit key.  key =
+// (order(v) << 32) | ~index, where order() maps float bits to unsigned integers in
+// value order, so the largest key is the largest value with the smallest index:
+// deterministic in any order of reduction.  Up to kArgRows rows the chunks' keys meet
+// by an atomic maximum beside the row's counter in the workspace, and the row's last
+// workgroup decodes the winner; more rows (whose counters a default workspace does not
+// hold) write the keys, which a second launch reduces.
+//
+// Bound by latency (152k logits are 0.6 MB): a thread's 8 values are loaded at once
+// (one by one in a loop, each load waited for, and with a second launch for every call, the
+// [1, 151936] pick behind its [151936, 896] Linear took 29.3 us a pair on MI355X; this
+// takes 27.1).
 #include "../launch.hpp"
 
 namespace mle {
 namespace {
 
 constexpr int kArgThreads = 256;
+constexpr int kArgVecs = 2;                              // 4-value loads a thread
+constexpr int kArgPiece = 4 * kArgVecs * kArgThreads;    // 2048 values
+constexpr int kArgRows = 4096 / kCounterStride;          // a default workspace's counters
 
 __device__ __forceinline__ uint64_t arg_key(float v, uint32_t i) {
   if (v != v) return 0;  // NaN: never selected
@@ -52,35 +62,8 @@ __device__ __forceinline__ uint64_t block_max(uint64_t k) {
   return r;
 }
 
-// Pass 1: workgroup (c, r) reduces logits[r, c*chunk : (c+1)*chunk).
-__global__ __launch_bounds__(kArgThreads) void argmax_chunks_kernel(const float* __restrict__ x,
-                                                                   int64_t n, int64_t chunk,
-                                                                   uint64_t* __restrict__ keys) {
-  const int64_t r = blockIdx.y;
-  const int64_t b = (int64_t)blockIdx.x * chunk;
-  const int64_t e = b + chunk < n ? b + chunk : n;
-  const float* row = x + r * n;
-  uint64_t k = 0;
-  for (int64_t i = b + threadIdx.x; i < e; i += kArgThreads) {
-    const uint64_t c = arg_key(row[i], (uint32_t)i);
-    k = c > k ? c : k;
-  }
-  k = block_max(k);
-  if (threadIdx.x == 0) keys[r * gridDim.x + blockIdx.x] = k;
-}
-
-// Pass 2: one workgroup per row over its `chunks` keys.
-__global__ __launch_bounds__(kArgThreads) void argmax_final_kernel(
-    const uint64_t* __restrict__ keys, int chunks, int32_t* __restrict__ idx,
-    float* __restrict__ val) {
-  const int64_t r = blockIdx.x;
-  uint64_t k = 0;
-  for (int i = threadIdx.x; i < chunks; i += kArgThreads) {
-    const uint64_t c = keys[r * chunks + i];
-    k = c > k ? c : k;
-  }
-  k = block_max(k);
-  if (threadIdx.x != 0) return;
+__device__ __forceinline__ void write_winner(uint64_t k, int64_t r, int32_t* __restrict__ idx,
+                                             float* __restrict__ val) {
   if (k == 0) {  // NaN only
     idx[r] = 0;
     if (val) val[r] = __builtin_nanf("");
@@ -94,6 +77,78 @@ __global__ __launch_bounds__(kArgThreads) void argmax_final_kernel(
   }
 }
 
+// Workgroup (c, r) reduces logits[r, c*chunk : (c+1)*chunk), chunk a multiple of
+// kArgPiece.  MEET: the chunks meet in counters[r * kCounterStride] (dwords 0-1 the
+// largest key, 2 the arrivals; zero before and after), else each writes its key.
+template <bool MEET>
+__global__ __launch_bounds__(kArgThreads) void argmax_chunks_kernel(
+    const float* __restrict__ x, int64_t n, int64_t chunk, uint64_t* __restrict__ keys,
+    uint32_t* __restrict__ counters, int32_t* __restrict__ idx, float* __restrict__ val) {
+  const int64_t r = blockIdx.y;
+  const int64_t b = (int64_t)blockIdx.x * chunk;
+  const int64_t e = b + chunk < n ? b + chunk : n;
+  const float* row = x + r * n;
+  uint64_t k = 0;
+  for (int64_t p = b; p < e; p += kArgPiece) {
+    const int64_t i0 = p + 4 * threadIdx.x;
+    float v[kArgVecs][4];
+    if (p + kArgPiece <= e) {  // rows are 4-byte aligned only
+#pragma unroll
+      for (int j = 0; j < kArgVecs; ++j)
+        __builtin_memcpy(v[j], __builtin_assume_aligned(row + i0 + j * 4 * kArgThreads, 4), 16);
+    } else {
+#pragma unroll
+      for (int j = 0; j < kArgVecs; ++j)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const int64_t i = i0 + j * 4 * kArgThreads + c;
+          const float u = row[i < e ? i : e - 1];
+          v[j][c] = i < e ? u : __builtin_nanf("");
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < kArgVecs; ++j)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const uint64_t key = arg_key(v[j][c], (uint32_t)(i0 + j * 4 * kArgThreads + c));
+        k = key > k ? key : k;
+      }
+  }
+  k = block_max(k);
+  if (threadIdx.x != 0) return;
+  if constexpr (!MEET) {
+    keys[r * gridDim.x + blockIdx.x] = k;
+  } else {
+    uint32_t* const count = counters + r * kCounterStride + 2;
+    uint64_t* const best = reinterpret_cast<uint64_t*>(counters + r * kCounterStride);
+    (void)__hip_atomic_fetch_max(best, k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_s_waitcnt(0);  // the maximum is in before the arrival counts
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    if (__hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) !=
+        gridDim.x - 1)
+      return;
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    k = __hip_atomic_exchange(best, (uint64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    write_winner(k, r, idx, val);
+  }
+}
+
+// More rows: one workgroup per row over its `chunks` keys.
+__global__ __launch_bounds__(kArgThreads) void argmax_final_kernel(
+    const uint64_t* __restrict__ keys, int chunks, int32_t* __restrict__ idx,
+    float* __restrict__ val) {
+  const int64_t r = blockIdx.x;
+  uint64_t k = 0;
+  for (int i = threadIdx.x; i < chunks; i += kArgThreads) {
+    const uint64_t c = keys[r * chunks + i];
+    k = c > k ? c : k;
+  }
+  k = block_max(k);
+  if (threadIdx.x == 0) write_winner(k, r, idx, val);
+}
+
 }  // namespace
 
 int argmax_chunks(int64_t n) {
@@ -102,13 +157,24 @@ int argmax_chunks(int64_t n) {
   return (int)(c < 1 ? 1 : c > 256 ? 256 : c);
 }
 
+size_t argmax_counters(int rows) {
+  return rows <= kArgRows ? (size_t)rows * kCounterStride : 0;
+}
+
 hipError_t launch_argmax(const float* x, int rows, int64_t n, int32_t* idx, float* val,
-                         uint64_t* keys, hipStream_t stream) {
+                         uint64_t* keys, uint32_t* counters, hipStream_t stream) {
   if (rows <= 0 || n <= 0 || n > 0x7fffffff || rows > 65535) return hipErrorInvalidValue;
   const int chunks = argmax_chunks(n);
-  const int64_t chunk = (n + chunks - 1) / chunks;
-  hipLaunchKernelGGL(argmax_chunks_kernel, dim3((unsigned)chunks, (unsigned)rows),
-                     dim3(kArgThreads), 0, stream, x, n, chunk, keys);
+  const int64_t pieces = (n + kArgPiece - 1) / kArgPiece;
+  const int64_t chunk = (pieces + chunks - 1) / chunks * kArgPiece;
+  const dim3 grid((unsigned)chunks, (unsigned)rows);
+  if (counters != nullptr) {
+    hipLaunchKernelGGL(argmax_chunks_kernel<true>, grid, dim3(kArgThreads), 0, stream, x, n, chunk,
+                       keys, counters, idx, val);
+    return hipGetLastError();
+  }
+  hipLaunchKernelGGL(argmax_chunks_kernel<false>, grid, dim3(kArgThreads), 0, stream, x, n, chunk,
+                     keys, counters, idx, val);
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) return err;
   hipLaunchKernelGGL(argmax_final_kernel, dim3((unsigned)rows), dim3(kArgThreads), 0, stream,

@@ -194,10 +194,12 @@ hipError_t launch_matmul(const float* a, const uint8_t* b, float* c, int M, int 
                          float* partials, uint32_t* counters, hipStream_t stream);
 
 // Greedy argmax of `rows` rows of n fp32 logits: idx (and val, if non-null) per
-// row; `keys` is a workspace of rows * argmax_chunks(n) 64-bit entries.
+// row; `keys` is a workspace of rows * argmax_chunks(n) 64-bit entries;
+// with `counters` (argmax_counters(rows) of them, zero) it takes one launch, else two.
 int argmax_chunks(int64_t n);
+size_t argmax_counters(int rows);
 hipError_t launch_argmax(const float* x, int rows, int64_t n, int32_t* idx, float* val,
-                         uint64_t* keys, hipStream_t stream);
+                         uint64_t* keys, uint32_t* counters, hipStream_t stream);
 
 // Top-n tokens of `rows` rows of n fp32 logits with their softmax
 // probabilities (temperature applied when > 0 and != 1): ids / probs are

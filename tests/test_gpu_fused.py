@@ -172,6 +172,41 @@ def test_argmax_matches_first_maximum(dev, rows, n):
     assert np.array_equal(val.cpu().numpy(), x[np.arange(rows), want])
 
 
+@pytest.mark.parametrize("rows,n", [(1, 1), (3, 2047), (2, 2048), (2, 2049), (5, 4097),
+                                    (128, 2050), (129, 2050), (1, 524289), (2, 600001)])
+def test_argmax_chunk_edges(dev, rows, n):
+    """The maximum at the ends of chunks and rows, rows of any 4-byte alignment, on both
+    sides of the one-launch bound; back-to-back calls and replays of a capture leave the
+    shared counters clean."""
+    import torch
+    note(f"argmax chunk edges rows={rows} n={n}")
+    x = S.activations(700, (rows, n))
+    places = [0, n - 1, min(n - 1, 2047), min(n - 1, 2048), n // 2]
+    wants, devs = [], []
+    for k in range(3):
+        for r in range(rows):
+            x[r, places[(r + k) % 5]] = 20.0 + k
+        wants.append(first_argmax(x))
+        devs.append(to_dev(x, dev))
+    idx, val = torch.empty(rows, dtype=torch.int32, device=dev), empty_f32((rows,), dev)
+    for k in (0, 1, 2, 0):
+        capi.argmax(devs[k], rows, n, idx, val)
+        assert idx.cpu().numpy().tolist() == wants[k].tolist()
+        assert to_host(val).tolist() == [20.0 + k] * rows
+    st = torch.cuda.Stream()
+    capi.workspace_reserve(16 * rows * 256, 0, stream=st)  # bytes alone are enough
+    g = torch.cuda.CUDAGraph()
+    y = devs[0].clone()
+    with torch.cuda.graph(g, stream=st):
+        capi.argmax(y, rows, n, idx, val, stream=st)
+    for k in (1, 2, 0):
+        y.copy_(devs[k])
+        g.replay()
+        capi.argmax(devs[k], rows, n, idx, val)
+        g.replay()
+        assert idx.cpu().numpy().tolist() == wants[k].tolist()
+
+
 def test_argmax_ties_signed_zero_and_nan(dev):
     import torch
     n = 10_000
