@@ -14,7 +14,7 @@
 // the order here is the logit, then the index.
 //
 // Two launches.  Pass 1 (grid chunks x rows, 256 threads) streams a 2048-value chunk:
-// its maximum, its sum of exp(value - maximum), a NaN flag, and the maxima of its
+// its maximum (+Inf where it holds a NaN), its sum of exp(value - maximum), and the maxima of its
 // groups of 64 values (1024 / top_n for fewer than 16 tokens, so that the workspace
 // stays within 2 top_n floats a chunk).  Pass 2 (one 1024-thread workgroup per row)
 // merges the chunk statistics in a fixed order (max, then the sum of sum_c *
@@ -38,8 +38,9 @@
 //
 // Latency bounds it, not bytes (8 rows x 152k logits are 4.9 MB).  Selecting top_n keys
 // in every chunk instead (a radix select per chunk, then one over 75 x top_n
-// candidates) took 31.7 us for 8 rows at top_n 40 and 28.5 for one (MI355X); this
-// takes 13.5 and 12.8.
+// candidates) took 31.6 us for 8 rows at top_n 40 (MI355X); this takes 12.5.  Pass 2
+// issues all its loads of a stage before it uses one, and a NaN travels as an infinite
+// maximum instead of through a reduction of its own (13.7 us otherwise).
 #include "../launch.hpp"
 
 namespace mle {
@@ -242,16 +243,16 @@ __device__ __forceinline__ uint32_t dist_bin(float mx, float v) {
 }
 
 // Pass 1: workgroup (c, r) over logits[r, c * kChunk : (c + 1) * kChunk).
-// maxima: [row][chunk][gpc] group maxima; stats: [row][chunk] x {max, sum, nan, rest of
-// the sum}.
+// maxima: [row][chunk][gpc] group maxima; stats: [row][chunk] x {max (+Inf beside a
+// NaN), sum, rest of the sum, 0}.
+typedef float f4 __attribute__((ext_vector_type(4), aligned(4)));  // rows are 4-byte aligned
+
 __global__ __launch_bounds__(kP1Threads) void topk_chunks_kernel(
     const float* __restrict__ x, int64_t n, int gpc, float inv_temp, int scale,
     float* __restrict__ maxima, float* __restrict__ stats) {
   __shared__ float gmax[kChunk / kGroup];
   __shared__ float fpart[kP1Threads / 64];
   __shared__ double dpart[kP1Threads / 64];
-  __shared__ int ipart[kP1Threads / 64];
-  typedef float f4 __attribute__((ext_vector_type(4), aligned(4)));  // rows are 4-byte aligned
   const int64_t r = blockIdx.y;
   const int64_t b = (int64_t)blockIdx.x * kChunk;
   const float* row = x + r * n;
@@ -259,7 +260,7 @@ __global__ __launch_bounds__(kP1Threads) void topk_chunks_kernel(
   static_assert(kGroup == 64, "16 lanes x 4 values are a group");
   float v[PER];
   float mx = -__builtin_inff();
-  int nan = 0;
+  bool nan = false;
 #pragma unroll
   for (int j = 0; j < Q; ++j) {
     const int64_t i = b + 4 * ((int)threadIdx.x + kP1Threads * j);
@@ -284,8 +285,8 @@ __global__ __launch_bounds__(kP1Threads) void topk_chunks_kernel(
     if ((threadIdx.x & 15) == 0) gmax[threadIdx.x / 16 + kP1Threads / 16 * j] = g;
     mx = fmaxf(mx, g);
   }
+  if (nan) mx = __builtin_inff();  // the row is uniform either way
   mx = block_reduce<kP1Threads>(mx, [](float a, float c) { return fmaxf(a, c); }, fpart);
-  nan = block_reduce<kP1Threads>(nan, [](int a, int c) { return a | c; }, ipart);
   double sum = 0.0;  // one chunk can hold most of the row's sum: its rounding is the row's
   if (mx > -__builtin_inff() && mx < __builtin_inff()) {
 #pragma unroll
@@ -303,8 +304,8 @@ __global__ __launch_bounds__(kP1Threads) void topk_chunks_kernel(
   if (threadIdx.x == 0) {
     stats[slot * 4 + 0] = mx;
     stats[slot * 4 + 1] = (float)sum;
-    stats[slot * 4 + 2] = nan ? 1.0f : 0.0f;
-    stats[slot * 4 + 3] = (float)(sum - (float)sum);
+    stats[slot * 4 + 2] = (float)(sum - (float)sum);
+    stats[slot * 4 + 3] = 0.0f;
   }
 }
 
@@ -321,7 +322,6 @@ __global__ __launch_bounds__(kP2Threads) void topk_final_kernel(
   __shared__ int list[kP2Keys / kGroup];
   __shared__ float fpart[kP2Threads / 64];
   __shared__ double dpart[kP2Threads / 64];
-  __shared__ int ipart[kP2Threads / 64];
   __shared__ uint32_t wsum[kP2Threads / 64];
   __shared__ uint32_t bin_at, groups_in, nlist;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -334,20 +334,22 @@ __global__ __launch_bounds__(kP2Threads) void topk_final_kernel(
   const int groups = (int)((n + ((int64_t)1 << gshift) - 1) >> gshift);
   const float* mrow = maxima + r * (int64_t)total_max;
   float gv[GPT];
+  if (gm == 1) {  // all loads in flight
 #pragma unroll
-  for (int e = 0; e < GPT; ++e) {
-    const int gi = tid + kP2Threads * e;
-    float g = -__builtin_inff();
-    if (gi < groups)
-      for (int j = 0; j < gm && gi * gm + j < total_max; ++j) g = fmaxf(g, mrow[gi * gm + j]);
-    gv[e] = g;
+    for (int e = 0; e < GPT; ++e) gv[e] = mrow[min(tid + kP2Threads * e, groups - 1)];
+  } else {
+#pragma unroll
+    for (int e = 0; e < GPT; ++e) {
+      const int gi = tid + kP2Threads * e;
+      float g = -__builtin_inff();
+      if (gi < groups)
+        for (int j = 0; j < gm && gi * gm + j < total_max; ++j) g = fmaxf(g, mrow[gi * gm + j]);
+      gv[e] = g;
+    }
   }
-  float mx = -__builtin_inff();
-  int bad = 0;
-  for (int c = tid; c < chunks; c += kP2Threads) {
-    mx = fmaxf(mx, st[c * 4 + 0]);
-    bad |= st[c * 4 + 2] != 0.0f;
-  }
+  const f4 st0 = *reinterpret_cast<const f4*>(st + 4 * min(tid, chunks - 1));
+  float mx = st0.x;
+  for (int c = tid + kP2Threads; c < chunks; c += kP2Threads) mx = fmaxf(mx, st[c * 4]);
   for (int i = tid; i < kBins / 4; i += kP2Threads)
     reinterpret_cast<uint4*>(hist)[i] = uint4{0u, 0u, 0u, 0u};
   if (tid == 0) {
@@ -357,17 +359,22 @@ __global__ __launch_bounds__(kP2Threads) void topk_final_kernel(
     sm.ncand = 0;
   }
   mx = block_reduce<kP2Threads>(mx, [](float a, float c) { return fmaxf(a, c); }, fpart);
-  bad = block_reduce<kP2Threads>(bad, [](int a, int c) { return a | c; }, ipart);
   double sum = 0.0;
   const bool finite_max = mx > -__builtin_inff() && mx < __builtin_inff();
   if (finite_max) {
-    for (int c = tid; c < chunks; c += kP2Threads) {
-      const float mc = st[c * 4 + 0];
-      if (mc > -__builtin_inff()) sum += ((double)st[c * 4 + 1] + st[c * 4 + 3]) * exp((double)mc - (double)mx);
-    }
+    // The first bin B at which kk groups have a maximum within it (scanned below).
+#pragma unroll
+    for (int e = 0; e < GPT; ++e)
+      if (tid + kP2Threads * e < groups) atomicAdd(&hist[dist_bin(mx, gv[e])], 1u);
+    auto add = [&](const f4 c) {
+      if (c.x > -__builtin_inff()) sum += ((double)c.y + c.z) * exp((double)c.x - (double)mx);
+    };
+    if (tid < chunks) add(st0);
+    for (int c = tid + kP2Threads; c < chunks; c += kP2Threads)
+      add(*reinterpret_cast<const f4*>(st + c * 4));
   }
   sum = block_reduce<kP2Threads>(sum, [](double a, double c) { return a + c; }, dpart);
-  const bool uniform = bad || !finite_max || !(sum > 0.0) || !(sum < __builtin_inf());
+  const bool uniform = !finite_max || !(sum > 0.0) || !(sum < __builtin_inf());
   int32_t* oid = ids + r * kk;
   float* opr = probs + r * kk;
   if (uniform) {
@@ -378,11 +385,6 @@ __global__ __launch_bounds__(kP2Threads) void topk_final_kernel(
     }
     return;
   }
-  // The first bin B at which kk groups have a maximum within it.
-#pragma unroll
-  for (int e = 0; e < GPT; ++e)
-    if (tid + kP2Threads * e < groups) atomicAdd(&hist[dist_bin(mx, gv[e])], 1u);
-  __syncthreads();
   {
     constexpr int BPT = kBins / kP2Threads;
     uint32_t h[BPT], local = 0;
@@ -436,15 +438,24 @@ __global__ __launch_bounds__(kP2Threads) void topk_final_kernel(
   constexpr int PER = kP2Keys / kP2Threads;
   const int total = (int)(ngroups << gshift);
   const float* row = x + r * n;
+  auto index_of = [&](int j) {
+    return ((int64_t)list[j >> gshift] << gshift) + (j & ((1 << gshift) - 1));
+  };
   uint64_t key[PER];
+  float val[PER];
+#pragma unroll
+  for (int e = 0; e < PER; ++e) {  // all loads in flight
+    val[e] = 0.0f;
+    if (kP2Threads * e < total) val[e] = row[min(index_of(min(tid + kP2Threads * e, total - 1)), n - 1)];
+  }
 #pragma unroll
   for (int e = 0; e < PER; ++e) {
     const int j = tid + kP2Threads * e;
     key[e] = 0;
     if (j < total) {
-      const int64_t i = ((int64_t)list[j >> gshift] << gshift) + (j & ((1 << gshift) - 1));
+      const int64_t i = index_of(j);
       if (i < n) {
-        float t = row[i];
+        float t = val[e];
         if (scale) t *= inv_temp;
         if (dist_bin(mx, t) <= bin) {
           key[e] = topk_key(t, (uint32_t)i);
