@@ -292,8 +292,11 @@ int mle_q8_0_linear_multi_tiled(const float* x, int count, const uint8_t* const*
  *   output sizes N[0..count), input size K, on raw (tiled == 0) or 16-row
  *   tiled weights (0 / 0 for launches that need none: the FP32 GEMVs, and the
  *   decode of tiled plain Linears by whole row ranges), or MLE_OP_MATMUL
- *   (count 1, mle_q8_0_matmul: A [M, K], B [K, N[0]]; tiled ignored).  Launches
- *   nothing.  Errors: NULL outputs / N, M or K or an
+ *   (count 1, mle_q8_0_matmul: A [M, K], B [K, N[0]]; tiled ignored).  Above 16
+ *   tokens it is the most that any call of 1 to M tokens on these weights uses, so
+ *   one reservation made for the longest prompt holds the decode steps and the
+ *   shorter prompts (a MatMul: of 1 to M rows of A up to 8 and from 64, of 9 to M
+ *   rows between).  Launches nothing.  Errors: NULL outputs / N, M or K or an
  *   N <= 0, a bad count or op -> InvalidArgument; K % 32 != 0 (MatMul: or
  *   N % 32 != 0) -> Unsupported.
  * mle_workspace_reserve: grows the eager and the graph workspace of (current

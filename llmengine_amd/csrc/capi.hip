@@ -593,6 +593,15 @@ int noalloc_scratch(hipStream_t stream, uint8_t** base) {
   return MLE_OK;
 }
 
+// Workspace of a MatMul on the kernels of matmul.hip.
+mle::SplitKNeed matmul_need(int M, int N, int K) {
+  const mle::MatmulNeed mm = mle::matmul_workspace(M, N, K);
+  mle::SplitKNeed need;
+  need.partial_floats = mm.partial_floats;
+  need.counters = mm.counters;
+  return need;
+}
+
 // MatMul from 64 rows of A on the bf16 MFMA GEMM (B[K, N] dequantised
 // transposed into its W tile); below that, and where B's offsets would not fit
 // 32 bits, the FP32 kernel of matmul.hip.  Fills the GEMM's tile choice and
@@ -604,6 +613,42 @@ bool matmul_on_gemm(int M, int N, int K, mle::GemmConfig* c, mle::LinearSegs* s)
   s->layout = mle::WeightLayout::kKN;
   *c = mle::gemm_mfma_pick_kn(M, N, K);
   return mle::gemm_mfma_fits(*c, M, N, K) && mle::gemm_mfma_kn_fits(*s, K);
+}
+
+// What a plan for M tokens reserves: a decode step's own need up to 16 tokens; beyond
+// that, whatever any call of fewer tokens on the same weights takes, so that a workspace
+// sized for a serving loop's longest prompt holds its decode steps and shorter prompts
+// (their launches may split K where the longest one's does not).  `plan_at` records the
+// need of one token count; each is looked at up to 128, where the paths change, and the
+// GEMM's by row tiles beyond.
+template <typename F>
+int plan_linear(const mle::LinearSegs& s, int M, int K, const Exec& ex, F plan_at) {
+  MLE_TRY(plan_at(M));
+  if (M <= 16) return ok();
+  for (int m = 1; m <= std::min(M, 128); ++m) (void)plan_at(m);  // a refused one needs nothing
+  if (M >= 64) {
+    mle::SplitKWorkspace ws;
+    std::unique_lock<std::mutex> hold;
+    (void)workspace_for(mle::gemm_mfma_workspace_up_to(M, s, K), ex, &ws, &hold);
+  }
+  return ok();
+}
+
+// The MatMul's: up to 8 rows of A (splits that meet by counters), 9 to 63 (second
+// launches, no counters) and 64 or more (the bf16 GEMM, or matmul.hip for an A that is
+// not 16-byte aligned) each name what the fewer rows of their range need, 64 or more also
+// what all of the others do.
+void plan_matmul(int M, int N, int K, const Exec& ex) {
+  mle::SplitKWorkspace ws;
+  std::unique_lock<std::mutex> hold;
+  mle::GemmConfig gc;
+  mle::LinearSegs gs;
+  for (int m = M >= 9 && M < 64 ? 9 : 1; m <= std::min(M, 63); ++m)
+    (void)workspace_for(matmul_need(m, N, K), ex, &ws, &hold);
+  if (M < 64) return;
+  (void)workspace_for(matmul_need(M, N, K), ex, &ws, &hold);
+  if (matmul_on_gemm(M, N, K, &gc, &gs))
+    (void)workspace_for(mle::gemm_mfma_workspace_up_to(M, gs, K), ex, &ws, &hold);
 }
 
 }  // namespace
@@ -778,13 +823,19 @@ int mle_q8_0_linear_noalloc(const float* x, const uint8_t* w_q8_0, const float* 
     plan.fixed_counter_count = kNoAllocCounters;
     MLE_TRY(run_linear(x, w_q8_0, bias, y, M, N, K, 0, Tune{}, plan));
   }
-  if (bytes > kNoAllocBytes || counters > kNoAllocCounters)
+  if (bytes > kNoAllocBytes || counters > kNoAllocCounters) {
+    size_t most = 0, most_counters = 0;
+    (void)mle_q8_0_workspace_size(MLE_OP_LINEAR, M, 1, &N, K, 0, &most, &most_counters);
     return fail(MLE_UNSUPPORTED,
                 "hip linear_noalloc: this shape needs " + std::to_string(bytes) +
                     " bytes and " + std::to_string(counters) +
                     " counters of scratch; the no-allocation entry point holds " +
                     std::to_string(kNoAllocBytes) + " bytes and " +
-                    std::to_string(kNoAllocCounters) + " counters (use mle_q8_0_linear)");
+                    std::to_string(kNoAllocCounters) + " counters (use mle_q8_0_linear; a " +
+                    "reservation for up to " + std::to_string(M) + " tokens is " +
+                    std::to_string(most) + " bytes and " + std::to_string(most_counters) +
+                    " counters)");
+  }
   Exec ex;
   ex.stream = stream;
   ex.fixed = true;  // launches needing no workspace get none
@@ -811,16 +862,18 @@ int mle_q8_0_workspace_size(int op, int M, int count, const int* N, int K, int t
   MLE_TRY(check_positive(ctx, K, "K"));
   if (K % 32 != 0)
     return fail(MLE_UNSUPPORTED, std::string("hip ") + ctx + " requires K to be a multiple of 32");
-  const mle::WeightLayout layout = tiled ? mle::WeightLayout::kTiled : mle::WeightLayout::kRaw;
+  mle::LinearSegs s;
+  s.layout = tiled ? mle::WeightLayout::kTiled : mle::WeightLayout::kRaw;
   Exec ex;
   ex.plan_bytes = bytes;
   ex.plan_counters = counters;
-  mle::LinearSegs s;
-  s.layout = layout;
   if (op == MLE_OP_LINEAR) {
     if (count != 1) return fail(MLE_INVALID_ARGUMENT, std::string("hip ") + ctx + ": a Linear has count 1");
     MLE_TRY(check_positive(ctx, N[0], "N"));
-    return run_linear(nullptr, nullptr, nullptr, nullptr, M, N[0], K, 0, Tune{}, ex, layout);
+    s.seg[0].N = N[0];
+    return plan_linear(s, M, K, ex, [&](int m) {
+      return run_linear(nullptr, nullptr, nullptr, nullptr, m, N[0], K, 0, Tune{}, ex, s.layout);
+    });
   }
   if (op == MLE_OP_LINEAR_SWIGLU) {
     if (count != 2 || N[0] != N[1])
@@ -830,7 +883,7 @@ int mle_q8_0_workspace_size(int op, int M, int count, const int* N, int K, int t
     s.mode = mle::Epilogue::kSwiGLU;
     s.count = 2;
     s.seg[0].N = s.seg[1].N = N[0];
-    return run_segs(ctx, nullptr, s, M, K, ex);
+    return plan_linear(s, M, K, ex, [&](int m) { return run_segs(ctx, nullptr, s, m, K, ex); });
   }
   if (op == MLE_OP_LINEAR_MULTI) {
     if (count < 1 || count > 3)
@@ -840,27 +893,14 @@ int mle_q8_0_workspace_size(int op, int M, int count, const int* N, int K, int t
       MLE_TRY(check_positive(ctx, N[i], "N"));
       s.seg[i].N = N[i];
     }
-    return run_segs(ctx, nullptr, s, M, K, ex);
+    return plan_linear(s, M, K, ex, [&](int m) { return run_segs(ctx, nullptr, s, m, K, ex); });
   }
   if (op == MLE_OP_MATMUL) {
     if (count != 1) return fail(MLE_INVALID_ARGUMENT, std::string("hip ") + ctx + ": a MatMul has count 1");
     MLE_TRY(check_positive(ctx, N[0], "N"));
     if (N[0] % 32 != 0)
       return fail(MLE_UNSUPPORTED, std::string("hip ") + ctx + " requires a MatMul's N to be a multiple of 32");
-    mle::GemmConfig gc;
-    mle::LinearSegs gs;
-    if (matmul_on_gemm(M, N[0], K, &gc, &gs)) {
-      const mle::SplitKNeed need = mle::gemm_mfma_workspace_segs(gc, M, gs, K);
-      *bytes = need_bytes(need);
-      *counters = need.counters;
-      return ok();
-    }
-    const mle::MatmulNeed mm = mle::matmul_workspace(M, N[0], K);
-    mle::SplitKNeed need;
-    need.partial_floats = mm.partial_floats;
-    need.counters = mm.counters;
-    *bytes = need_bytes(need);
-    *counters = need.counters;
+    plan_matmul(M, N[0], K, ex);
     return ok();
   }
   return fail(MLE_INVALID_ARGUMENT, std::string("hip ") + ctx + ": unknown op " + std::to_string(op));
@@ -1016,13 +1056,9 @@ int mle_q8_0_matmul(const float* a, const uint8_t* b_q8_0, float* c, int M, int 
     return check_launch(mle::launch_gemm_mfma_segs(gc, a, gs, M, K, ws, stream),
                         "hip sgemm Q8_0 launch failed");
   }
-  const mle::MatmulNeed mm = mle::matmul_workspace(M, N, K);
-  mle::SplitKNeed need;
-  need.partial_floats = mm.partial_floats;
-  need.counters = mm.counters;
   mle::SplitKWorkspace ws;
   std::unique_lock<std::mutex> hold;  // released after the launch is enqueued
-  MLE_TRY(get_workspace(need, stream, &ws, &hold));
+  MLE_TRY(get_workspace(matmul_need(M, N, K), stream, &ws, &hold));
   return check_launch(
       mle::launch_matmul(a, b_q8_0, c, M, N, K, ws.partials, ws.counters, stream),
       "hip sgemm Q8_0 launch failed");

@@ -73,6 +73,7 @@
 #include "../launch.hpp"
 #include "../q8_0_device.hpp"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace mle {
@@ -757,6 +758,33 @@ SplitKNeed gemm_mfma_workspace_segs(const GemmConfig& c, int M, const LinearSegs
   need.counters = g.splits > 1 ? tiles : 0;
   need.scratch_bytes = (xf_bytes_of(M, K) + kScratchAlign - 1) / kScratchAlign * kScratchAlign;
   return need;
+}
+
+// Tokens that take the same numbers of row tiles have the same launches to choose from,
+// their estimates linear in the tokens: a launch picked at both ends of a range is picked
+// within it, and its bytes are largest at the upper end.
+static void need_between(int lo, int hi, const LinearSegs& s, int K, SplitKNeed* most) {
+  const GemmConfig a = gemm_mfma_pick_segs(lo, s, K), b = gemm_mfma_pick_segs(hi, s, K);
+  const bool same = a.bm == b.bm && a.bn == b.bn && a.splits == b.splits;
+  if (!same && hi - lo > 1) {
+    need_between(lo, (lo + hi) / 2, s, K, most);
+    need_between((lo + hi) / 2, hi, s, K, most);
+    return;
+  }
+  for (const int m : {lo, hi}) {
+    if (same && m != hi) continue;
+    const SplitKNeed n = gemm_mfma_workspace_segs(m == hi ? b : a, m, s, K);
+    const size_t partials = (n.partial_floats * sizeof(float) + 255) / 256 * 256;
+    most->scratch_bytes = std::max(most->scratch_bytes, partials + n.scratch_bytes);
+    most->counters = std::max(most->counters, n.counters);
+  }
+}
+
+SplitKNeed gemm_mfma_workspace_up_to(int M, const LinearSegs& s, int K) {
+  SplitKNeed most;
+  for (int64_t end = 128; end - 128 < M; end += 128)
+    need_between((int)std::max<int64_t>(64, end - 127), (int)std::min<int64_t>(M, end), s, K, &most);
+  return most;
 }
 
 SplitKNeed gemm_mfma_workspace(const GemmConfig& c, int M, int N, int K) {

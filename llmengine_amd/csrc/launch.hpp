@@ -173,6 +173,8 @@ hipError_t launch_gemm_mfma(const GemmConfig& c, const float* x, const uint8_t* 
 // Segmented / fused form (kSwiGLU: BN/2 rows of each weight per tile).
 GemmConfig gemm_mfma_pick_segs(int M, const LinearSegs& s, int K);
 SplitKNeed gemm_mfma_workspace_segs(const GemmConfig& c, int M, const LinearSegs& s, int K);
+// Bytes (as scratch_bytes) and counters that hold the pick's launch of any 64 to M tokens.
+SplitKNeed gemm_mfma_workspace_up_to(int M, const LinearSegs& s, int K);
 hipError_t launch_gemm_mfma_segs(const GemmConfig& c, const float* x, const LinearSegs& s,
                                  int M, int K, const SplitKWorkspace& ws, hipStream_t stream);
 // Whether a MatMul (layout kKN: one plain segment, seg[0].w = B[K, N]) fits the

@@ -399,3 +399,26 @@ def test_workspace_size_matches_launch_plan():
     assert code == 1 and "equal N" in msg
     code, msg, _, _ = capi.workspace_size_status(7, 1, [64], 64)
     assert code == 1 and "unknown op" in msg
+
+
+@pytest.mark.parametrize("op,Ns,K,M", [
+    (capi.OP_LINEAR, [11008], 4096, 1536), (capi.OP_LINEAR, [4096], 11008, 2048),
+    (capi.OP_LINEAR, [4096], 4096, 1024), (capi.OP_LINEAR, [12288], 4096, 512),
+    (capi.OP_LINEAR, [4096], 11008, 128), (capi.OP_LINEAR, [5120], 5120, 128),
+    (capi.OP_LINEAR, [4864], 896, 2048), (capi.OP_LINEAR, [151936], 896, 63),
+    (capi.OP_LINEAR_MULTI, [4096, 1024, 1024], 4096, 1024),
+    (capi.OP_LINEAR_SWIGLU, [11008, 11008], 4096, 2048),
+    (capi.OP_LINEAR_SWIGLU, [4864, 4864], 896, 300),
+    (capi.OP_MATMUL, [65536], 4096, 8), (capi.OP_MATMUL, [11008], 4096, 63),
+    (capi.OP_MATMUL, [4096], 4096, 512), (capi.OP_MATMUL, [11008], 4096, 600)])
+def test_workspace_plan_covers_fewer_tokens(op, Ns, K, M):
+    """A reservation for a serving loop's longest prompt holds its decode steps and its
+    shorter prompts: bytes and counters of a plan above 16 tokens (the MatMul's: within
+    1-8, within 9-63, and above) are at least those of every plan for fewer tokens, also
+    where the longest prompt's own launch splits no K and takes no counters."""
+    first = 9 if op == capi.OP_MATMUL and 9 <= M < 64 else 1
+    for tiled in (False, True):
+        b, c = capi.workspace_size(op, M, Ns, K, tiled)
+        needs = {m: capi.workspace_size(op, m, Ns, K, tiled) for m in range(first, M)}
+        short = {m: n for m, n in needs.items() if n[0] > b or n[1] > c}
+        assert not short, (b, c, len(short), list(short.items())[:3])
