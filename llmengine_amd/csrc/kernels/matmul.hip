@@ -13,7 +13,7 @@
 // instead):
 //   * one or two rows of A: the half-block kernel below, lanes
 //     reading 16-byte pieces of whole blocks along a B row, fp32 FMAs;
-//   * more: the MFMA kernel below, up to 64 rows a launch, B read once.
+//   * more: the MFMA kernel below, B read once per tile of up to 64 rows.
 // Where column tiles alone leave the GPU's 256 CUs short of work, K is spread over S
 // workgroups per tile.  Up to 8 rows of A they meet through a tile counter (a second
 // launch costs the host as much as such a call takes: 4 x 1632 x 2272 10.6 us a call with
@@ -65,7 +65,7 @@ constexpr int kMfWaves = 8;
 constexpr int kMfNT = 64 * kMfWaves;
 
 struct MfGrid {
-  unsigned tiles, splits;
+  unsigned tiles, splits, row_tiles;
   int tt, nbw, steps_per_split;
 };
 
@@ -75,11 +75,15 @@ MfGrid mf_grid(int M, int N, int K) {
   if (g.tt > 4) g.tt = 4;
   g.nbw = g.tt <= 2 ? 4 : 2;
   g.tiles = (unsigned)((N / kBlockElems + g.nbw - 1) / g.nbw);
+  // More than 64 rows (an A that is not 16-byte aligned, or past the GEMM's offsets): all
+  // row tiles in one launch.  A launch a tile took 4055 x 224 x 160 418 us against 28 on
+  // fp32 FMAs; in one it takes 7.4 (2048 x 4096 x 4096 704 -> 450, MI355X).
+  g.row_tiles = (unsigned)((M + 16 * g.tt - 1) / (16 * g.tt));
   const int steps = K / kBlockElems;
   // At most two workgroups a CU at one token tile (126 registers), else one; each wave
   // at least one K step.  Rounded down: a third round for a few workgroups costs more
   // (11008 x 4096 at 16 rows: 22.6 us with 5 splits, 25.7 with 6).
-  int s = (int)((g.tt == 1 ? 512 : 256) / g.tiles);
+  int s = (int)((g.tt == 1 ? 512 : 256) / ((int64_t)g.tiles * g.row_tiles));
   if (s > steps / kMfWaves) s = steps / kMfWaves;
   if (s < 1) s = 1;
   g.steps_per_split = (steps + s - 1) / s;
@@ -131,9 +135,10 @@ __global__ __launch_bounds__(kMfNT, 2) void matmul_q8_0_mfma_kernel(
   const int brow = lane / LPR, bcol = lane % LPR;
   const uint8_t* const bp = b + ((int64_t)brow * NB + min(blk0 + (bcol >> 1), NB - 1)) * kBlockBytes;
   const int arow = lane >> 3, acol = lane & 7;
+  const int m0 = blockIdx.z * 16 * TT;
   const float* ap[2 * TT];
 #pragma unroll
-  for (int i = 0; i < 2 * TT; ++i) ap[i] = a + (int64_t)min(arow + 8 * i, M - 1) * K + 4 * acol;
+  for (int i = 0; i < 2 * TT; ++i) ap[i] = a + (int64_t)min(m0 + arow + 8 * i, M - 1) * K + 4 * acol;
   struct Stage {
     u32x4 q[BL];
     uint16_t s[BL];
@@ -298,7 +303,7 @@ __global__ __launch_bounds__(kMfNT, 2) void matmul_q8_0_mfma_kernel(
   // Output tile i of the workgroup: rows 4 g .. + 3 of its token tile, column r16.
   auto store = [&](float* dst, int i, const f32x4 v) {
     const int n = i / (2 * TT), j = i / TT % 2, t = i % TT;
-    const int m = 16 * t + 4 * g;
+    const int m = m0 + 16 * t + 4 * g;
     const int64_t col = (blk0 + n) * kBlockElems + j * 16 + r16;
     if (blk0 + n >= NB) return;
 #pragma unroll
@@ -617,8 +622,8 @@ __global__ __launch_bounds__(256) void matmul_splits_kernel(const float* __restr
 template <int TT, int NBW>
 void launch_mf(const MfGrid& g, const float* a, const uint8_t* b, float* dst, int M, int N, int K,
                float* partials, uint32_t* counters, hipStream_t stream) {
-  hipLaunchKernelGGL((matmul_q8_0_mfma_kernel<TT, NBW>), dim3(g.tiles, g.splits), dim3(kMfNT), 0,
-                     stream, a, b, dst, M, N, K, g.steps_per_split, partials, counters);
+  hipLaunchKernelGGL((matmul_q8_0_mfma_kernel<TT, NBW>), dim3(g.tiles, g.splits, g.row_tiles),
+                     dim3(kMfNT), 0, stream, a, b, dst, M, N, K, g.steps_per_split, partials, counters);
 }
 
 template <int MR, int U>
@@ -652,8 +657,7 @@ MatmulNeed matmul_workspace(int M, int N, int K) {
     return need;
   }
   const MfGrid g = mf_grid(M, N, K);
-  const int rows = M < 16 * g.tt ? M : 16 * g.tt;  // of one launch
-  if (g.splits > 1) need.partial_floats = (size_t)g.splits * rows * N;
+  if (g.splits > 1) need.partial_floats = (size_t)g.splits * M * N;
   if (g.splits > 1 && mf_handoff(M)) {
     need.partial_floats = (size_t)g.tiles * g.splits * kMfWaves * 256;
     need.counters = (size_t)g.tiles * kCounterStride;
@@ -679,33 +683,25 @@ hipError_t launch_matmul(const float* a, const uint8_t* b, float* c, int M, int 
     }
     return hipGetLastError();
   }
-  // Up to 64 rows of A a launch (more only where the GEMM does not take the call).
   const MfGrid g = mf_grid(M, N, K);
+  if (g.row_tiles > 65535 || g.splits > 65535) return hipErrorInvalidValue;
   if (g.splits > 1 && partials == nullptr) return hipErrorInvalidValue;
   const bool handoff = g.splits > 1 && mf_handoff(M);
   if (handoff && counters == nullptr) return hipErrorInvalidValue;
   if (!handoff) counters = nullptr;
-  for (int m0 = 0; m0 < M; m0 += 16 * g.tt) {
-    const int mc = M - m0 < 16 * g.tt ? M - m0 : 16 * g.tt;
-    const float* am = a + (int64_t)m0 * K;
-    float* cm = c + (int64_t)m0 * N;
-    float* dst = g.splits > 1 && !handoff ? partials : cm;
-    switch (g.tt) {
-      case 1: launch_mf<1, 4>(g, am, b, dst, mc, N, K, partials, counters, stream); break;
-      case 2: launch_mf<2, 4>(g, am, b, dst, mc, N, K, partials, counters, stream); break;
-      case 3: launch_mf<3, 2>(g, am, b, dst, mc, N, K, partials, counters, stream); break;
-      default: launch_mf<4, 2>(g, am, b, dst, mc, N, K, partials, counters, stream); break;
-    }
-    hipError_t err = hipGetLastError();
-    if (err != hipSuccess) return err;
-    if (g.splits == 1 || handoff) continue;
-    const int64_t mn4 = (int64_t)mc * N / 4;
-    hipLaunchKernelGGL(matmul_splits_kernel, dim3((unsigned)((mn4 + kSpCols - 1) / kSpCols)),
-                       dim3(256), 0, stream, partials, cm, mn4, (int)g.splits);
-    err = hipGetLastError();
-    if (err != hipSuccess) return err;
+  float* dst = g.splits > 1 && !handoff ? partials : c;
+  switch (g.tt) {
+    case 1: launch_mf<1, 4>(g, a, b, dst, M, N, K, partials, counters, stream); break;
+    case 2: launch_mf<2, 4>(g, a, b, dst, M, N, K, partials, counters, stream); break;
+    case 3: launch_mf<3, 2>(g, a, b, dst, M, N, K, partials, counters, stream); break;
+    default: launch_mf<4, 2>(g, a, b, dst, M, N, K, partials, counters, stream); break;
   }
-  return hipSuccess;
+  hipError_t err = hipGetLastError();
+  if (err != hipSuccess || g.splits == 1 || handoff) return err;
+  const int64_t mn4 = (int64_t)M * N / 4;
+  hipLaunchKernelGGL(matmul_splits_kernel, dim3((unsigned)((mn4 + kSpCols - 1) / kSpCols)),
+                     dim3(256), 0, stream, partials, c, mn4, (int)g.splits);
+  return hipGetLastError();
 }
 
 }  // namespace mle

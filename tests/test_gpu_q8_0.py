@@ -832,6 +832,37 @@ def test_matmul_mfma_remainders(dev, orc, M, N, K):
     assert rel_l2(to_host(out), orc.sgemm(a, b, M, N, K)) <= 1e-5
 
 
+@pytest.mark.parametrize("M,N,K", [(65, 96, 64), (200, 32, 2080), (1111, 160, 96)])
+def test_matmul_unaligned_rows_take_one_launch(dev, orc, M, N, K):
+    """64 and more rows of A at a 4-byte offset: all row tiles in one launch (and one that
+    adds the K splits, where there are any), counted as the nodes of a capture."""
+    import ctypes
+    import torch
+    note(f"matmul unaligned rows M={M} N={N} K={K}")
+    b, a = weight(520 + N, K, N), acts(521 + K, M, K)
+    db = to_dev(b, dev)
+    abuf = torch.zeros(M * K + 4, dtype=torch.float32, device=dev)
+    abuf[1:1 + M * K] = to_dev(a, dev).view(-1)
+    out, eager = empty_f32((M, N), dev), empty_f32((M, N), dev)
+    capi.matmul(abuf[1:], db, eager, M, N, K)
+    assert rel_l2(to_host(eager), orc.sgemm(a, b, M, N, K)) <= 1e-5
+    st = torch.cuda.Stream()
+    capi.workspace_reserve(*capi.workspace_size(capi.OP_MATMUL, M, [N], K), stream=st)
+    g = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(g, stream=st):
+        capi.matmul(abuf[1:], db, out, M, N, K, stream=st)
+    nodes = ctypes.c_size_t(0)
+    rc = capi.load().hipGraphGetNodes(ctypes.c_void_p(g.raw_cuda_graph()), None,
+                                      ctypes.byref(nodes))
+    assert rc == 0 and 1 <= nodes.value <= 2
+    g.instantiate()
+    for _ in range(3):
+        out.fill_(float("nan"))
+        g.replay()
+        torch.cuda.synchronize()
+        assert_bitexact(to_host(out), to_host(eager), "replay vs eager")
+
+
 @pytest.mark.parametrize("M", [5, 40])
 def test_matmul_mfma_special_values(dev, orc, M):
     """Non-finite scales and activations, and activations whose product with a scale
