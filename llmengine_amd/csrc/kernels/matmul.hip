@@ -43,10 +43,13 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t mm_rsrc(const void* base, uint
 // into the activations instead: for one 32-column block, c[m, n] = sum_k (a[m, k]
 // d[k]) q[k, n].  The fp32 product a * d (one rounding, as the FMA chain rounds each
 // sum) is split exactly into three bf16 parts by truncation, the quants are exact in
-// bf16, and v_mfma_f32_16x16x32_bf16 forms the products exactly with fp32 sums.  K
-// steps that hold a non-finite scale or an activation past 2^100 (whose product could
-// leave the range where d * q would not) are summed by fp32 FMAs instead, v = d * q
-// first, as the reference does.
+// bf16, and v_mfma_f32_16x16x32_bf16 forms the products exactly with fp32 sums.  The
+// matrix cores take parts below 2^-126 as zero, so the sums are formed 2^40 times too
+// large (exact) and brought back at the end: what is lost stays below fp32's smallest
+// value (unscaled, activations of 1e-36 gave a relative error of 4e-3, of 1e-40 zeros).
+// From the first K step of a wave that holds a non-finite scale or an activation past
+// 2^40 (whose scaled sums could overflow) it sums by fp32 FMAs instead, unscaled, v = d *
+// q first, as the reference does.
 //
 // A workgroup owns NBW 32-column blocks and one K split; its 8 waves take 32-row K
 // steps in turn and add their sums in LDS.  Per step a wave reads its 32 B rows as
@@ -169,7 +172,14 @@ __global__ __launch_bounds__(kMfNT, 2) void matmul_q8_0_mfma_kernel(
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     __builtin_amdgcn_wave_barrier();
   };
-  // Registers -> wave-private LDS; whether the step is all finite and small.
+  bool scaled = true;  // uniform: the sums are kUp times too large
+  constexpr float kUp = 0x1p40f;
+  auto unscale = [&] {
+#pragma unroll
+    for (int i = 0; i < SLOTS; ++i) acc[i / (2 * TT)][i / TT % 2][i % TT] *= 1.0f / kUp;
+  };
+  // Registers -> wave-private LDS; the first step that is not all finite and small ends
+  // the scaled sums.
   auto stage = [&](const Stage& st) {
     bool fine = true;
 #pragma unroll
@@ -183,9 +193,12 @@ __global__ __launch_bounds__(kMfNT, 2) void matmul_q8_0_mfma_kernel(
     for (int i = 0; i < 2 * TT; ++i) {
       *reinterpret_cast<f32x4*>(as + (arow + 8 * i) * AS + 4 * acol) = st.x[i];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) fine &= __builtin_fabsf(st.x[i][e]) < 0x1p100f;  // false on NaN
+      for (int e = 0; e < 4; ++e) fine &= __builtin_fabsf(st.x[i][e]) < 0x1p40f;  // false on NaN
     }
-    return __builtin_amdgcn_ballot_w64(!fine) == 0;
+    if (scaled && __builtin_amdgcn_ballot_w64(!fine) != 0) {
+      scaled = false;
+      unscale();
+    }
   };
   auto multiply = [&] {
     float x[TT][8];
@@ -204,8 +217,9 @@ __global__ __launch_bounds__(kMfNT, 2) void matmul_q8_0_mfma_kernel(
       const u32x4 sc = *reinterpret_cast<const u32x4*>(ss + n * 32 + 8 * g);
       float d[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e)
-        d[e] = scale_to_f32_fast(e & 1 ? sc[e >> 1] >> 16 : sc[e >> 1] & 0xffffu);
+      for (int e = 0; e < 8; ++e)  // one v_fma_mix_f32 each: the scaling is free
+        d[e] = __builtin_fmaf(
+            scale_to_f32_fast(e & 1 ? sc[e >> 1] >> 16 : sc[e >> 1] & 0xffffu), kUp, 0.0f);
       bf16x8 wf[2];
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
@@ -272,16 +286,18 @@ __global__ __launch_bounds__(kMfNT, 2) void matmul_q8_0_mfma_kernel(
   if (step < s1) {
     load(step, st);
     for (; step < s1; step += kMfWaves) {
-      const bool fine = stage(st);
+      stage(st);
       wave_sync();
       if (step + kMfWaves < s1) load(step + kMfWaves, st);
-      if (fine)
+      if (scaled)
         multiply();
       else
         multiply_fp32();
       wave_sync();  // the step's LDS reads come before the next one's writes
     }
   }
+
+  if (scaled) unscale();
 
   // Waves w and w + 4 add first, then the four pairs' sums in order.
   __syncthreads();

@@ -863,6 +863,33 @@ def test_matmul_unaligned_rows_take_one_launch(dev, orc, M, N, K):
         assert_bitexact(to_host(out), to_host(eager), "replay vs eager")
 
 
+@pytest.mark.parametrize("M,N,K", [(3, 96, 512), (8, 1024, 4096), (20, 160, 96), (40, 64, 1056)])
+def test_matmul_mfma_tiny_activations(dev, M, N, K):
+    """Rows of A down to the smallest normal magnitudes keep fp32 accuracy (products with
+    a scale far below 2^-126 included), also beside a row so large that its K steps leave
+    the scaled sums; against float64 (a row's result is above 1e-40, where fp32's
+    subnormal spacing is below 2e-5 of it: 1e-4 there, 1e-5 for normal results)."""
+    import torch
+    note(f"matmul tiny activations M={M} N={N} K={K}")
+    b = weight(530 + N, K, N)
+    blocks = b.reshape(K, N // 32, 34)
+    d = blocks[:, :, :2].copy().view(np.float16).astype(np.float64)
+    v = (d * blocks[:, :, 2:].view(np.int8)).reshape(K, N)
+    mags = np.array([1e-36, 1e-30, 1e-38, 1.0, 1e-34])
+    for large in (False, True):
+        a = acts(531 + M, M, K).astype(np.float64) * mags[np.arange(M) % 5][:, None]
+        if large:
+            a[M - 1, K // 2:] *= 1e14 / np.abs(a[M - 1]).max()
+        a = a.astype(np.float32)
+        out = empty_f32((M, N), dev)
+        capi.matmul(to_dev(a, dev), to_dev(b, dev), out, M, N, K)
+        want, got = a.astype(np.float64) @ v, to_host(out)
+        for r in range(M):
+            rms = np.sqrt(np.mean(want[r] ** 2))
+            bar = 1e-5 if rms > 1e-37 else 1e-4
+            assert rms > 1e-40 and rel_l2(got[r], want[r]) <= bar, (large, r, rms)
+
+
 @pytest.mark.parametrize("M", [5, 40])
 def test_matmul_mfma_special_values(dev, orc, M):
     """Non-finite scales and activations, and activations whose product with a scale
