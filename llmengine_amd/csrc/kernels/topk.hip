@@ -237,9 +237,17 @@ __device__ void select_top(const uint64_t (&key)[E], int k, uint64_t* __restrict
   __syncthreads();
 }
 
-// Distance bin of a value below the row's finite maximum (0: at it).
+// A logit under the temperature, rounded once.  Never contracted with what uses it: both
+// passes have to see the same value, or a row's own maximum could lie above its maximum.
+__device__ __forceinline__ float scaled_logit(float v, float inv_temp) {
+#pragma clang fp contract(off)
+  return v * inv_temp;
+}
+
+// Distance bin of a value not above the row's finite maximum (0: at it, +Inf: 8160).  The
+// sign goes: a maximum held as -0 beside a +0 is at distance -0.
 __device__ __forceinline__ uint32_t dist_bin(float mx, float v) {
-  return __builtin_bit_cast(uint32_t, mx - v) >> 18;  // mx >= v: sign clear, +Inf bin 8160
+  return __builtin_bit_cast(uint32_t, __builtin_fabsf(mx - v)) >> 18;
 }
 
 // Pass 1: workgroup (c, r) over logits[r, c * kChunk : (c + 1) * kChunk).
@@ -275,7 +283,7 @@ __global__ __launch_bounds__(kP1Threads) void topk_chunks_kernel(
     float g = -__builtin_inff();
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const float u = scale && i + e < n ? t[e] * inv_temp : t[e];
+      const float u = scale && i + e < n ? scaled_logit(t[e], inv_temp) : t[e];
       v[4 * j + e] = u;
       nan |= u != u;
       g = fmaxf(g, u);  // ignores NaN
@@ -456,7 +464,7 @@ __global__ __launch_bounds__(kP2Threads) void topk_final_kernel(
       const int64_t i = index_of(j);
       if (i < n) {
         float t = val[e];
-        if (scale) t *= inv_temp;
+        if (scale) t = scaled_logit(t, inv_temp);
         if (dist_bin(mx, t) <= bin) {
           key[e] = topk_key(t, (uint32_t)i);
           const uint32_t slot = atomicAdd(&sm.ncand, 1u);

@@ -147,3 +147,35 @@ def test_top_tokens_group_selection(dev, kind, n, top_n):
         want_ids, want_p = ref_top_tokens(x[r], top_n, 0.8)
         assert np.array_equal(ids[r], want_ids), r
         np.testing.assert_allclose(probs[r], want_p, rtol=1e-5, atol=1e-37)
+
+
+@pytest.mark.parametrize("n,top_n", [(5, 3), (4096, 40), (151936, 2), (9000, 128)])
+def test_top_tokens_signed_zero_maximum(dev, n, top_n):
+    """A row whose maximum is a mix of +0 and -0 (one value, ties to the lower index):
+    neither the group nor the token that holds the other zero is lost."""
+    note(f"top_tokens signed zero maximum n={n} top_n={top_n}")
+    rng = np.random.default_rng(n)
+    x = -np.abs(S.activations(440, (4, n))) - np.float32(1)
+    for r in range(4):
+        at = rng.permutation(n)[:min(n, top_n + 3)]
+        x[r, at] = np.where(rng.random(at.size) < 0.5, np.float32(0.0), np.float32(-0.0))
+        x[r, at[0]] = np.float32(0.0) if r % 2 else np.float32(-0.0)
+    ids, probs = run(x, 4, n, top_n, 1.0, dev)
+    for r in range(4):
+        want_ids, want_p = ref_top_tokens(x[r], top_n, 1.0)
+        assert np.array_equal(ids[r], want_ids), r
+        np.testing.assert_allclose(probs[r], want_p, rtol=1e-5)
+
+
+@pytest.mark.parametrize("temperature", [0.3, 0.7, 1.7])
+def test_top_tokens_inexact_temperature(dev, temperature):
+    """Temperatures whose scaling rounds nearly every logit: the one token asked for is the
+    maximum, whose distance from the maximum (itself, rounded once) is zero."""
+    note(f"top_tokens inexact temperature {temperature}")
+    rows, n = 64, 3001
+    x = (S.activations(441, (rows, n)) * np.float32(7.3)).astype(np.float32)
+    ids, probs = run(x, rows, n, 1, temperature, dev)
+    for r in range(rows):
+        want_ids, want_p = ref_top_tokens(x[r], 1, temperature)
+        assert np.array_equal(ids[r], want_ids), r
+        np.testing.assert_allclose(probs[r], want_p, rtol=1e-5)
