@@ -28,13 +28,13 @@
 //   * Values within that distance are ranked by counting the larger keys (64-bit:
 //     order(value) << 32 | ~index, all distinct); more than 256 go through the
 //     radix select.
-// Selection (exact): a radix select over the keys' upper 32 bits (four 8-bit digit
-// histograms in LDS, most significant first) finds the top_n-th largest value T; the
-// keys >= T (T's ties included) are gathered and sorted by one wave in registers
-// (bitonic network, lane shuffles, no barriers), and the first top_n are the result.
-// If more than 256 keys reach T the whole set is sorted in LDS instead.  Results are
-// deterministic: the keys are distinct, so neither the ranks nor the sorted order
-// depend on the order of gathering.
+// Selection (exact): a radix select over the keys (8-bit digit histograms in LDS, most
+// significant first) narrows a prefix until at most 256 keys reach it; those are gathered
+// and sorted by one wave in registers (bitonic network, lane shuffles, no barriers), and
+// the first top_n are the result.  Rows of few distinct values need the index's digits
+// too; sorting all 16384 keys in LDS there took 157 us for a constant row at top_n 3
+// (MI355X), the digits 31.  Results are deterministic: the keys are distinct, so
+// neither the ranks nor the sorted order depend on the order of gathering.
 //
 // Latency bounds it, not bytes (8 rows x 152k logits are 4.9 MB).  Selecting top_n keys
 // in every chunk instead (a radix select per chunk, then one over 75 x top_n
@@ -50,7 +50,7 @@ constexpr int kChunk = 2048;           // values per pass-1 workgroup
 constexpr int kGroup = 64;             // values per group (top_n >= 16)
 constexpr int kP1Threads = 256;
 constexpr int kP2Threads = 1024;
-constexpr int kP2Keys = 16384;         // values of the picked groups (128 KB of LDS)
+constexpr int kP2Keys = 16384;         // values of the picked groups (16 a thread)
 constexpr int kP2Groups = 8192;        // groups of a row that pass 2 picks from
 constexpr int kBins = 8192;            // distance bins: 8 exponent and 5 mantissa bits
 
@@ -73,25 +73,6 @@ __device__ __forceinline__ float key_value(uint64_t k) {
   uint32_t u = (uint32_t)(k >> 32);
   u = (u & 0x80000000u) ? (u & 0x7fffffffu) : ~u;
   return __builtin_bit_cast(float, u);
-}
-
-// In-place descending bitonic sort of nk (a power of two) keys by NT threads.
-template <int NT>
-__device__ void bitonic_desc(uint64_t* s, int nk) {
-  for (int size = 2; size <= nk; size <<= 1)
-    for (int stride = size >> 1; stride > 0; stride >>= 1) {
-      for (int i = threadIdx.x; i < nk / 2; i += NT) {
-        const int lo = 2 * i - (i & (stride - 1));
-        const int hi = lo + stride;
-        const bool desc = (lo & size) == 0;
-        const uint64_t a = s[lo], b = s[hi];
-        if ((a < b) == desc) {
-          s[lo] = b;
-          s[hi] = a;
-        }
-      }
-      __syncthreads();
-    }
 }
 
 template <int NT, typename T, typename Op>
@@ -152,25 +133,39 @@ __device__ void wave_sort256_desc(uint64_t (&v)[4]) {
     }
 }
 
-// Top k (k <= kTopTokensMax) of the keys held E per thread by NT threads
+// hist[bin] += 1 for every lane with `in`.  Lanes that all name one bin (ties, the leading
+// digits) add once: 16384 single adds to one LDS word took 7 us a digit (MI355X).
+__device__ __forceinline__ void count_bin(uint32_t* hist, uint32_t bin, bool in) {
+  const uint64_t lanes = __builtin_amdgcn_ballot_w64(in);
+  if (lanes == 0) return;  // uniform
+  const int first = __builtin_ctzll(lanes);
+  const uint32_t one = (uint32_t)__builtin_amdgcn_readlane((int)bin, first);
+  if (__builtin_amdgcn_ballot_w64(in && bin == one) == lanes) {
+    if ((int)(threadIdx.x & 63) == first) atomicAdd(&hist[one], (uint32_t)__builtin_popcountll(lanes));
+  } else if (in) {
+    atomicAdd(&hist[bin], 1u);
+  }
+}
+
+// Top k (k <= kTopTokensMax) of the distinct keys held E per thread by NT threads
 // (0 = no key), written sorted descending to out[0, k) (zeros past the number
-// of keys).  `full` (NT * E keys of LDS) is used only when more than 256 keys
-// tie at the threshold.
+// of keys).
 template <int NT, int E>
 __device__ void select_top(const uint64_t (&key)[E], int k, uint64_t* __restrict__ out,
-                           SelectLds& sm, uint64_t* full) {
+                           SelectLds& sm) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  uint32_t prefix = 0, mask = 0;
+  uint64_t prefix = 0, mask = 0;
   int need = k;
   bool all = false;  // fewer keys than k: every key is a candidate
-  for (int shift = 24; shift >= 0; shift -= 8) {
+  // Digits from the top until at most 256 keys reach the prefix: values' digits first,
+  // the index's too where more than 256 keys tie at the value.
+  for (int shift = 56; shift >= 0; shift -= 8) {
     for (int i = tid; i < 256; i += NT) sm.hist[i] = 0;
     __syncthreads();
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-      const uint32_t u = (uint32_t)(key[e] >> 32);
-      if (key[e] != 0 && (u & mask) == prefix) atomicAdd(&sm.hist[(u >> shift) & 255u], 1u);
-    }
+    for (int e = 0; e < E; ++e)
+      count_bin(sm.hist, (uint32_t)(key[e] >> shift) & 255u,
+                key[e] != 0 && (key[e] & mask) == prefix);
     __syncthreads();
     if (wave == 0) {
       uint32_t h[4], local = 0;
@@ -198,41 +193,32 @@ __device__ void select_top(const uint64_t (&key)[E], int k, uint64_t* __restrict
       }
     }
     __syncthreads();
-    if (shift == 24 && sm.total <= (uint32_t)k) {
+    if (shift == 56 && sm.total <= (uint32_t)k) {
       all = true;
       break;
     }
     need -= (int)sm.above;
-    prefix |= sm.digit << shift;
-    mask |= 255u << shift;
+    prefix |= (uint64_t)sm.digit << shift;
+    mask |= (uint64_t)255u << shift;
+    if ((uint32_t)(k - need) + sm.eq <= 256u) break;  // always so once the key is whole
   }
-  // Candidates: every key (all) or the keys with value >= T = prefix.
-  const uint32_t ncand = all ? sm.total : (uint32_t)(k - need) + sm.eq;
-  if (ncand <= 256) {
-    if (tid == 0) sm.ncand = 0;
-    for (int i = tid; i < 256; i += NT) sm.cand[i] = 0;
-    __syncthreads();
+  // Candidates: every key (all) or the keys from the prefix up.
+  __syncthreads();
+  if (tid == 0) sm.ncand = 0;
+  for (int i = tid; i < 256; i += NT) sm.cand[i] = 0;
+  __syncthreads();
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-      const uint32_t u = (uint32_t)(key[e] >> 32);
-      if (key[e] != 0 && (all || u >= prefix)) sm.cand[atomicAdd(&sm.ncand, 1u)] = key[e];
-    }
-    __syncthreads();
-    if (wave == 0) {
-      uint64_t v[4];
+  for (int e = 0; e < E; ++e)
+    if (key[e] != 0 && (all || key[e] >= prefix)) sm.cand[atomicAdd(&sm.ncand, 1u)] = key[e];
+  __syncthreads();
+  if (wave == 0) {
+    uint64_t v[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) v[j] = sm.cand[4 * lane + j];
-      wave_sort256_desc(v);
+    for (int j = 0; j < 4; ++j) v[j] = sm.cand[4 * lane + j];
+    wave_sort256_desc(v);
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (4 * lane + j < k) out[4 * lane + j] = v[j];
-    }
-  } else {
-#pragma unroll
-    for (int e = 0; e < E; ++e) full[tid * E + e] = key[e];
-    __syncthreads();
-    bitonic_desc<NT>(full, NT * E);
-    for (int j = tid; j < k; j += NT) out[j] = full[j];
+    for (int j = 0; j < 4; ++j)
+      if (4 * lane + j < k) out[4 * lane + j] = v[j];
   }
   __syncthreads();
 }
@@ -324,7 +310,7 @@ __global__ __launch_bounds__(kP2Threads) void topk_final_kernel(
     const float* __restrict__ x, const float* __restrict__ maxima,
     const float* __restrict__ stats, int chunks, int gpc, int gm, int gshift, int64_t n, int kk,
     float inv_temp, int scale, int32_t* __restrict__ ids, float* __restrict__ probs) {
-  __shared__ __attribute__((aligned(16))) uint64_t s[kP2Keys];  // bins, then massive ties
+  __shared__ __attribute__((aligned(16))) uint32_t hist[kBins];
   __shared__ SelectLds sm;
   __shared__ uint64_t top[kTopTokensMax];
   __shared__ int list[kP2Keys / kGroup];
@@ -335,7 +321,6 @@ __global__ __launch_bounds__(kP2Threads) void topk_final_kernel(
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int64_t r = blockIdx.x;
   const float* st = stats + r * chunks * 4;
-  uint32_t* const hist = reinterpret_cast<uint32_t*>(s);
   // The group maxima first: nothing below waits for more than they do.
   constexpr int GPT = kP2Groups / kP2Threads;
   const int total_max = chunks * gpc;  // per row
@@ -373,7 +358,7 @@ __global__ __launch_bounds__(kP2Threads) void topk_final_kernel(
     // The first bin B at which kk groups have a maximum within it (scanned below).
 #pragma unroll
     for (int e = 0; e < GPT; ++e)
-      if (tid + kP2Threads * e < groups) atomicAdd(&hist[dist_bin(mx, gv[e])], 1u);
+      count_bin(hist, dist_bin(mx, gv[e]), tid + kP2Threads * e < groups);
     auto add = [&](const f4 c) {
       if (c.x > -__builtin_inff()) sum += ((double)c.y + c.z) * exp((double)c.x - (double)mx);
     };
@@ -436,7 +421,7 @@ __global__ __launch_bounds__(kP2Threads) void topk_final_kernel(
       const int gi = tid + kP2Threads * e;
       gk[e] = gi < groups ? topk_key(gv[e], (uint32_t)gi) : 0;
     }
-    select_top<kP2Threads, GPT>(gk, kk, top, sm, s);
+    select_top<kP2Threads, GPT>(gk, kk, top, sm);
     ngroups = (uint32_t)(kk < groups ? kk : groups);
     for (int j = tid; j < (int)ngroups; j += kP2Threads) list[j] = (int)~(uint32_t)top[j];
     if (tid == 0) sm.ncand = 0;
@@ -487,7 +472,7 @@ __global__ __launch_bounds__(kP2Threads) void topk_final_kernel(
     if (mine != 0 && (tid & 3) == 0 && rank < kk) top[rank] = mine;
     __syncthreads();
   } else {
-    select_top<kP2Threads, PER>(key, kk, top, sm, s);
+    select_top<kP2Threads, PER>(key, kk, top, sm);
   }
   for (int j = tid; j < kk; j += kP2Threads) {
     const uint64_t kv = top[j];
@@ -501,7 +486,7 @@ __global__ __launch_bounds__(kP2Threads) void topk_final_kernel(
 int topk_chunks(int64_t n) { return (int)((n + kChunk - 1) / kChunk); }
 
 int topk_max_n(int k) {
-  // The values of k groups must fit pass 2's LDS; kept at chunks * k <= kP2Keys.
+  // The values of k groups must fit pass 2's registers; kept at chunks * k <= kP2Keys.
   return k <= 0 ? 0 : (kP2Keys / k) * kChunk;
 }
 

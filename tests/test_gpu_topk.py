@@ -11,7 +11,7 @@ which std::partial_sort leaves unordered, go to the lower index on the device.
 import numpy as np
 import pytest
 
-from helpers import note, to_dev
+from helpers import empty_f32, note, to_dev
 from llmengine_amd import capi
 from llmengine_amd import synthetic as S
 
@@ -179,3 +179,43 @@ def test_top_tokens_inexact_temperature(dev, temperature):
         want_ids, want_p = ref_top_tokens(x[r], 1, temperature)
         assert np.array_equal(ids[r], want_ids), r
         np.testing.assert_allclose(probs[r], want_p, rtol=1e-5)
+
+
+@pytest.mark.parametrize("kind,n,top_n", [("equal", 32000, 3), ("equal", 151936, 128),
+                                          ("masked", 128256, 64), ("equal", 800, 64),
+                                          ("two", 50257, 128)])
+def test_top_tokens_massive_ties_cost(dev, kind, n, top_n):
+    """Rows of one or two values and masked rows with fewer kept logits than tokens asked
+    for: exact ids, and no more than 6 times the time of rows of distinct logits (a sort of
+    all 16384 candidate values took 14 times that; the best of several timings of each)."""
+    import torch
+    note(f"top_tokens massive ties {kind} n={n} top_n={top_n}")
+    rows = 2
+    plain = (S.activations(442, (rows, n)) * np.float32(3)).astype(np.float32)
+    x = np.full_like(plain, 0.5)
+    if kind == "masked":
+        x[:] = np.finfo(np.float32).min
+        x[:, 7::n // 50] = plain[:, 7::n // 50]
+    elif kind == "two":
+        x[:, 1::3] = 1.5
+    ids, probs = run(x, rows, n, top_n, 1.0, dev)
+    for r in range(rows):
+        want_ids, want_p = ref_top_tokens(x[r], top_n, 1.0)
+        assert np.array_equal(ids[r], want_ids), r
+        np.testing.assert_allclose(probs[r], want_p, rtol=1e-5, atol=1e-37)
+    out_i = torch.empty((rows, top_n), dtype=torch.int32, device=dev)
+    out_p = empty_f32((rows, top_n), dev)
+
+    def best(v):
+        d, t = to_dev(v, dev), []
+        for _ in range(6):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            for _ in range(20):
+                capi.top_tokens(d, rows, n, top_n, out_i, out_p, 1.0)
+            b.record()
+            b.synchronize()
+            t.append(a.elapsed_time(b) / 20)
+        return min(t)
+
+    assert best(x) <= 6 * best(plain)
