@@ -984,7 +984,7 @@ int mle_argmax_f32(const float* logits, int rows, int n, int32_t* idx, float* va
   MLE_TRY(check_align(ctx, val, 4, "val"));
   mle::SplitKNeed need;
   need.partial_floats = (size_t)rows * mle::argmax_chunks(n) * 2;  // 64-bit keys
-  need.counters = mle::argmax_counters(rows);
+  need.counters = mle::argmax_counters(rows, n);
   if (need.counters != 0 && stream_capturing(stream)) {  // a reservation of bytes alone serves
     size_t bytes = 0, counters = 0;
     graph_workspace_capacity(stream, &bytes, &counters);

@@ -12,15 +12,20 @@
 // A workgroup (grid chunks x rows) reduces a chunk of a row to one 64-bit key.  key =
 // (order(v) << 32) | ~index, where order() maps float bits to unsigned integers in
 // value order, so the largest key is the largest value with the smallest index:
-// deterministic in any order of reduction.  Up to kArgRows rows the chunks' keys meet
-// by an atomic maximum beside the row's counter in the workspace, and the row's last
-// workgroup decodes the winner; more rows (whose counters a default workspace does not
-// hold) write the keys, which a second launch reduces.
+// deterministic in any order of reduction.  Up to kArgRows rows of kArgMeetPieces pieces
+// the chunks' keys meet by an atomic maximum beside the row's counter in the workspace,
+// and the row's last workgroup decodes the winner; more rows (whose counters a default
+// workspace does not hold) and longer ones write the keys, which a second launch reduces.
 //
 // Bound by latency (152k logits are 0.6 MB): a thread's 8 values are loaded at once
 // (one by one in a loop, each load waited for, and with a second launch for every call, the
 // [1, 151936] pick behind its [151936, 896] Linear took 29.3 us a pair on MI355X; this
-// takes 27.1).
+// takes 27.1).  A row's chunks take turns at its counter, so at most kArgChunks of them
+// meet, two pieces each where there are more pieces (300000 logits: 5.3 us, 6.1 with a
+// chunk a piece, 5.9 in two launches), and rows past two pieces a chunk take two launches
+// (524288 logits: 5.8 us, 6.0 with 96 chunks meeting, 9.0 with 256).
+#include <algorithm>
+
 #include "../launch.hpp"
 
 namespace mle {
@@ -30,6 +35,8 @@ constexpr int kArgThreads = 256;
 constexpr int kArgVecs = 2;                              // 4-value loads a thread
 constexpr int kArgPiece = 4 * kArgVecs * kArgThreads;    // 2048 values
 constexpr int kArgRows = 4096 / kCounterStride;          // a default workspace's counters
+constexpr int kArgChunks = 96;                           // of a row that meet
+constexpr int kArgMeetPieces = 2 * kArgChunks;
 
 __device__ __forceinline__ uint64_t arg_key(float v, uint32_t i) {
   if (v != v) return 0;  // NaN: never selected
@@ -157,14 +164,15 @@ int argmax_chunks(int64_t n) {
   return (int)(c < 1 ? 1 : c > 256 ? 256 : c);
 }
 
-size_t argmax_counters(int rows) {
-  return rows <= kArgRows ? (size_t)rows * kCounterStride : 0;
+size_t argmax_counters(int rows, int64_t n) {
+  return rows <= kArgRows && n <= (int64_t)kArgMeetPieces * kArgPiece ? (size_t)rows * kCounterStride
+                                                                      : 0;
 }
 
 hipError_t launch_argmax(const float* x, int rows, int64_t n, int32_t* idx, float* val,
                          uint64_t* keys, uint32_t* counters, hipStream_t stream) {
   if (rows <= 0 || n <= 0 || n > 0x7fffffff || rows > 65535) return hipErrorInvalidValue;
-  const int chunks = argmax_chunks(n);
+  const int chunks = counters != nullptr ? std::min(argmax_chunks(n), kArgChunks) : argmax_chunks(n);
   const int64_t pieces = (n + kArgPiece - 1) / kArgPiece;
   const int64_t chunk = (pieces + chunks - 1) / chunks * kArgPiece;
   const dim3 grid((unsigned)chunks, (unsigned)rows);

@@ -197,9 +197,10 @@ hipError_t launch_matmul(const float* a, const uint8_t* b, float* c, int M, int 
 
 // Greedy argmax of `rows` rows of n fp32 logits: idx (and val, if non-null) per
 // row; `keys` is a workspace of rows * argmax_chunks(n) 64-bit entries;
-// with `counters` (argmax_counters(rows) of them, zero) it takes one launch, else two.
+// with `counters` (argmax_counters(rows, n) of them, zero; 0: none taken) it takes one
+// launch, else two.
 int argmax_chunks(int64_t n);
-size_t argmax_counters(int rows);
+size_t argmax_counters(int rows, int64_t n);
 hipError_t launch_argmax(const float* x, int rows, int64_t n, int32_t* idx, float* val,
                          uint64_t* keys, uint32_t* counters, hipStream_t stream);
 

@@ -207,6 +207,36 @@ def test_argmax_chunk_edges(dev, rows, n):
         assert idx.cpu().numpy().tolist() == wants[k].tolist()
 
 
+@pytest.mark.parametrize("rows,n", [(1, 196608), (3, 196609), (2, 300001), (1, 393216),
+                                    (2, 393217), (1, 524288)])
+def test_argmax_long_rows(dev, rows, n):
+    """Rows of more pieces than meet at a counter: two pieces a chunk, then (counted as the
+    nodes of a capture) two launches; the maximum in any piece, the first of ties."""
+    import ctypes
+    import torch
+    note(f"argmax long rows rows={rows} n={n}")
+    x = np.zeros((rows, n), np.float32)
+    x[:, ::3] = -1.0
+    idx, val = torch.empty(rows, dtype=torch.int32, device=dev), empty_f32((rows,), dev)
+    for at in (0, 1, 2047, 2048, 4096, 196607, n - 2, n - 1):
+        y = x.copy()
+        y[:, min(at, n - 1):] = np.where(y[:, min(at, n - 1):] < 0, 2.0, 1.0)
+        capi.argmax(to_dev(y, dev), rows, n, idx, val)
+        want = first_argmax(y)
+        assert np.array_equal(idx.cpu().numpy(), want)
+        assert np.array_equal(to_host(val), y[np.arange(rows), want])
+    st = torch.cuda.Stream()
+    capi.workspace_reserve(16 * rows * 256, rows * 32, stream=st)
+    g = torch.cuda.CUDAGraph(keep_graph=True)
+    d = to_dev(x, dev)
+    with torch.cuda.graph(g, stream=st):
+        capi.argmax(d, rows, n, idx, val, stream=st)
+    nodes = ctypes.c_size_t(0)
+    rc = capi.load().hipGraphGetNodes(ctypes.c_void_p(g.raw_cuda_graph()), None,
+                                      ctypes.byref(nodes))
+    assert rc == 0 and nodes.value == (1 if n <= 393216 else 2)
+
+
 def test_argmax_ties_signed_zero_and_nan(dev):
     import torch
     n = 10_000
