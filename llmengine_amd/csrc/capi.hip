@@ -908,6 +908,9 @@ int mle_q8_0_workspace_size(int op, int M, int count, const int* N, int K, int t
 
 int mle_workspace_reserve(size_t bytes, size_t counters, hipStream_t stream) {
   if (bytes == 0 && counters == 0) return ok();
+  // Also a reservation of bytes alone holds the smallest counter buffer, which every greedy
+  // pick that takes counters fits.
+  if (counters == 0) counters = 1;
   std::lock_guard<std::mutex> lock(g_ws_mu);
   StreamWorkspace* e = nullptr;
   MLE_TRY(ensure_workspace(bytes, counters, stream, false, &e));
@@ -985,11 +988,6 @@ int mle_argmax_f32(const float* logits, int rows, int n, int32_t* idx, float* va
   mle::SplitKNeed need;
   need.partial_floats = (size_t)rows * mle::argmax_chunks(n) * 2;  // 64-bit keys
   need.counters = mle::argmax_counters(rows, n);
-  if (need.counters != 0 && stream_capturing(stream)) {  // a reservation of bytes alone serves
-    size_t bytes = 0, counters = 0;
-    graph_workspace_capacity(stream, &bytes, &counters);
-    if (need.counters > counters) need.counters = 0;
-  }
   mle::SplitKWorkspace ws;
   std::unique_lock<std::mutex> hold;  // released after the launch is enqueued
   MLE_TRY(get_workspace(need, stream, &ws, &hold));

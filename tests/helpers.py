@@ -133,3 +133,16 @@ def untile_ref(tiled: np.ndarray, N: int, K: int) -> np.ndarray:
     d = t[nq:].reshape(G, KP, 16, 2, 2).transpose(0, 2, 1, 3, 4).reshape(G * 16, 2 * KP, 2)
     out = np.concatenate([d[:N, :KB], q[:N, :KB]], axis=2)
     return out.reshape(-1)
+
+
+def own_stream():
+    """A new stream of its own, with no workspace yet: torch.cuda.Stream() hands out the
+    streams of a pool of 32 in turn, so each one taken in a test shifts which stream, used
+    or unused, a later test gets."""
+    import ctypes
+    import torch
+    from llmengine_amd import capi
+    h = ctypes.c_void_p()
+    rc = capi.load().hipStreamCreateWithFlags(ctypes.byref(h), 1)  # non-blocking
+    assert rc == 0, rc
+    return torch.cuda.ExternalStream(h.value)

@@ -15,7 +15,7 @@ import functools
 import numpy as np
 import pytest
 
-from helpers import empty_f32, note, rel_l2, to_dev, to_host
+from helpers import empty_f32, note, own_stream, rel_l2, to_dev, to_host
 from llmengine_amd import capi
 from llmengine_amd import synthetic as S
 
@@ -193,18 +193,23 @@ def test_argmax_chunk_edges(dev, rows, n):
         capi.argmax(devs[k], rows, n, idx, val)
         assert idx.cpu().numpy().tolist() == wants[k].tolist()
         assert to_host(val).tolist() == [20.0 + k] * rows
-    st = torch.cuda.Stream()
-    capi.workspace_reserve(16 * rows * 256, 0, stream=st)  # bytes alone are enough
-    g = torch.cuda.CUDAGraph()
-    y = devs[0].clone()
-    with torch.cuda.graph(g, stream=st):
-        capi.argmax(y, rows, n, idx, val, stream=st)
-    for k in (1, 2, 0):
-        y.copy_(devs[k])
-        g.replay()
-        capi.argmax(devs[k], rows, n, idx, val)
-        g.replay()
-        assert idx.cpu().numpy().tolist() == wants[k].tolist()
+    for counters in (0, rows * 32):  # bytes alone are enough
+        st = own_stream() if counters else torch.cuda.Stream()
+        capi.workspace_reserve(16 * rows * 256, counters, stream=st)
+        g = torch.cuda.CUDAGraph()
+        y = devs[0].clone()
+        idx2, val2 = torch.empty_like(idx), torch.empty_like(val)
+        with torch.cuda.graph(g, stream=st):
+            capi.argmax(y, rows, n, idx, val, stream=st)
+        for k in (1, 2, 0):
+            y.copy_(devs[k])
+            for _ in range(2):
+                idx.fill_(-1)
+                val.fill_(float("nan"))
+                g.replay()
+                assert idx.cpu().numpy().tolist() == wants[k].tolist()
+                assert to_host(val).tolist() == [20.0 + k] * rows
+                capi.argmax(devs[(k + 1) % 3], rows, n, idx2, val2)
 
 
 @pytest.mark.parametrize("rows,n", [(1, 196608), (3, 196609), (2, 300001), (1, 393216),
@@ -225,7 +230,7 @@ def test_argmax_long_rows(dev, rows, n):
         want = first_argmax(y)
         assert np.array_equal(idx.cpu().numpy(), want)
         assert np.array_equal(to_host(val), y[np.arange(rows), want])
-    st = torch.cuda.Stream()
+    st = own_stream()
     capi.workspace_reserve(16 * rows * 256, rows * 32, stream=st)
     g = torch.cuda.CUDAGraph(keep_graph=True)
     d = to_dev(x, dev)
@@ -235,6 +240,34 @@ def test_argmax_long_rows(dev, rows, n):
     rc = capi.load().hipGraphGetNodes(ctypes.c_void_p(g.raw_cuda_graph()), None,
                                       ctypes.byref(nodes))
     assert rc == 0 and nodes.value == (1 if n <= 393216 else 2)
+
+
+def test_argmax_on_a_reservation_of_bytes_allocates_nothing(dev):
+    """A loop that reserved bytes alone for its greedy picks: eager calls allocate nothing
+    (the pick's counters included), and captured ones are accepted."""
+    import torch
+    note("argmax on a reservation of bytes")
+    rows, n = 128, 5000
+    x = S.activations(710, (rows, n))
+    d, want = to_dev(x, dev), first_argmax(x)
+    idx, val = torch.empty(rows, dtype=torch.int32, device=dev), empty_f32((rows,), dev)
+    st = own_stream()
+    capi.workspace_reserve(16 * rows * 256, 0, stream=st)
+    gen = capi.workspace_info(st)[2]
+    torch.cuda.synchronize()
+    for _ in range(3):
+        capi.argmax(d, rows, n, idx, val, stream=st)
+    st.synchronize()
+    assert np.array_equal(idx.cpu().numpy(), want)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=st):
+        capi.argmax(d, rows, n, idx, val, stream=st)
+    for _ in range(3):
+        idx.fill_(-1)
+        g.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(idx.cpu().numpy(), want)
+    assert capi.workspace_info(st)[2] == gen
 
 
 def test_argmax_ties_signed_zero_and_nan(dev):

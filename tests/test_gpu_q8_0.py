@@ -11,7 +11,7 @@ import functools
 import numpy as np
 import pytest
 
-from helpers import (assert_bitexact, bits, empty_f32, hybrid_decode, note, rel_l2, sha,
+from helpers import (assert_bitexact, bits, empty_f32, hybrid_decode, note, own_stream, rel_l2, sha,
                      to_dev, to_host)
 from llmengine_amd import capi
 from llmengine_amd import synthetic as S
@@ -846,7 +846,7 @@ def test_matmul_unaligned_rows_take_one_launch(dev, orc, M, N, K):
     out, eager = empty_f32((M, N), dev), empty_f32((M, N), dev)
     capi.matmul(abuf[1:], db, eager, M, N, K)
     assert rel_l2(to_host(eager), orc.sgemm(a, b, M, N, K)) <= 1e-5
-    st = torch.cuda.Stream()
+    st = own_stream()
     capi.workspace_reserve(*capi.workspace_size(capi.OP_MATMUL, M, [N], K), stream=st)
     g = torch.cuda.CUDAGraph(keep_graph=True)
     with torch.cuda.graph(g, stream=st):
