@@ -1,6 +1,5 @@
 // linear_mid.hip -- Q8_0 Linear for a serving batch or a short prompt (17-128
-// tokens, and 9-16 on short rows) on bf16 MFMA for gfx950, every weight
-// byte read once per launch.
+// tokens) on bf16 MFMA for gfx950, every weight byte read once per launch.
 //
 // y[m, n] = sum_k x[m, k] * d[n, k/32] * q[n, k]  (+ bias[n]), as
 // cpu::sgemm_nt(const float*, const uint8_t*, ...) computes it
@@ -661,8 +660,11 @@ hipError_t launch_mid_rg(const MidConfig& c, const MidGrid& gr, WeightLayout lay
 // Whether a launch takes this kernel, and its shape (tt == 0: it does not).
 //
 // Tokens: 17-63 always (1.2-2.7 times as fast as 16-token chunks on every shape
-// measured, raw and tiled); 9-16 on rows of up to 1024 elements (0.79-0.93x the time),
-// not on longer ones (4096 x 4096 at 16 tokens: 10.3 us vs 8.5).  From 64
+// measured, raw and tiled).  Not 9-16, where one launch of the decode reads the weights
+// once as well: rows of 672-1024 elements take 0.8x its time here on up to 256 row groups,
+// but up to 1.5x on 400 and more (16384 x 896 raw at 16 tokens: 12.2 us vs 9.0), and the
+// kernel cannot follow the groups, since a fused launch has to keep the bits of its outputs'
+// own launches.  From 64
 // tokens the GEMM reuses each dequantised weight more: it keeps launches of more
 // than 512 row groups up to 80 tokens (12288 x 4096 at 77: 28.0 vs 27.8 us), 304 up to 96
 // (5120 x 6912 at 96: 28.5 vs 27.5) and 256 up to 128 (and rows past 4096 elements on
@@ -679,12 +681,11 @@ hipError_t launch_mid_rg(const MidConfig& c, const MidGrid& gr, WeightLayout lay
 // (304: 4864 x 896 runs as well with one group in 304 workgroups as with two).
 MidConfig linear_mid_pick(int M, const LinearSegs& s, int K) {
   MidConfig c;
-  if (M < 9 || M > 128 || s.layout == WeightLayout::kKN) return c;
+  if (M < 17 || M > 128 || s.layout == WeightLayout::kKN) return c;
   const MidArgs a = mid_args(s);
   const bool swi = a.swiglu != 0;
   const int64_t G = a.grp_end[a.count - 1];  // output row groups
   const int KB = K / kBlockElems;
-  if (M <= 16 && K > 1024) return c;
   if (M >= 64) {
     const bool takes = M <= 80 ? G <= 512 : M <= 96 ? G <= 304 : G <= 64 || (G <= 256 && K <= 4096);
     if (swi || !takes) return c;
@@ -724,7 +725,6 @@ hipError_t launch_linear_mid(const MidConfig& c, const float* x, const LinearSeg
   const MidGrid gr = mid_grid(c, s, K);
   if (c.parts == 3) {
     switch (c.tt) {
-      case 1: return launch_mid_rg<1, 3>(c, gr, s.layout, x, M, K, ws, stream);
       case 2: return launch_mid_rg<2, 3>(c, gr, s.layout, x, M, K, ws, stream);
       case 3: return launch_mid_rg<3, 3>(c, gr, s.layout, x, M, K, ws, stream);
       case 4: return launch_mid_rg<4, 3>(c, gr, s.layout, x, M, K, ws, stream);

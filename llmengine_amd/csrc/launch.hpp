@@ -138,7 +138,7 @@ hipError_t launch_gemv_mfma_segs(const DecodeMfmaConfig& c, const float* x,
                                  const LinearSegs& s, int M, int K, const SplitKWorkspace& ws,
                                  hipStream_t stream);
 
-// Linear of a serving batch or a short prompt (9-128 tokens): 64 rg weight rows per
+// Linear of a serving batch or a short prompt (17-128 tokens): 64 rg weight rows per
 // workgroup, all tokens (tt tiles of 16), `splits` K splits.
 struct MidConfig {
   int tt = 0;      // token tiles of 16 (16 tt >= M); 0: the launch is not this kernel's

@@ -1,4 +1,5 @@
-"""GPU parity of the Linear for 9-128 tokens (linear_mid.hip).
+"""GPU parity of the Linear for 17-128 tokens (linear_mid.hip), and the cases of 9-16 beside
+it (the 16-token MFMA decode).
 
 Raw and tiled weights (the same bits: same products, same order) against the CPU oracle
 (cpu_kernels.cpp:208-218), against the general paths that the tuning hook forces (the
@@ -203,3 +204,19 @@ def test_mid_multi_past_the_split_bound(dev):
     for w, y in zip(ws, ys):
         capi.linear(x, w, None, one, M, N, K)
         assert_bitexact(to_host(y), to_host(one), "fused vs single")
+
+
+@pytest.mark.parametrize("M,N,K", [(9, 100, 32), (12, 6000, 896), (16, 1024, 1024)])
+def test_up_to_16_tokens_take_the_decode(dev, M, N, K):
+    """9-16 tokens on rows of any length run the 16-token decode: its bits, on both layouts
+    and in a fused launch."""
+    note(f"16-token decode M={M} N={N} K={K}")
+    x, dw = to_dev(S.activations(980, (M, K)), dev), to_dev(weight(981, N, K), dev)
+    y, yt, yd, y0, y1 = (empty_f32((M, N), dev) for _ in range(5))
+    capi.linear(x, dw, None, y, M, N, K)
+    capi.linear_tiled(x, tiled_dev(dw, N, K, dev), None, yt, M, N, K)
+    capi.linear_ex(x, dw, None, yd, M, N, K, path=3)
+    capi.linear_multi(x, [dw, dw], [None] * 2, [y0, y1], [N] * 2, M, K)
+    want = to_host(yd)
+    for got in (y, yt, y0, y1):
+        assert_bitexact(to_host(got), want, "decode bits")
