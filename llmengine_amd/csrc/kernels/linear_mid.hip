@@ -601,6 +601,18 @@ struct MidGrid {
   int phases_per_split;
   MidArgs args;
 };
+// Phases of a K split, and the K splits a launch makes of them (fewer than asked for where
+// whole phases do not fill them).
+int mid_phases_per_split(const MidConfig& c, int K) {
+  const int phases = (K / kBlockElems + kPhaseBlocks - 1) / kPhaseBlocks;
+  return (phases + c.splits - 1) / c.splits;
+}
+int mid_splits(const MidConfig& c, int K) {
+  const int phases = (K / kBlockElems + kPhaseBlocks - 1) / kPhaseBlocks;
+  const int per = mid_phases_per_split(c, K);
+  return (phases + per - 1) / per;
+}
+
 MidGrid mid_grid(const MidConfig& c, const LinearSegs& s, int K) {
   MidGrid gr{};
   gr.args = mid_args(s);
@@ -609,9 +621,8 @@ MidGrid mid_grid(const MidConfig& c, const LinearSegs& s, int K) {
   gr.tiles = (groups + per - 1) / per;
   gr.tiles_per_launch = c.tiles_per_launch > 0 ? std::min(gr.tiles, (unsigned)c.tiles_per_launch)
                                                : gr.tiles;
-  const int phases = (K / kBlockElems + kPhaseBlocks - 1) / kPhaseBlocks;
-  gr.phases_per_split = (phases + c.splits - 1) / c.splits;
-  gr.splits = (unsigned)((phases + gr.phases_per_split - 1) / gr.phases_per_split);
+  gr.phases_per_split = mid_phases_per_split(c, K);
+  gr.splits = (unsigned)mid_splits(c, K);
   return gr;
 }
 
@@ -677,8 +688,43 @@ hipError_t launch_mid_rg(const MidConfig& c, const MidGrid& gr, WeightLayout lay
 // partials stay within the 16-token decode's); one split for weights whose rows alone
 // fill the GPU several times over (3072 groups).  A SwiGLU pair,
 // which no single launch has to match, halves them until its grid fits the CUs.
-// Row groups per wave: the fewest that keep the grid within about one workgroup a CU
-// (304: 4864 x 896 runs as well with one group in 304 workgroups as with two).
+// Row groups per wave (which no bits depend on).
+//   * Up to two token tiles: the fewest groups of one to three that keep the grid within
+//     one workgroup a CU (304 with one group, 4864 x 896 runs as well so as with two, and
+//     with two in splits of up to 3 phases), else two, which are resident twice a CU and
+//     hide each other's start.  288 workgroups leave a last round of 32 (9216 x 5120 raw at
+//     17 tokens 39.1 us, 27.6 with three groups), and four groups in two rounds of 384 or 512
+//     take 1.2-1.5x the time of two (49136 x 768 raw 32.7 -> 24.5, 50880 x 4096 raw 124 -> 78).
+//   * More tiles are resident once a CU.  Splits of up to 3 phases are over before a second
+//     round costs much: the fewest groups within 304 workgroups (of the splits asked for).
+//     Longer ones: the fewest rounds (a second one of up to 64 workgroups counts 0.6), a
+//     workgroup costing its groups and one more for the activations (13824 x 4096 at 48
+//     tokens: 4 groups in 216 workgroups 0.51x the chunks' time, 3 in 288 0.71x; 4864 x
+//     1024 at 33: 1 in 304 0.46x, 2 in 152 0.55x).
+static int mid_row_groups(const MidConfig& c, int64_t G, int K) {
+  const int rg_max = max_rg(c.tt, c.parts);
+  const int splits = mid_splits(c, K);
+  const bool brief = mid_phases_per_split(c, K) <= 3;
+  auto grid = [&](int rg) { return (G + kWN * rg - 1) / (kWN * rg) * splits; };
+  if (c.tt <= 2) {
+    for (int rg = 1; rg <= 3; ++rg)
+      if (grid(rg) <= (rg == 1 || (rg == 2 && brief) ? 304 : 256)) return rg;
+    return 2;
+  }
+  int best = 1;
+  if (brief) {
+    while (best < rg_max && (G + kWN * best - 1) / (kWN * best) * c.splits > 304) ++best;
+    return best;
+  }
+  auto cost = [&](int rg) {  // in fifths of a round
+    const int64_t wgs = grid(rg);
+    return (wgs > 256 && wgs <= 320 ? 8 : (wgs + 255) / 256 * 5) * (rg + 1);
+  };
+  for (int rg = 2; rg <= rg_max; ++rg)
+    if (cost(rg) <= cost(best)) best = rg;
+  return best;
+}
+
 MidConfig linear_mid_pick(int M, const LinearSegs& s, int K) {
   MidConfig c;
   if (M < 17 || M > 128 || s.layout == WeightLayout::kKN) return c;
@@ -693,14 +739,12 @@ MidConfig linear_mid_pick(int M, const LinearSegs& s, int K) {
   c.parts = M < 64 ? 3 : 1;
   c.tt = M < 64 ? (M + 15) / 16 : M <= 64 ? 4 : M <= 80 ? 5 : M <= 96 ? 6 : 8;
   c.splits = G >= 3072 || KB <= 16 ? 1 : KB <= 128 ? 4 : c.tt == 3 ? 7 : 8;
-  const int rg_max = max_rg(c.tt, c.parts);
-  auto grid = [&](int rg) { return (G + kWN * rg - 1) / (kWN * rg) * c.splits; };
   if (swi) {
+    auto grid = [&](int rg) { return (G + kWN * rg - 1) / (kWN * rg) * c.splits; };
     c.rg = grid(1) <= 304 ? 2 : 4;  // half of each weight
     while (c.splits > 1 && grid(c.rg / 2) > 304) c.splits /= 2;
   } else {
-    c.rg = 1;
-    while (c.rg < rg_max && grid(c.rg) > 304) ++c.rg;
+    c.rg = mid_row_groups(c, G, K);
   }
   return c;
 }

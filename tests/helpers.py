@@ -146,3 +146,23 @@ def own_stream():
     rc = capi.load().hipStreamCreateWithFlags(ctypes.byref(h), 1)  # non-blocking
     assert rc == 0, rc
     return torch.cuda.ExternalStream(h.value)
+
+
+def slower_by(fn, than, rounds: int = 9) -> float:
+    """Time of fn() over the time of than(), the two timed in turn, each at its best of
+    `rounds` runs of back-to-back calls."""
+    import torch
+    best = [float("inf")] * 2
+    for f in (fn, than):
+        f()
+    torch.cuda.synchronize()
+    for _ in range(rounds):
+        for i, f in enumerate((fn, than)):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            for _ in range(10):
+                f()
+            b.record()
+            b.synchronize()
+            best[i] = min(best[i], a.elapsed_time(b))
+    return best[0] / best[1]
