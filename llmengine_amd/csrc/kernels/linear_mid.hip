@@ -675,12 +675,15 @@ hipError_t launch_mid_rg(const MidConfig& c, const MidGrid& gr, WeightLayout lay
 // once as well: rows of 672-1024 elements take 0.8x its time here on up to 256 row groups,
 // but up to 1.5x on 400 and more (16384 x 896 raw at 16 tokens: 12.2 us vs 9.0), and the
 // kernel cannot follow the groups, since a fused launch has to keep the bits of its outputs'
-// own launches.  From 64
-// tokens the GEMM reuses each dequantised weight more: it keeps launches of more
-// than 512 row groups up to 80 tokens (12288 x 4096 at 77: 28.0 vs 27.8 us), 304 up to 96
-// (5120 x 6912 at 96: 28.5 vs 27.5) and 256 up to 128 (and rows past 4096 elements on
-// more than 64: 4096 x 11008 at 128 34.9 vs 31.6), and SwiGLU pairs (11008 x 4096 at
-// 64: 40.5 vs 39.8).
+// own launches.  From 64 tokens the GEMM reuses each dequantised weight more:
+//   * of rows of up to 4096 elements it keeps launches of more than 512 row groups up to 80
+//     tokens (12288 x 4096 at 77: 28.0 vs 27.8 us), 288 up to 96 (4864 x 896 from 84 tokens
+//     on 1.04-1.07x its time here, 4864 x 4096 tiled 1.04) and 256 beyond;
+//   * longer rows' 8 K splits fill the GPU from fewer groups: it keeps more than 256 up to
+//     80 tokens (4864 x 5120 at 80 1.08x its time here, 8192 x 11008 1.07-1.17x), 128 up to
+//     96 (4096 x 6400 1.05-1.09x, 4864 x 11008 1.42x) and 64 beyond (4096 x 11008 at 128 34.9
+//     vs 31.6);
+//   * and SwiGLU pairs (11008 x 4096 at 64: 40.5 vs 39.8).
 //
 // K splits: by K alone, about 32 blocks each, none up to 16 blocks, where the 16-token
 // decode needs no workspace either (8 splits past 4096 elements: 896 x 4864
@@ -733,8 +736,8 @@ MidConfig linear_mid_pick(int M, const LinearSegs& s, int K) {
   const int64_t G = a.grp_end[a.count - 1];  // output row groups
   const int KB = K / kBlockElems;
   if (M >= 64) {
-    const bool takes = M <= 80 ? G <= 512 : M <= 96 ? G <= 304 : G <= 64 || (G <= 256 && K <= 4096);
-    if (swi || !takes) return c;
+    const int most = K <= 4096 ? (M <= 80 ? 512 : M <= 96 ? 288 : 256) : M <= 80 ? 256 : M <= 96 ? 128 : 64;
+    if (swi || G > most) return c;
   }
   c.parts = M < 64 ? 3 : 1;
   c.tt = M < 64 ? (M + 15) / 16 : M <= 64 ? 4 : M <= 80 ? 5 : M <= 96 ? 6 : 8;
