@@ -293,28 +293,35 @@ void graph_workspace_capacity(hipStream_t stream, size_t* bytes, size_t* counter
 // need: a plan names the larger of both, so a workspace sized for a batch serves the
 // smaller steps that take the general path.  Where the K splits' partials do not fit
 // (a caller-fixed workspace, or a captured stream's reservation made for the general
-// path) the row tiles go in several launches that reuse it: the same bits.  Where the
-// outputs of a fused launch alone would take another number of K splits, each gets a
-// launch of its own, so that it keeps the single Linear's bits.
+// path) the row tiles go in several launches that reuse it: the same bits.  The outputs
+// of a fused launch take the K splits that each takes alone, those that differ in a launch
+// of their own, so that every output keeps the single Linear's bits.
 bool run_mid(const char* what, const float* x, const mle::LinearSegs& s, int M, int K,
              const mle::SplitKNeed& general, const Exec& ex, int* rc) {
   mle::MidConfig c = mle::linear_mid_pick(M, s, K);
   if (c.tt == 0 || !mle::linear_mid_fits(M, K)) return false;
   if (s.mode == mle::Epilogue::kPlain && s.count > 1 && M < 64) {
-    mle::LinearSegs one[3];
-    bool same = true;
+    int splits[3];
     for (int i = 0; i < s.count; ++i) {
-      one[i] = s;
-      one[i].count = 1;
-      one[i].seg[0] = s.seg[i];
-      same &= mle::linear_mid_pick(M, one[i], K).splits == c.splits;
+      mle::LinearSegs one = s;
+      one.count = 1;
+      one.seg[0] = s.seg[i];
+      splits[i] = mle::linear_mid_pick(M, one, K).splits;
     }
-    if (!same) {
+    // The outputs that split as the first does, then the others.
+    mle::LinearSegs part[2] = {s, s};
+    part[0].count = part[1].count = 0;
+    for (int i = 0; i < s.count; ++i) {
+      mle::LinearSegs& p = part[splits[i] != splits[0]];
+      p.seg[p.count++] = s.seg[i];
+    }
+    if (part[1].count > 0) {
       *rc = MLE_OK;
-      for (int i = 0; i < s.count && *rc == MLE_OK; ++i)
-        (void)run_mid(what, x, one[i], M, K, general, ex, rc);
+      for (int g = 0; g < 2 && *rc == MLE_OK; ++g)
+        (void)run_mid(what, x, part[g], M, K, general, ex, rc);
       return true;
     }
+    c = mle::linear_mid_pick(M, s, K, splits[0]);
   }
   mle::SplitKNeed need = mle::linear_mid_workspace(c, s, K);
   if (ex.fixed || (!ex.planning() && stream_capturing(ex.stream))) {

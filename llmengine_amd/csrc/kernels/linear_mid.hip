@@ -20,8 +20,10 @@
 // lane's accumulators belong to one weight row and need one scale.  The K waves add
 // their sums in LDS; the K splits of a tile meet as in the MFMA decode (device-scope
 // partials, completion wait, counter, read-back in split order: deterministic).
-// The number of K splits follows K alone (linear_mid_pick), so a fused launch and
-// its single Linears add in the same order, as do raw and tiled weights.
+// The number of K splits follows K, the token tiles and, for vocabulary-sized weights
+// and very long rows, the output's own row groups (linear_mid_pick).  Raw and tiled
+// weights split alike; a fused launch below 64 tokens takes the splits that its outputs
+// take alone, in a second launch where they differ, so that it adds in the same order.
 //
 // What bounds it: the vector ALUs (activation split, int8 -> bf16, scale FMAs; the
 // MFMAs run beside them) and, on K = 4096, a fixed ~7 us of launch, first loads and
@@ -685,12 +687,17 @@ hipError_t launch_mid_rg(const MidConfig& c, const MidGrid& gr, WeightLayout lay
 //     vs 31.6);
 //   * and SwiGLU pairs (11008 x 4096 at 64: 40.5 vs 39.8).
 //
-// K splits: by K alone, about 32 blocks each, none up to 16 blocks, where the 16-token
-// decode needs no workspace either (8 splits past 4096 elements: 896 x 4864
-// at 32 tokens 9.1 us vs 12.0 with 4; 7 at three token tiles, as fast as 8, whose
-// partials stay within the 16-token decode's); one split for weights whose rows alone
-// fill the GPU several times over (3072 groups).  A SwiGLU pair,
-// which no single launch has to match, halves them until its grid fits the CUs.
+// K splits: about 32 blocks each, none up to 16 blocks, where the 16-token decode needs no
+// workspace either (8 splits past 4096 elements: 896 x 4864 at 32 tokens 9.1 us vs 12.0
+// with 4; 7 at three token tiles, as fast as 8, whose partials stay within the 16-token
+// decode's); one split for weights whose rows alone fill the GPU several times over (3072
+// groups).  Rows past 11264 elements of few groups: twice as many while the workgroups are
+// at most one a CU and a split keeps 16 blocks (32 x 65536 raw at 18 tokens 54.3 us with 8,
+// 16.5 with 64, 23.1 in two 16-token launches).  Shorter rows keep one count for every number of
+// groups, so that a fused launch and its outputs' own split alike (run_mid forms the launch
+// of outputs that do not by groups that do).  A SwiGLU pair, which no single launch has to
+// match, doubles them from any K while a split keeps 12 blocks (24 past 32 splits), and
+// halves them until its grid fits the CUs.
 // Row groups per wave (which no bits depend on).
 //   * Up to two token tiles: the fewest groups of one to three that keep the grid within
 //     one workgroup a CU (304 with one group, 4864 x 896 runs as well so as with two, and
@@ -728,7 +735,7 @@ static int mid_row_groups(const MidConfig& c, int64_t G, int K) {
   return best;
 }
 
-MidConfig linear_mid_pick(int M, const LinearSegs& s, int K) {
+MidConfig linear_mid_pick(int M, const LinearSegs& s, int K, int splits) {
   MidConfig c;
   if (M < 17 || M > 128 || s.layout == WeightLayout::kKN) return c;
   const MidArgs a = mid_args(s);
@@ -741,9 +748,16 @@ MidConfig linear_mid_pick(int M, const LinearSegs& s, int K) {
   }
   c.parts = M < 64 ? 3 : 1;
   c.tt = M < 64 ? (M + 15) / 16 : M <= 64 ? 4 : M <= 80 ? 5 : M <= 96 ? 6 : 8;
+  auto grid = [&](int rg) { return (G + kWN * rg - 1) / (kWN * rg) * c.splits; };
   c.splits = G >= 3072 || KB <= 16 ? 1 : KB <= 128 ? 4 : c.tt == 3 ? 7 : 8;
+  if (c.parts == 3 && c.splits > 1 && (swi || KB > 352)) {
+    const int least = swi ? 12 : 16;
+    while (grid(1) * 2 <= 256 && c.splits <= 32 &&
+           KB >= 2 * c.splits * (swi && c.splits >= 32 ? 24 : least))
+      c.splits *= 2;
+  }
+  if (splits > 0) c.splits = splits;
   if (swi) {
-    auto grid = [&](int rg) { return (G + kWN * rg - 1) / (kWN * rg) * c.splits; };
     c.rg = grid(1) <= 304 ? 2 : 4;  // half of each weight
     while (c.splits > 1 && grid(c.rg / 2) > 304) c.splits /= 2;
   } else {

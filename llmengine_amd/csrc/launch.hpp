@@ -147,7 +147,8 @@ struct MidConfig {
   int splits = 1;  // K splits asked for
   int tiles_per_launch = 0;  // row tiles a launch, the workspace reused; 0: all in one
 };
-MidConfig linear_mid_pick(int M, const LinearSegs& s, int K);
+// `splits` > 0: that many K splits instead of the pick's.
+MidConfig linear_mid_pick(int M, const LinearSegs& s, int K, int splits = 0);
 bool linear_mid_fits(int M, int K);
 SplitKNeed linear_mid_workspace(const MidConfig& c, const LinearSegs& s, int K);
 hipError_t launch_linear_mid(const MidConfig& c, const float* x, const LinearSegs& s, int M, int K,

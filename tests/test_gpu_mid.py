@@ -254,3 +254,59 @@ def test_mid_is_no_slower_than_the_gemm(dev, M, N, K):
                       lambda: capi.linear_ex(x, w, None, yg, M, N, K, path=2))
     assert rel_l2(to_host(y), to_host(yg)) <= 1e-2
     assert ratio <= 1.05, ratio
+
+
+@pytest.mark.parametrize("M,N,K,tiled", [(18, 24, 60000, False), (38, 100, 48000, True),
+                                         (20, 300, 27008, False), (34, 40, 58464, False)])
+def test_mid_long_rows_are_no_slower_than_chunks(dev, M, N, K, tiled):
+    """Few outputs of very long rows: K splits enough to occupy the GPU, so the launch takes
+    no longer than the 16-token chunks (these took 1.2-2.2 times as long with 8 splits)."""
+    note(f"mid long rows M={M} N={N} K={K} tiled={tiled}")
+    x, w = to_dev(S.activations(994, (M, K)), dev), to_dev(weight(995, N, K), dev)
+    if tiled:
+        w = tiled_dev(w, N, K, dev)
+    y, yd = empty_f32((M, N), dev), empty_f32((M, N), dev)
+    auto = capi.linear_tiled if tiled else capi.linear
+    ratio = slower_by(lambda: auto(x, w, None, y, M, N, K),
+                      lambda: capi.linear_ex(x, w, None, yd, M, N, K, path=3, tiled=tiled))
+    assert rel_l2(to_host(y), to_host(yd)) <= 1e-6
+    assert ratio <= 1.05, ratio
+
+
+@pytest.mark.parametrize("M,N,K", [(24, 640, 54336), (20, 200, 19680), (32, 400, 8192)])
+def test_mid_swiglu_long_rows_are_no_slower_than_chunks(dev, M, N, K):
+    """The same for a gate/up pair, against its calls for 16 tokens and for the rest."""
+    note(f"mid swiglu long rows M={M} N={N} K={K}")
+    x = to_dev(S.activations(996, (M, K)), dev)
+    g, u = to_dev(weight(997, N, K), dev), to_dev(weight(998, N, K), dev)
+    y, yc = empty_f32((M, N), dev), empty_f32((M, N), dev)
+
+    def chunks():
+        capi.linear_swiglu(x[:16], g, u, yc[:16], 16, N, K)
+        capi.linear_swiglu(x[16:], g, u, yc[16:], M - 16, N, K)
+
+    ratio = slower_by(lambda: capi.linear_swiglu(x, g, u, y, M, N, K), chunks)
+    assert rel_l2(to_host(y), to_host(yc)) <= 2e-6
+    assert ratio <= 1.05, ratio
+
+
+@pytest.mark.parametrize("Ns,K", [((4096, 512, 80), 12288), ((1000, 1000, 1000), 12288),
+                                  ((32, 2048, 32), 22528), ((16384, 16384, 16384), 1024),
+                                  ((49200, 64, 96), 544)])
+def test_mid_multi_of_different_splits(dev, Ns, K):
+    """Outputs that split K differently alone keep their single Linears' bits in one fused
+    call, and outputs that split alike share a launch."""
+    M = 21
+    note(f"mid multi of different splits Ns={Ns} K={K}")
+    x = to_dev(S.activations(975, (M, K)), dev)
+    ws = [to_dev(weight(976 + i, n, K), dev) for i, n in enumerate(Ns)]
+    ys = [empty_f32((M, n), dev) for n in Ns]
+    yt = [empty_f32((M, n), dev) for n in Ns]
+    capi.linear_multi(x, ws, [None] * 3, ys, Ns, M, K)
+    capi.linear_multi_tiled(x, [tiled_dev(w, n, K, dev) for w, n in zip(ws, Ns)], [None] * 3, yt,
+                            Ns, M, K)
+    for w, n, y, t in zip(ws, Ns, ys, yt):
+        one = empty_f32((M, n), dev)
+        capi.linear(x, w, None, one, M, n, K)
+        assert_bitexact(to_host(y), to_host(one), "fused vs single")
+        assert_bitexact(to_host(t), to_host(one), "tiled vs raw")
