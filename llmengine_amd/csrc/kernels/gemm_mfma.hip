@@ -685,12 +685,15 @@ GemmConfig gemm_mfma_pick_segs(int M, const LinearSegs& s, int K) {
   // 256 x 96 (tiled 212 -> 175 us, raw 220 -> 181), 2048 x 4096 x 4096 82 -> 74, 2048 x
   // 11008 x 4096 191 -> 182, three 4096 x 4096 outputs at 512 tokens (258 tiles of 96
   // columns) 76 -> 58; where both take the same rounds the narrower tile is faster
-  // (512 x 11008 x 4096 53 vs 60).
+  // (512 x 11008 x 4096 53 vs 60).  Their K step takes 1.00 us; they are taken where that
+  // estimate is a tenth below the others' (1.11), since a round also writes twice the
+  // outputs of a 128 x 128 one: of 3707 drawn shapes where the plain estimate was lower 94
+  // lost 3-16% (49722 x 1408 at 345 tokens 116 -> 127), with the margin 26 of 3328.
   struct Shape {
     int bm, bn;
     double step_us;
   };
-  static const Shape shapes[] = {{256, 128, 1.00}, {256, 96, 0.90}, {256, 64, 0.75}, {128, 128, 0.85},
+  static const Shape shapes[] = {{256, 128, 1.11}, {256, 96, 0.90}, {256, 64, 0.75}, {128, 128, 0.85},
                                  {128, 96, 0.62}, {128, 64, 0.52}};
   const bool swi = s.mode == Epilogue::kSwiGLU;
   const int count = swi ? 1 : s.count;

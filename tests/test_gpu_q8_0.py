@@ -12,7 +12,7 @@ import numpy as np
 import pytest
 
 from helpers import (assert_bitexact, bits, empty_f32, hybrid_decode, note, own_stream, rel_l2, sha,
-                     to_dev, to_host)
+                     slower_by, to_dev, to_host)
 from llmengine_amd import capi
 from llmengine_amd import synthetic as S
 
@@ -702,6 +702,22 @@ def test_linear_gemm_wide_tiles(dev, orc, M, N, K):
     assert rel_l2(got[rows], want) <= 1e-2
     g = (want - bias).astype(np.float64)
     assert rel_l2(to_host(ys)[rows], g / (1.0 + np.exp(-g)) * g) <= 1e-2
+
+
+@pytest.mark.parametrize("M,N,K,bm,bn", [(302, 53978, 32, 128, 128), (340, 52709, 5312, 128, 128),
+                                         (345, 49722, 1408, 128, 128)])
+def test_gemm_wide_tiles_only_where_they_gain(dev, M, N, K, bm, bn):
+    """Wide outputs of little more than one row tile: no slower than the narrower tiles that
+    the tuning hook forces (the best of nine runs each, in turn; the 256 x 128 tiles taken
+    for a round or two less took 1.07-1.16 times as long)."""
+    note(f"gemm wide tiles only where they gain M={M} N={N} K={K}")
+    x, w = to_dev(acts(540, M, K), dev), to_dev(weight(541, N, K), dev)
+    y, yg = empty_f32((M, N), dev), empty_f32((M, N), dev)
+    ratio = slower_by(lambda: capi.linear(x, w, None, y, M, N, K),
+                      lambda: capi.linear_ex(x, w, None, yg, M, N, K, path=2, splits=1, bm=bm,
+                                             bn=bn))
+    assert_bitexact(to_host(y), to_host(yg), "the same K steps in order")
+    assert ratio <= 1.05, ratio
 
 
 # ----------------------------------------------------------------------------- matmul
