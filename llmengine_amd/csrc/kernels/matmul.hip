@@ -11,8 +11,8 @@
 //
 // Kernels (from 64 rows of A, 16-byte aligned, the MatMul runs the bf16 MFMA GEMM
 // instead):
-//   * one or two rows of A: the half-block kernel below, lanes
-//     reading 16-byte pieces of whole blocks along a B row, fp32 FMAs;
+//   * one or two rows of A, and three on few columns of long K: the half-block kernel
+//     below, lanes reading 16-byte pieces of whole blocks along a B row, fp32 FMAs;
 //   * more: the MFMA kernel below, B read once per tile of up to 64 rows.
 // Where column tiles alone leave the GPU's 256 CUs short of work, K is spread over S
 // workgroups per tile.  Up to 8 rows of A they meet through a tile counter (a second
@@ -72,6 +72,9 @@ struct MfGrid {
   int tt, nbw, steps_per_split;
 };
 
+// Whether the K splits meet inside the launch (else in a second one).
+bool mf_handoff(int M) { return M <= 8; }
+
 MfGrid mf_grid(int M, int N, int K) {
   MfGrid g;
   g.tt = (M + 15) / 16;
@@ -88,14 +91,14 @@ MfGrid mf_grid(int M, int N, int K) {
   // (11008 x 4096 at 16 rows: 22.6 us with 5 splits, 25.7 with 6).
   int s = (int)((g.tt == 1 ? 512 : 256) / ((int64_t)g.tiles * g.row_tiles));
   if (s > steps / kMfWaves) s = steps / kMfWaves;
+  // A tile's last workgroup adds its splits alone: few columns of very long K are faster
+  // with fewer (4 x 480 x 32608 18.9 us with 127, 15.2 with 48; 16 take 21).
+  if (mf_handoff(M) && s > 48) s = 48;
   if (s < 1) s = 1;
   g.steps_per_split = (steps + s - 1) / s;
   g.splits = (unsigned)((steps + g.steps_per_split - 1) / g.steps_per_split);
   return g;
 }
-
-// Whether the K splits meet inside the launch (else in a second one).
-bool mf_handoff(int M) { return M <= 8; }
 
 template <int TT, int NBW>
 __global__ __launch_bounds__(kMfNT, 2) void matmul_q8_0_mfma_kernel(
@@ -378,7 +381,7 @@ __global__ __launch_bounds__(kMfNT, 2) void matmul_q8_0_mfma_kernel(
   }
 }
 
-// Half-block kernel (M <= 2).  A workgroup owns a tile of 256 output columns (8
+// Half-block kernel (M <= 2, and 3 on few columns).  A workgroup owns a tile of 256 output columns (8
 // blocks of a B row) for MR token rows and a run of K.  Lane c of a 16-lane group
 // takes 16 columns, half h = c % 2 of block c / 2 of the tile, of one B row per
 // step, so a group reads the tile's 272 contiguous bytes of a row and a wave four
@@ -652,9 +655,16 @@ void launch_ln(const LnGrid& g, const float* a, const uint8_t* b, float* c, int 
 
 // The half-block kernel's calls: up to two rows of A (MI355X, two rows: 4096 x 4096
 // 10.6 us vs 11.2 on the MFMA kernel, 11008 x 4096 20.3 vs 21.3; three and four rows
-// 13.9-14.5 vs 11.8, 21-28 vs 21.4) and B below 2 GiB (32-bit buffer offsets).
+// 13.9-14.5 vs 11.8, 21-28 vs 21.4), three where K is long over few columns, whose 16-row
+// MFMA tiles stay mostly empty (two row tiles read B twice, from the L2: 3 x 480 x 32608
+// 12.0 us vs 14.9, 3 x 1024 x 8192 1.24x, 3 x 2048 x 4096 1.11x; above 8.6 million elements
+// of B on more than 512 columns the MFMA kernel wins, 2048 x 5120 0.93x), and B below 2 GiB
+// (32-bit buffer offsets).
 bool use_half(int M, int N, int K) {
-  return M <= 2 && (int64_t)K * (N / kBlockElems) * kBlockBytes < (int64_t(1) << 31) &&
+  const int64_t elems = (int64_t)N * K;
+  const bool three = M == 3 && ((N <= 512 && K >= 8192) ||
+                                (K >= 3072 && elems >= 5000000 && elems <= 8600000));
+  return (M <= 2 || three) && (int64_t)K * (N / kBlockElems) * kBlockBytes < (int64_t(1) << 31) &&
          (int64_t)M * K * 4 < (int64_t(1) << 31);
 }
 
