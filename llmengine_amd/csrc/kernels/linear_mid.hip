@@ -155,7 +155,8 @@ __global__ __launch_bounds__(kNT, 2) void linear_mid_kernel(const float* __restr
   const int wn = wave / kWK, wk = wave % kWK;
   const int g = lane >> 4, r16 = lane & 15;
   const int KB = K / kBlockElems, KP = (KB + 1) >> 1;
-  const bool swi = args.swiglu != 0;
+  constexpr bool kPairs = PARTS == 3 && RG % 2 == 0;  // what a SwiGLU launch takes
+  const bool swi = kPairs && args.swiglu != 0;
   const int ph0 = blockIdx.y * phases_per_split;
   // Blocks [ph0 CB, KBE) are this split's; blocks past KBE read as zero
   // activations and zero scales.
@@ -482,7 +483,7 @@ __global__ __launch_bounds__(kNT, 2) void linear_mid_kernel(const float* __restr
 #pragma unroll
       for (int t = 0; t < TT; ++t) acc[rg][t] += red[((wn * RG + rg) * TT + t) * 64 + lane];
     if (swi) {
-      if constexpr (RG % 2 == 0) {
+      if constexpr (kPairs) {
 #pragma unroll
         for (int rg = 0; rg < RG / 2; ++rg) {
           const Out o = out_of(group_of(rg));
@@ -530,7 +531,7 @@ __global__ __launch_bounds__(kNT, 2) void linear_mid_kernel(const float* __restr
   if (tid == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   // Item i = (output group, token tile) goes to K wave i % kWK; all of a wave's
   // items of four splits are in flight at once.
-  constexpr int IT = RG % 2 == 0 ? 2 * ((RG / 2 * TT + 1) / 2) : (RG * TT + 1) / 2;
+  constexpr int IT = kPairs ? 2 * ((RG / 2 * TT + 1) / 2) : (RG * TT + 1) / 2;
   static_assert(kWK == 2, "two K waves share the items");
   const int items = RGO * TT;
   f32x4 sum[IT];
@@ -564,7 +565,7 @@ __global__ __launch_bounds__(kNT, 2) void linear_mid_kernel(const float* __restr
       for (int u = 0; u < IT; ++u) sum[u] += v[j][u];
   }
   if (swi) {
-    if constexpr (RG % 2 == 0) {
+    if constexpr (kPairs) {
 #pragma unroll
       for (int u = 0; u + 1 < IT; u += 2) {
         const int i = (u >> 1) * kWK + wk;
@@ -594,8 +595,9 @@ MidArgs mid_args(const LinearSegs& s) {
   return a;
 }
 
-// Row groups per wave that fit the registers without spills.
-constexpr int max_rg(int tt, int parts) { return parts == 3 ? 4 : tt <= 5 ? 3 : 2; }
+// Row groups per wave: all that fit the registers without spills below 64 tokens, from 64
+// on all that the pick's bounds on the row groups ask for.
+constexpr int max_rg(int tt, int parts) { return parts == 3 ? 4 : tt <= 6 ? 2 : 1; }
 
 struct MidGrid {
   unsigned tiles, splits;
@@ -655,7 +657,10 @@ hipError_t launch_mid_rg(const MidConfig& c, const MidGrid& gr, WeightLayout lay
                          hipStream_t stream) {
   switch (c.rg) {
     case 1: return launch_mid_k<TT, PARTS, 1>(gr, layout, x, M, K, ws, stream);
-    case 2: return launch_mid_k<TT, PARTS, 2>(gr, layout, x, M, K, ws, stream);
+    case 2:
+      if constexpr (max_rg(TT, PARTS) >= 2)
+        return launch_mid_k<TT, PARTS, 2>(gr, layout, x, M, K, ws, stream);
+      break;
     case 3:
       if constexpr (max_rg(TT, PARTS) >= 3)
         return launch_mid_k<TT, PARTS, 3>(gr, layout, x, M, K, ws, stream);
