@@ -116,7 +116,8 @@ int mle_q8_0_linear_swiglu(const float* x, const uint8_t* w_gate, const uint8_t*
 
 /*
  * Multi-output Q8_0 Linear: y[i][M,N[i]] = x[M,K] . W[i]^T (+ bias[i][N[i]]) for
- * i < count (1..3), in one launch that reads x once for all weights.
+ * i < count (1..3), in one launch that reads x once for all weights (17-63 tokens: in
+ * two where an output of 49152 rows, or of rows past 11264 elements, splits K otherwise).
  *
  * Replaces the q/k/v projections of one layer, three Linears on the same input
  * (src/model/transformer_graph_builder.cpp:214-221).  `bias` may be NULL (no
@@ -136,10 +137,11 @@ int mle_q8_0_linear_multi(const float* x, int count, const uint8_t* const* w,
  *
  * Replaces minillm::cuda::sgemm(const float* A, const uint8_t* B_q8_0, float* C,
  * int M, int N, int K)  (reference cuda_kernels.h:13, cuda_kernels.cu:852-868).
- * Elements as the reference CPU kernel cpu::sgemm(q8_0) forms them
- * (src/runtime/kernels/cpu_kernels.cpp:116-130), v = d*q in fp32.
- *   M < 64 (or A not 16-byte aligned): FP32 FMAs for one or two rows of A, else
- *   bf16 MFMA on a * d split exactly into three bf16 parts; the K sum is split into
+ * The reference CPU kernel cpu::sgemm(q8_0) sums a * (d * q), v = d*q in fp32
+ * (src/runtime/kernels/cpu_kernels.cpp:116-130).
+ *   M < 64 (or A not 16-byte aligned): FP32 FMAs on d * q for one or two rows of A
+ *   (three on few columns of long K), else bf16 MFMA on the fp32 product a * d split
+ *   exactly into three bf16 parts; the K sum is split into
  *   fixed pieces added in a fixed order (as the reference's device kernel
  *   splits K over warps), so results are deterministic and within fp32
  *   rounding of the CPU kernel (relative L2 <= 1e-5; small exact cases match it
@@ -222,7 +224,7 @@ int mle_argmax_f32(const float* logits, int rows, int n, int32_t* idx, float* va
  * The top_n tokens of each logits row with their softmax probabilities, on the
  * device: Sampler::get_top_tokens (src/runtime/sampler.cpp:141-197).  Row r of
  * n logits is scaled by 1 / temperature when temperature > 0 and != 1, then
- * p = exp(v - max) * (1 / sum); ids[r*k + j], probs[r*k + j] (k = min(top_n, n))
+ * p = exp(v - max) / sum (sum and quotient in fp64, rounded once); ids[r*k + j], probs[r*k + j] (k = min(top_n, n))
  * are the top k tokens, largest probability first, ties to the lower index.  A
  * row with a NaN, a non-finite maximum or a non-finite or zero sum gives the
  * uniform 1/n (ids 0, 1, ...), as the reference does.  With the k candidates

@@ -350,8 +350,8 @@ bool run_mid(const char* what, const float* x, const mle::LinearSegs& s, int M, 
 
 // Tiled weights (mle::WeightLayout::kTiled): the tiled FP32 GEMV where
 // mle::gemv_tiled_wins (one token; two below vocabulary-sized outputs; up to
-// four on short rows), else the MFMA decode below 64 tokens and the MFMA GEMM
-// from 64.
+// four on short rows), else the MFMA decode up to 16 tokens, the batch kernel of
+// linear_mid.hip (run_mid) from 17 and, on more row groups, the MFMA GEMM from 64.
 int run_linear(const float* x, const uint8_t* w, const void* bias, float* y, int M,
                int N, int K, int path, const Tune& tune, const Exec& ex,
                mle::WeightLayout layout = mle::WeightLayout::kRaw, bool bias_bf16 = false) {
@@ -450,8 +450,9 @@ int run_linear(const float* x, const uint8_t* w, const void* bias, float* y, int
 // One launch over 1-3 output segments (multi-output Linear) or a gate/up pair
 // (SwiGLU): the same path choice as a single Linear (bf16 MFMA GEMM for
 // M >= 64, FP32 GEMV for M == 1, for M <= 4 on short rows and for M == 2 on
-// rows of 2048-4096 elements, else the MFMA
-// decode kernel in chunks of up to 16 tokens with FP32-exact activations);
+// rows of 2048-4096 elements, the batch kernel for 17-63 tokens and, on few row groups,
+// up to 128 (run_mid), else the MFMA decode kernel with FP32-exact activations, in chunks
+// of up to 16 tokens where the batch kernel's offsets do not fit);
 // SwiGLU takes the GEMV for M == 1 only.
 int run_segs(const char* ctx, const float* x, const mle::LinearSegs& s, int M, int K,
              const Exec& ex) {
@@ -611,7 +612,7 @@ mle::SplitKNeed matmul_need(int M, int N, int K) {
 
 // MatMul from 64 rows of A on the bf16 MFMA GEMM (B[K, N] dequantised
 // transposed into its W tile); below that, and where B's offsets would not fit
-// 32 bits, the FP32 kernel of matmul.hip.  Fills the GEMM's tile choice and
+// 32 bits, the kernels of matmul.hip (fp32 rounding).  Fills the GEMM's tile choice and
 // segment (B and C are set by the caller).
 bool matmul_on_gemm(int M, int N, int K, mle::GemmConfig* c, mle::LinearSegs* s) {
   if (M < 64) return false;

@@ -2,10 +2,11 @@
 //
 // B is one Q8_0 stream in row-major [K, N] order, so element (k, n) is flat
 // index k*N + n and blocks run along N (reference
-// src/runtime/kernels/cpu_kernels.cpp:116-130, cuda_kernels.cu:296-331).  Each
-// element is formed as the reference forms it, v = d * q in fp32, and the K sum
-// is an fp32 FMA chain split into fixed pieces added in a fixed order, so the
-// result is deterministic and within fp32 rounding of the reference's
+// src/runtime/kernels/cpu_kernels.cpp:116-130, cuda_kernels.cu:296-331).  The
+// reference forms v = d * q in fp32 and sums a * v.  The half-block kernel does so in
+// fp32 FMA chains; the MFMA kernel rounds a * d to fp32 instead (q is exact beside it)
+// and sums on the matrix cores.  Both split the K sum into fixed pieces added in a fixed
+// order, so the result is deterministic and within fp32 rounding of the reference's
 // sequential sum (relative L2 ~1e-7), as the reference's own device kernel is
 // (it splits K over 8 warps and adds their partials).
 //
@@ -37,7 +38,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t mm_rsrc(const void* base, uint
                                            0x00020000);
 }
 
-// MFMA kernel (3 to 64 rows of A), fp32-exact operands.
+// MFMA kernel (3 and more rows of A, up to 64 a workgroup), fp32-exact operands.
 //
 // A block of B holds 32 columns of one k, so its scale cannot leave the K sum; it goes
 // into the activations instead: for one 32-column block, c[m, n] = sum_k (a[m, k]
@@ -60,10 +61,10 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t mm_rsrc(const void* base, uint
 //
 // Bound by the vector ALUs (8 products, the split of 8 values and 16 int8 -> bf16
 // conversions a lane for 6 TT MFMAs).  Measured (MI355X, rotated B, us, against fp32
-// FMAs on up to 8 rows at a time): 4096 x 4096 at M = 4 / 8 / 16 / 63 14.5 / 28.0 /
-// 43.4 / 127 -> 11.9 / 12.0 / 13.3 / 23.6; 11008 x 4096 21.4 / 38.0 / 102 / 370 -> 21.4
-// / 21.7 / 22.6 / 52.5; [896, 151936] 48.7 / 87.1 / 288 / 1028 -> 43.4 / 44.5 / 47.8 /
-// 146.  256-column wave tiles (one workgroup a CU) were 1.1-1.5x slower.
+// FMAs on up to 8 rows at a time): 4096 x 4096 at M = 4 / 8 / 16 / 63 14.1 / 27.4 /
+// 40.7 / 121 -> 11.7 / 11.5 / 12.4 / 21.6; 11008 x 4096 21.2 / 38.7 / 103 / 371 -> 21.1
+// / 20.7 / 22.6 / 51.4; [896, 151936] 49.3 / 90.6 / 293 / 1029 -> 43.9 / 43.7 / 45.1 /
+// 147.  256-column wave tiles (one workgroup a CU) were 1.1-1.5x slower.
 constexpr int kMfWaves = 8;
 constexpr int kMfNT = 64 * kMfWaves;
 

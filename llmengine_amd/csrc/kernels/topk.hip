@@ -2,9 +2,9 @@
 //
 // For each row r of n logits: scaled = logits * (1 / temperature) when
 // temperature > 0 and != 1 (else the logits as they are); p = softmax(scaled),
-// computed as exp(scaled - max) * (1 / sum); ids[r, j], probs[r, j] for
-// j < min(top_n, n) are the top_n tokens by probability, largest first, ties
-// to the lower index.  A row whose maximum is not finite, whose sum is not
+// computed as exp(scaled - max) / sum (the sum and the quotient in fp64); ids[r, j],
+// probs[r, j] for j < min(top_n, n) are the top_n tokens by probability, largest
+// first, ties to the lower index.  A row whose maximum is not finite, whose sum is not
 // finite or not positive, or that holds a NaN gives the uniform distribution
 // 1 / n, i.e. ids 0, 1, 2, ... .  This is Sampler::get_top_tokens
 // (src/runtime/sampler.cpp:141-197; the same softmax as Sampler::sample,
@@ -38,7 +38,7 @@
 //
 // Latency bounds it, not bytes (8 rows x 152k logits are 4.9 MB).  Selecting top_n keys
 // in every chunk instead (a radix select per chunk, then one over 75 x top_n
-// candidates) took 31.6 us for 8 rows at top_n 40 (MI355X); this takes 12.5.  Pass 2
+// candidates) took 31.6 us for 8 rows at top_n 40 (MI355X); this takes 12.3.  Pass 2
 // issues all its loads of a stage before it uses one, and a NaN travels as an infinite
 // maximum instead of through a reduction of its own (13.7 us otherwise).
 #include "../launch.hpp"

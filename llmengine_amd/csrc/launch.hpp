@@ -186,7 +186,7 @@ GemmConfig gemm_mfma_pick_kn(int M, int N, int K);
 
 // MatMul C[M,N] = A[M,K] . B[K,N] with B in Q8_0 blocks along N.  When the
 // launch spreads K over several workgroups per tile it needs the workspace
-// matmul_workspace(M, N, K) names: `partials` floats and, for M <= 2, tile
+// matmul_workspace(M, N, K) names: `partials` floats and, for M <= 8, tile
 // counters (zero between launches; the kernel resets them).
 struct MatmulNeed {
   size_t partial_floats = 0;
