@@ -89,11 +89,6 @@ __device__ __forceinline__ uint32_t cvt_bf16x2(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, bf16x2));
 }
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* base, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes,
-                                           0x00020000);
-}
-
 int padded_k(int K) { return (K + BK - 1) / BK * BK; }
 
 // X fp32 [M, K] -> Xf: bf16 (round to nearest even) in MFMA fragment order.
@@ -152,11 +147,6 @@ struct GemmArgs {
   unsigned tile_end[3];
   int count;
 };
-
-// silu(g) * u with the reference's operation order (cpu_kernels.cpp:848-858).
-__device__ __forceinline__ float silu_mul(float g, float u) {
-  return (g / (1.0f + expf(-g))) * u;
-}
 
 // MODE 0: plain / multi-output Linear.  MODE 1 (SwiGLU): tile columns
 // [0, BN/2) are rows of the gate weight and [BN/2, BN) the same rows of the up
@@ -285,7 +275,7 @@ __global__ __launch_bounds__(Roles<MI>::kThreads, 1) void gemm_q8_0_mfma_kernel(
   constexpr int SC1 = 16;  // cache-policy bit: device scope
   const uint32_t tile = blockIdx.y * gridDim.x + blockIdx.x;
   const __amdgpu_buffer_rsrc_t prs =
-      rsrc(partials + (int64_t)tile * gridDim.z * TILE_ELEMS, gridDim.z * TILE_ELEMS * 4u);
+      buffer_rsrc(partials + (int64_t)tile * gridDim.z * TILE_ELEMS, gridDim.z * TILE_ELEMS * 4u);
   auto slot = [&](int i, int jj, int q) {  // byte offset of 4 accumulators
     return (uint32_t)((((i * NJ + jj) * 4 + q) * (64 * CW) + tid) * 16);
   };
@@ -350,7 +340,7 @@ __global__ __launch_bounds__(Roles<MI>::kThreads, 1) void gemm_q8_0_mfma_kernel(
         for (int v = 0; v < 16; ++v) acc[i][jj][v] = 0.0f;
     // A: fragments of 32-row tile R at step s start at byte ((R n_steps + s) 4
     // + j) KB; tiles past the converted rows read as zero.
-    const __amdgpu_buffer_rsrc_t xrs = rsrc(xf, xf_bytes);
+    const __amdgpu_buffer_rsrc_t xrs = buffer_rsrc(xf, xf_bytes);
     uint32_t xoff[MW];
 #pragma unroll
     for (int i = 0; i < MW; ++i)
@@ -431,14 +421,14 @@ __global__ __launch_bounds__(Roles<MI>::kThreads, 1) void gemm_q8_0_mfma_kernel(
     const uint8_t* wsrc = up_rows ? args.seg[1].w : w;
     const int64_t wrows = min((int64_t)BNO, (int64_t)N - n0);
     const uint8_t* wtile = wsrc + n0 * row_bytes;
-    const __amdgpu_buffer_rsrc_t wrs = rsrc(wtile, (uint32_t)(wrows * row_bytes));
+    const __amdgpu_buffer_rsrc_t wrs = buffer_rsrc(wtile, (uint32_t)(wrows * row_bytes));
     const uint32_t boff = (uint32_t)prow * row_bytes + (uint32_t)wn_h * kBlockBytes;
     // MatMul: B row k holds NB = N / 32 blocks; the item's blocks are column
     // block n0 / 32 + kn_c of rows 64 s + 2 kn_kp and + 1.  Rows past K read as
     // zero through the range check, column blocks past N are masked.
     const int NBK = N / kBlockElems;
     const uint32_t kn_row = (uint32_t)NBK * kBlockBytes;
-    const __amdgpu_buffer_rsrc_t knrs = rsrc(wsrc, (uint32_t)((int64_t)K * kn_row));
+    const __amdgpu_buffer_rsrc_t knrs = buffer_rsrc(wsrc, (uint32_t)((int64_t)K * kn_row));
     const bool kn_live = n0 / kBlockElems + kn_c < NBK;
     const uint32_t kn_off = (uint32_t)(2 * kn_kp) * kn_row + (uint32_t)(n0 / kBlockElems + kn_c) * kBlockBytes;
     const uint32_t kn_mis0 = (uint32_t)(((uintptr_t)wsrc + kn_off) & 2u);
@@ -458,8 +448,8 @@ __global__ __launch_bounds__(Roles<MI>::kThreads, 1) void gemm_q8_0_mfma_kernel(
     const int64_t ngr = min((int64_t)(BNO / kTileRows), G - g0);
     const uint8_t* tq_base = wsrc + g0 * KP * kTilePieceBytes;
     const uint8_t* ts_base = wsrc + G * KP * kTilePieceBytes + g0 * KP * kTileScaleBytes;
-    const __amdgpu_buffer_rsrc_t tqrs = rsrc(tq_base, (uint32_t)(ngr * KP * kTilePieceBytes));
-    const __amdgpu_buffer_rsrc_t tsrs = rsrc(ts_base, (uint32_t)(ngr * KP * kTileScaleBytes));
+    const __amdgpu_buffer_rsrc_t tqrs = buffer_rsrc(tq_base, (uint32_t)(ngr * KP * kTilePieceBytes));
+    const __amdgpu_buffer_rsrc_t tsrs = buffer_rsrc(ts_base, (uint32_t)(ngr * KP * kTileScaleBytes));
     const uint32_t tqv = (uint32_t)(prow / kTileRows) * KP * kTilePieceBytes +
                          (uint32_t)(32 * wn_h + prow % kTileRows) * 16;
     const uint32_t tsv = (uint32_t)(prow / kTileRows) * KP * kTileScaleBytes +

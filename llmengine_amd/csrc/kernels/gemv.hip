@@ -42,11 +42,6 @@ struct GemvArgs {
   int count;
 };
 
-// silu(g) * u with the reference's operation order (cpu_kernels.cpp:848-858).
-__device__ __forceinline__ float silu_mul(float g, float u) {
-  return (g / (1.0f + expf(-g))) * u;
-}
-
 // One lane's contribution of block `blk[r]` (activations from LDS) to acc[m][r].
 template <int MT, int RW>
 __device__ __forceinline__ void consume(float (&acc)[MT][RW], const Block (&blk)[RW],
@@ -267,11 +262,6 @@ __global__ __launch_bounds__(256) void gemv_q8_0_kernel(const float* __restrict_
 // (each lane's whole share requested up front).
 constexpr int kRawkRows = 4;
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t gemv_rsrc(const void* base, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes,
-                                           0x00020000);
-}
-
 // Sums each of the V per-lane values v[0..V) over the wave's 64 lanes (V a power
 // of two, <= 64).  On return v[0] of lane l holds the total of value l >> (6 - log2 V).
 template <int V>
@@ -324,9 +314,9 @@ __global__ __launch_bounds__(512) void gemv_rawk_kernel(const float* __restrict_
   // the offset's.
   const int64_t live_rows = N - row0 < RPW ? N - row0 : RPW;
   const uint8_t* base = w + row0 * row_bytes;
-  const __amdgpu_buffer_rsrc_t wrs = gemv_rsrc(base, (uint32_t)(live_rows * row_bytes));
+  const __amdgpu_buffer_rsrc_t wrs = buffer_rsrc(base, (uint32_t)(live_rows * row_bytes));
   const uint32_t phase = (uint32_t)((uintptr_t)base & 2u);
-  const __amdgpu_buffer_rsrc_t xrs = gemv_rsrc(x, (uint32_t)K * 4u);
+  const __amdgpu_buffer_rsrc_t xrs = buffer_rsrc(x, (uint32_t)K * 4u);
 
   float acc[RPW];
 #pragma unroll

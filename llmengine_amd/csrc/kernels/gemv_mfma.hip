@@ -54,13 +54,6 @@
 namespace mle {
 namespace {
 
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-
-__device__ __forceinline__ uint32_t top_halves(uint32_t lo_word, uint32_t hi_word) {
-  // bf16 pair from the upper 16 bits of two fp32 bit patterns (lo in bits 0-15).
-  return __builtin_amdgcn_perm(hi_word, lo_word, 0x07060302u);
-}
-
 // Splits 8 activations into packed bf16 hi / mid / lo parts (4 dwords each):
 // hi = x with the low 16 bits cleared, r = x - hi (exact), mid = r with the low
 // 16 bits cleared, lo = r - mid (exact, <= 8 significant bits).  Finite x only.
@@ -107,16 +100,6 @@ __device__ __forceinline__ void split3_any(const float (&v)[8], uint32_t (&hi)[4
     mid[p] = top_halves(rb[2 * p], rb[2 * p + 1]);
     lo[p] = top_halves(lb[2 * p], lb[2 * p + 1]);
   }
-}
-
-// 8 int8 quants (two dwords) -> 8 bf16 (exact).
-__device__ __forceinline__ bf16x8_t quants_to_bf16(uint32_t q0, uint32_t q1) {
-  u32x4 o;
-  o.x = top_halves(__builtin_bit_cast(uint32_t, q_at(q0, 0)), __builtin_bit_cast(uint32_t, q_at(q0, 1)));
-  o.y = top_halves(__builtin_bit_cast(uint32_t, q_at(q0, 2)), __builtin_bit_cast(uint32_t, q_at(q0, 3)));
-  o.z = top_halves(__builtin_bit_cast(uint32_t, q_at(q1, 0)), __builtin_bit_cast(uint32_t, q_at(q1, 1)));
-  o.w = top_halves(__builtin_bit_cast(uint32_t, q_at(q1, 2)), __builtin_bit_cast(uint32_t, q_at(q1, 3)));
-  return __builtin_bit_cast(bf16x8_t, o);
 }
 
 // In-register 4 x 4 transpose of 8-byte chunks across the four 16-lane rows of
@@ -202,12 +185,6 @@ __device__ __forceinline__ int bslot_rd(int kb, int p, int c, int n) {
   return bslot<MT, W, P>(kb, p, c, n);
 }
 
-// Buffer resource over [base, base + bytes): loads past the end return zero.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes,
-                                           0x00020000);
-}
-
 // Output segments as the kernel sees them: segment i owns the row tiles
 // [tile_end[i-1], tile_end[i]) of the grid.
 struct DecodeArgs {
@@ -215,11 +192,6 @@ struct DecodeArgs {
   unsigned tile_end[3];
   int count;
 };
-
-// silu(g) * u with the reference's operation order (cpu_kernels.cpp:848-858).
-__device__ __forceinline__ float silu_mul(float g, float u) {
-  return (g / (1.0f + expf(-g))) * u;
-}
 
 // MODE 0: plain / multi-output Linear.  MODE 1 (SwiGLU): waves [0, W/2) take
 // rows of the gate weight, waves [W/2, W) the same rows of the up weight, and
@@ -280,7 +252,7 @@ __global__ __launch_bounds__(64 * W) void gemv_q8_0_mfma_kernel(
   // alignment (the realignment case of load_block_raw) never changes.
   const uint8_t* wbase = w + n0 * row_bytes;
   const int64_t rows_here = min((int64_t)ROUT, (int64_t)N - n0);
-  const __amdgpu_buffer_rsrc_t wrs = make_rsrc(wbase, (uint32_t)(rows_here * row_bytes));
+  const __amdgpu_buffer_rsrc_t wrs = buffer_rsrc(wbase, (uint32_t)(rows_here * row_bytes));
   const uint32_t lane_off = (uint32_t)(wrow * 16 + r16) * row_bytes +
                             (uint32_t)(kb0 + g) * kBlockBytes;
   const uint32_t mis = (uint32_t)(((uintptr_t)wbase + lane_off) & 2u);
@@ -292,7 +264,7 @@ __global__ __launch_bounds__(64 * W) void gemv_q8_0_mfma_kernel(
   //    barrier overlap the weight loads still in flight.  Item = (token m
   //    fastest, k quarter, block); items past the end (token >= M, block >=
   //    nblk, or no item) read zeros.
-  const __amdgpu_buffer_rsrc_t xrs = make_rsrc(x, (uint32_t)((int64_t)M * K * 4));
+  const __amdgpu_buffer_rsrc_t xrs = buffer_rsrc(x, (uint32_t)((int64_t)M * K * 4));
   f32x4 xv[XPT][2];
 #pragma unroll
   for (int i = 0; i < XPT; ++i) {
@@ -346,9 +318,9 @@ __global__ __launch_bounds__(64 * W) void gemv_q8_0_mfma_kernel(
     const uint8_t* qb = w + rgc * KP * kTilePieceBytes;
     const uint8_t* sb = w + G * KP * kTilePieceBytes + rgc * KP * kTileScaleBytes;
     const __amdgpu_buffer_rsrc_t qrs =
-        make_rsrc(qb, rg < G ? (uint32_t)KP * kTilePieceBytes : 0u);
+        buffer_rsrc(qb, rg < G ? (uint32_t)KP * kTilePieceBytes : 0u);
     const __amdgpu_buffer_rsrc_t srs =
-        make_rsrc(sb, rg < G ? (uint32_t)KP * kTileScaleBytes : 0u);
+        buffer_rsrc(sb, rg < G ? (uint32_t)KP * kTileScaleBytes : 0u);
     const int p0 = kb0 >> 1;  // KSL is even
     {
 #pragma unroll
@@ -434,14 +406,14 @@ __global__ __launch_bounds__(64 * W) void gemv_q8_0_mfma_kernel(
   // Block kc of chunk (kb = block within the slice): P chained MFMAs against
   // the token columns, then the fp32 scale FMA into an accumulator that takes
   // every other block (even blocks in accs[0], odd in accs[1], in K order).
-  auto block_mma = [&](int kc, int kb, const bf16x8_t a, f32x4& a4) {
+  auto block_mma = [&](int kc, int kb, const bf16x8 a, f32x4& a4) {
     f32x4 d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-        a, *reinterpret_cast<const bf16x8_t*>(bfr + bslot_rd<MT, W, P>(kb, 0, g, r16)),
+        a, *reinterpret_cast<const bf16x8*>(bfr + bslot_rd<MT, W, P>(kb, 0, g, r16)),
         f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
     for (int p = 1; p < P; ++p)
       d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-          a, *reinterpret_cast<const bf16x8_t*>(bfr + bslot_rd<MT, W, P>(kb, p, g, r16)), d, 0,
+          a, *reinterpret_cast<const bf16x8*>(bfr + bslot_rd<MT, W, P>(kb, p, g, r16)), d, 0,
           0, 0);
     // D layout: lane l holds rows 4 (l/16) + v (v = 0..3), virtual column l % 16.
     const f32x4 sc = *reinterpret_cast<const f32x4*>(&scl[wave][kc][4 * g]);
@@ -548,7 +520,7 @@ __global__ __launch_bounds__(64 * W) void gemv_q8_0_mfma_kernel(
   constexpr int REGION = S::R * MT;
   constexpr int SC1 = 16;  // cache-policy bit: device scope
   const __amdgpu_buffer_rsrc_t prs =
-      make_rsrc(partials + (int64_t)blockIdx.x * gridDim.y * REGION,
+      buffer_rsrc(partials + (int64_t)blockIdx.x * gridDim.y * REGION,
                 (uint32_t)(gridDim.y * REGION * 4));
 #pragma unroll
   for (int o = 0; o < S::OPL; ++o) {
@@ -747,7 +719,7 @@ __global__ __launch_bounds__(64 * WG * NG) void gemv_mfma_rows_kernel(
 
   // Activations of one phase: item (token m fastest, k quarter, block), 8 fp32.
   // Items past M or K read zeros through the range check of the per-lane offset.
-  const __amdgpu_buffer_rsrc_t xrs = make_rsrc(x, (uint32_t)((int64_t)M * K * 4));
+  const __amdgpu_buffer_rsrc_t xrs = buffer_rsrc(x, (uint32_t)((int64_t)M * K * 4));
   f32x4 xv[NPH][XPT][2];
   auto load_x = [&](int ph) {
 #pragma unroll
@@ -774,12 +746,12 @@ __global__ __launch_bounds__(64 * WG * NG) void gemv_mfma_rows_kernel(
   // lane's 4-byte alignment phase is fixed.
   const uint8_t* qb = w + rgc * KP * kTilePieceBytes;
   const uint8_t* sb = w + G * KP * kTilePieceBytes + rgc * KP * kTileScaleBytes;
-  const __amdgpu_buffer_rsrc_t qrs = make_rsrc(qb, live_g ? (uint32_t)KP * kTilePieceBytes : 0u);
-  const __amdgpu_buffer_rsrc_t srs = make_rsrc(sb, live_g ? (uint32_t)KP * kTileScaleBytes : 0u);
+  const __amdgpu_buffer_rsrc_t qrs = buffer_rsrc(qb, live_g ? (uint32_t)KP * kTilePieceBytes : 0u);
+  const __amdgpu_buffer_rsrc_t srs = buffer_rsrc(sb, live_g ? (uint32_t)KP * kTileScaleBytes : 0u);
   const uint32_t row_bytes = (uint32_t)KB * kBlockBytes;
   const uint8_t* gbase = w + rgc * kTileRows * (int64_t)row_bytes;
   const int64_t grows = live_g ? min((int64_t)kTileRows, (int64_t)N - rgc * kTileRows) : 0;
-  const __amdgpu_buffer_rsrc_t wrs = make_rsrc(gbase, (uint32_t)(grows * row_bytes));
+  const __amdgpu_buffer_rsrc_t wrs = buffer_rsrc(gbase, (uint32_t)(grows * row_bytes));
   const uint32_t lane_off = (uint32_t)r16 * row_bytes + (uint32_t)(2 * qw * WPP + g) * kBlockBytes;
   const uint32_t mis = (uint32_t)(((uintptr_t)gbase + lane_off) & 2u);
   const uint32_t voff = lane_off + mis;
@@ -845,14 +817,14 @@ __global__ __launch_bounds__(64 * WG * NG) void gemv_mfma_rows_kernel(
   }
 
   f32x4 accs[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
-  auto block_mma = [&](const uint8_t* bb, int kc, int kb, const bf16x8_t a, f32x4& a4) {
+  auto block_mma = [&](const uint8_t* bb, int kc, int kb, const bf16x8 a, f32x4& a4) {
     f32x4 d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-        a, *reinterpret_cast<const bf16x8_t*>(bb + bslot_rd<MT, 4, P>(kb, 0, g, r16)),
+        a, *reinterpret_cast<const bf16x8*>(bb + bslot_rd<MT, 4, P>(kb, 0, g, r16)),
         f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
     for (int p = 1; p < P; ++p)
       d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-          a, *reinterpret_cast<const bf16x8_t*>(bb + bslot_rd<MT, 4, P>(kb, p, g, r16)), d, 0,
+          a, *reinterpret_cast<const bf16x8*>(bb + bslot_rd<MT, 4, P>(kb, p, g, r16)), d, 0,
           0, 0);
     const f32x4 sc = *reinterpret_cast<const f32x4*>(&scl[wave][kc][4 * g]);
     a4.x = __builtin_fmaf(sc.x, d.x, a4.x);
@@ -1165,7 +1137,7 @@ __global__ __launch_bounds__(64 * WG * NG) void gemv_mfma_hyb_kernel(
 
   // 0. This split's activations first: item (token m fastest, k quarter, block
   //    of the B area); items past M, past the split or past K read zeros.
-  const __amdgpu_buffer_rsrc_t xrs = make_rsrc(x, (uint32_t)((int64_t)M * K * 4));
+  const __amdgpu_buffer_rsrc_t xrs = buffer_rsrc(x, (uint32_t)((int64_t)M * K * 4));
   f32x4 xv[XPT][2];
 #pragma unroll
   for (int i = 0; i < XPT; ++i) {
@@ -1187,15 +1159,15 @@ __global__ __launch_bounds__(64 * WG * NG) void gemv_mfma_hyb_kernel(
   constexpr bool kTiled = LAYOUT == int(WeightLayout::kTiled);
   const uint8_t* qb = w + rg * KP * kTilePieceBytes;
   const uint8_t* sb = w + G * KP * kTilePieceBytes + rg * KP * kTileScaleBytes;
-  const __amdgpu_buffer_rsrc_t qrs = make_rsrc(qb, live_g ? (uint32_t)KP * kTilePieceBytes : 0u);
-  const __amdgpu_buffer_rsrc_t srs = make_rsrc(sb, live_g ? (uint32_t)KP * kTileScaleBytes : 0u);
+  const __amdgpu_buffer_rsrc_t qrs = buffer_rsrc(qb, live_g ? (uint32_t)KP * kTilePieceBytes : 0u);
+  const __amdgpu_buffer_rsrc_t srs = buffer_rsrc(sb, live_g ? (uint32_t)KP * kTileScaleBytes : 0u);
   // Raw: one buffer over the group's rows (rows past N read as zero); a chunk's
   // blocks start 8-block (272-byte) steps apart, so each lane's 4-byte alignment
   // phase is fixed.
   const uint32_t row_bytes = (uint32_t)KB * kBlockBytes;
   const uint8_t* gbase = w + rg * kTileRows * (int64_t)row_bytes;
   const int64_t grows = live_g ? min((int64_t)kTileRows, (int64_t)N - rg * kTileRows) : 0;
-  const __amdgpu_buffer_rsrc_t wrs = make_rsrc(gbase, (uint32_t)(grows * row_bytes));
+  const __amdgpu_buffer_rsrc_t wrs = buffer_rsrc(gbase, (uint32_t)(grows * row_bytes));
   const uint32_t lane_off =
       (uint32_t)r16 * row_bytes + (uint32_t)(kb0 + 2 * qw * WPP + g) * kBlockBytes;
   const uint32_t mis = (uint32_t)(((uintptr_t)gbase + lane_off) & 2u);
@@ -1287,14 +1259,14 @@ __global__ __launch_bounds__(64 * WG * NG) void gemv_mfma_hyb_kernel(
   // 3. Chunks in order as their loads land: P chained MFMAs per block, fp32
   //    scale FMA into the even / odd accumulators (the kernels' arithmetic).
   f32x4 accs[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
-  auto block_mma = [&](int kc, int kb, const bf16x8_t a, f32x4& a4) {
+  auto block_mma = [&](int kc, int kb, const bf16x8 a, f32x4& a4) {
     f32x4 d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-        a, *reinterpret_cast<const bf16x8_t*>(bfr + bslot_rd<MT, 4, P>(kb, 0, g, r16)),
+        a, *reinterpret_cast<const bf16x8*>(bfr + bslot_rd<MT, 4, P>(kb, 0, g, r16)),
         f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
     for (int p = 1; p < P; ++p)
       d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-          a, *reinterpret_cast<const bf16x8_t*>(bfr + bslot_rd<MT, 4, P>(kb, p, g, r16)), d, 0,
+          a, *reinterpret_cast<const bf16x8*>(bfr + bslot_rd<MT, 4, P>(kb, p, g, r16)), d, 0,
           0, 0);
     const f32x4 sc = *reinterpret_cast<const f32x4*>(&scl[wave][kc][4 * g]);
     a4.x = __builtin_fmaf(sc.x, d.x, a4.x);
@@ -1399,7 +1371,7 @@ __global__ __launch_bounds__(64 * WG * NG) void gemv_mfma_hyb_kernel(
   constexpr int SC1 = 16;  // cache-policy bit: device scope
   const unsigned nspl = gridDim.y;
   const __amdgpu_buffer_rsrc_t prs =
-      make_rsrc(partials + (int64_t)blockIdx.x * nspl * REGION, (uint32_t)(nspl * REGION * 4));
+      buffer_rsrc(partials + (int64_t)blockIdx.x * nspl * REGION, (uint32_t)(nspl * REGION * 4));
   if (qw == 0) {
 #pragma unroll
     for (int o = 0; o < OPL; ++o) {

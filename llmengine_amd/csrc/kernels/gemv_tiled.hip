@@ -24,20 +24,10 @@
 namespace mle {
 namespace {
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_of(const void* base, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes,
-                                           0x00020000);
-}
-
 // Orders this wave's LDS accesses on either side (other lanes' values are read).
 __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
   __builtin_amdgcn_wave_barrier();
-}
-
-// silu(g) * u with the reference's operation order (cpu_kernels.cpp:848-858).
-__device__ __forceinline__ float silu_mul_t(float g, float u) {
-  return (g / (1.0f + expf(-g))) * u;
 }
 
 struct TiledGemvArgs {
@@ -92,11 +82,11 @@ __global__ __launch_bounds__(1024) void gemv_tiled_kernel(const float* __restric
   const int64_t g = grp - grp0;
   const int64_t G = ((int64_t)N + kTileRows - 1) / kTileRows;
   const __amdgpu_buffer_rsrc_t qrs =
-      rsrc_of(w + g * KP * kTilePieceBytes, (uint32_t)KP * kTilePieceBytes);
+      buffer_rsrc(w + g * KP * kTilePieceBytes, (uint32_t)KP * kTilePieceBytes);
   const __amdgpu_buffer_rsrc_t srs =
-      rsrc_of(w + G * KP * kTilePieceBytes + g * KP * kTileScaleBytes,
+      buffer_rsrc(w + G * KP * kTilePieceBytes + g * KP * kTileScaleBytes,
               (uint32_t)KP * kTileScaleBytes);
-  const __amdgpu_buffer_rsrc_t xrs = rsrc_of(x, (uint32_t)((int64_t)M * K * 4));
+  const __amdgpu_buffer_rsrc_t xrs = buffer_rsrc(x, (uint32_t)((int64_t)M * K * 4));
   float* xs = smem + wave * (MT * XCH);
 
   float acc[MT];
@@ -173,7 +163,7 @@ __global__ __launch_bounds__(1024) void gemv_tiled_kernel(const float* __restric
   if constexpr (kSwi) {
     float u = 0.0f;
     for (int wi = 0; wi < wpg; ++wi) u += red[((wpg + wi) * MT + m) * 16 + rr];
-    y[(int64_t)m * N + n] = silu_mul_t(s, u);
+    y[(int64_t)m * N + n] = silu_mul(s, u);
   } else {
     y[(int64_t)m * N + n] = s + (bias ? bias_at(bias, bias_bf16, n) : 0.0f);
   }

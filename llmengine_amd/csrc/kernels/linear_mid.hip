@@ -56,25 +56,6 @@ constexpr int kWN = 4;  // waves along the rows
 constexpr int kWK = 2;  // waves along K
 constexpr int kNT = 64 * kWN * kWK;
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* base, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes,
-                                           0x00020000);
-}
-
-__device__ __forceinline__ uint32_t top_halves(uint32_t lo_word, uint32_t hi_word) {
-  return __builtin_amdgcn_perm(hi_word, lo_word, 0x07060302u);
-}
-
-// 8 int8 quants (two dwords) -> 8 bf16 (exact).
-__device__ __forceinline__ bf16x8 quants_to_bf16(uint32_t q0, uint32_t q1) {
-  u32x4 o;
-  o.x = top_halves(__builtin_bit_cast(uint32_t, q_at(q0, 0)), __builtin_bit_cast(uint32_t, q_at(q0, 1)));
-  o.y = top_halves(__builtin_bit_cast(uint32_t, q_at(q0, 2)), __builtin_bit_cast(uint32_t, q_at(q0, 3)));
-  o.z = top_halves(__builtin_bit_cast(uint32_t, q_at(q1, 0)), __builtin_bit_cast(uint32_t, q_at(q1, 1)));
-  o.w = top_halves(__builtin_bit_cast(uint32_t, q_at(q1, 2)), __builtin_bit_cast(uint32_t, q_at(q1, 3)));
-  return __builtin_bit_cast(bf16x8, o);
-}
-
 // The parts of 4 activations as packed bf16 (two dwords a part).  PARTS 3: hi / mid
 // / lo by truncation, exact for every finite x (Inf carried in hi, NaN in all), as
 // the MFMA decode splits them; PARTS 1: one rounding to nearest even.
@@ -111,11 +92,6 @@ __device__ __forceinline__ void split_x(const f32x4 x, u32x2 (&out)[PARTS]) {
       out[2][p] = top_halves(lb[2 * p], lb[2 * p + 1]);
     }
   }
-}
-
-// silu(g) * u with the reference's operation order (cpu_kernels.cpp:848-858).
-__device__ __forceinline__ float silu_mul(float g, float u) {
-  return (g / (1.0f + expf(-g))) * u;
 }
 
 // Output segments of a launch: segment i owns the 16-row groups
@@ -187,7 +163,7 @@ __global__ __launch_bounds__(kNT, 2) void linear_mid_kernel(const float* __restr
   // blocks past KBE are zero.  (Loading whole fragments, a lane a token, costs a
   // cache line lookup per lane: 64 tokens' phases took 0.9 us each, MI355X.)
   auto swz = [](int b, int q) { return (q | (b << 2)) & 7; };
-  const __amdgpu_buffer_rsrc_t xrs = rsrc(x, (uint32_t)((int64_t)M * K * 4));
+  const __amdgpu_buffer_rsrc_t xrs = buffer_rsrc(x, (uint32_t)((int64_t)M * K * 4));
   const int xr = 2 * wave + (lane >> 5), xb = (lane >> 3) & 3, xq = (lane >> 1) & 3;
   const uint32_t xslot = (uint32_t)((xq * 16 + (xr ^ swz(xb, xq))) * 16 + (lane & 1) * 8);
   struct XStage {
@@ -505,7 +481,7 @@ __global__ __launch_bounds__(kNT, 2) void linear_mid_kernel(const float* __restr
   // Split K: partials by device-scope stores, their completion, the tile's
   // counter; the last workgroup resets the counter and adds the splits in order.
   const __amdgpu_buffer_rsrc_t prs =
-      rsrc(reinterpret_cast<uint8_t*>(partials) + (int64_t)blockIdx.x * nspl * REGION, nspl * REGION);
+      buffer_rsrc(reinterpret_cast<uint8_t*>(partials) + (int64_t)blockIdx.x * nspl * REGION, nspl * REGION);
   if (wk == 0) {
 #pragma unroll
     for (int rg = 0; rg < RG; ++rg)

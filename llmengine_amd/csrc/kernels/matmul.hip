@@ -29,15 +29,6 @@ namespace {
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef int v2i __attribute__((ext_vector_type(2)));
 
-__device__ __forceinline__ uint32_t top_halves(uint32_t lo_word, uint32_t hi_word) {
-  return __builtin_amdgcn_perm(hi_word, lo_word, 0x07060302u);
-}
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t mm_rsrc(const void* base, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes,
-                                           0x00020000);
-}
-
 // MFMA kernel (3 and more rows of A, up to 64 a workgroup), fp32-exact operands.
 //
 // A block of B holds 32 columns of one k, so its scale cannot leave the K sum; it goes
@@ -353,7 +344,7 @@ __global__ __launch_bounds__(kMfNT, 2) void matmul_q8_0_mfma_kernel(
     const unsigned nspl = gridDim.y;
     const uint32_t mine = (uint32_t)(wave * 64 + lane) * 16;
     const __amdgpu_buffer_rsrc_t prs =
-        mm_rsrc(reinterpret_cast<uint8_t*>(partials) + (int64_t)bx * nspl * REGION, nspl * REGION);
+        buffer_rsrc(reinterpret_cast<uint8_t*>(partials) + (int64_t)bx * nspl * REGION, nspl * REGION);
     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, sum_of(wave)), prs,
                                            by * REGION + mine, 0, SC1);
     uint32_t* const counter = counters + (size_t)bx * kCounterStride;
@@ -457,8 +448,8 @@ __global__ __launch_bounds__(kLnNT) void matmul_q8_0_half_kernel(
   const uint32_t offx = cb + 16 * h + mis;
   const uint32_t offu = cb + 16 * h + (mis ? 0u : 16u);
   // Buffer resources: B rows past K and A entries past M or K read as zeros.
-  const __amdgpu_buffer_rsrc_t brs = mm_rsrc(b, (uint32_t)K * row_bytes);
-  const __amdgpu_buffer_rsrc_t ars = mm_rsrc(a, (uint32_t)M * (uint32_t)K * 4u);
+  const __amdgpu_buffer_rsrc_t brs = buffer_rsrc(b, (uint32_t)K * row_bytes);
+  const __amdgpu_buffer_rsrc_t ars = buffer_rsrc(a, (uint32_t)M * (uint32_t)K * 4u);
   const int m0 = blockIdx.z * MR;
   const int nbatches = (K + BATCH - 1) / BATCH;
   const int bt0 = blockIdx.y * batches_per_split;
@@ -532,7 +523,7 @@ __global__ __launch_bounds__(kLnNT) void matmul_q8_0_half_kernel(
   const bool split = gridDim.y > 1;
   const uint32_t region = MR * kLnCols;  // floats of one workgroup's partial sums
   const __amdgpu_buffer_rsrc_t prs =
-      mm_rsrc(partials, split ? (uint32_t)((tile + 1) * gridDim.y * region * 4) : 0u);
+      buffer_rsrc(partials, split ? (uint32_t)((tile + 1) * gridDim.y * region * 4) : 0u);
 #pragma unroll
   for (int r = 0; r < MR; ++r) {
     float* mine = red + (wave * 64 + lane) * 16;

@@ -107,6 +107,32 @@ __device__ __forceinline__ float q_at(uint32_t word, int j) {
   return (float)(int8_t)(word >> (8 * j));
 }
 
+// bf16 pair from the upper 16 bits of two fp32 bit patterns (lo in bits 0-15).
+__device__ __forceinline__ uint32_t top_halves(uint32_t lo_word, uint32_t hi_word) {
+  return __builtin_amdgcn_perm(hi_word, lo_word, 0x07060302u);
+}
+
+// 8 int8 quants (two dwords) -> 8 bf16 (exact).
+__device__ __forceinline__ bf16x8 quants_to_bf16(uint32_t q0, uint32_t q1) {
+  u32x4 o;
+  o.x = top_halves(__builtin_bit_cast(uint32_t, q_at(q0, 0)), __builtin_bit_cast(uint32_t, q_at(q0, 1)));
+  o.y = top_halves(__builtin_bit_cast(uint32_t, q_at(q0, 2)), __builtin_bit_cast(uint32_t, q_at(q0, 3)));
+  o.z = top_halves(__builtin_bit_cast(uint32_t, q_at(q1, 0)), __builtin_bit_cast(uint32_t, q_at(q1, 1)));
+  o.w = top_halves(__builtin_bit_cast(uint32_t, q_at(q1, 2)), __builtin_bit_cast(uint32_t, q_at(q1, 3)));
+  return __builtin_bit_cast(bf16x8, o);
+}
+
+// Buffer resource over [base, base + bytes): loads past the end return zero.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_rsrc(const void* base, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes,
+                                           0x00020000);
+}
+
+// silu(g) * u with the reference's operation order (cpu_kernels.cpp:848-858).
+__device__ __forceinline__ float silu_mul(float g, float u) {
+  return (g / (1.0f + expf(-g))) * u;
+}
+
 // Round-to-nearest-even fp32 -> bf16 of two values packed into one dword
 // (lo in bits 0-15).  Inputs here are finite.
 __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
