@@ -86,6 +86,10 @@ MfGrid mf_grid(int M, int N, int K) {
   // A tile's last workgroup adds its splits alone: few columns of very long K are faster
   // with fewer (4 x 480 x 32608 18.9 us with 127, 15.2 with 48; 16 take 21).
   if (mf_handoff(M) && s > 48) s = 48;
+  // Many rows over few columns stay without a workspace, so that a capture that reserved
+  // none is accepted: from 512 tiles of 8 rows x 256 columns on, as many as fill the GPU
+  // with one split on the fp32 kernel that took these calls first.
+  if (M > 64 && (int64_t)((N + 255) / 256) * ((M + 7) / 8) >= 512) s = 1;
   if (s < 1) s = 1;
   g.steps_per_split = (steps + s - 1) / s;
   g.splits = (unsigned)((steps + g.steps_per_split - 1) / g.steps_per_split);

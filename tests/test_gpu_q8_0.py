@@ -879,6 +879,29 @@ def test_matmul_unaligned_rows_take_one_launch(dev, orc, M, N, K):
         assert_bitexact(to_host(out), to_host(eager), "replay vs eager")
 
 
+def test_matmul_many_unaligned_rows_capture_without_a_reservation(dev):
+    """Many rows over few columns take no workspace: a stream that reserved none captures
+    them."""
+    import torch
+    M, N, K = 4100, 96, 1056
+    note(f"matmul many unaligned rows M={M} N={N} K={K}")
+    abuf = to_dev(acts(525, M * K + 4, 1).reshape(-1), dev)
+    db = to_dev(weight(526, K, N), dev)
+    out, eager = empty_f32((M, N), dev), empty_f32((M, N), dev)
+    capi.matmul(abuf[1:], db, eager, M, N, K)
+    st = own_stream()
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=st):
+        capi.matmul(abuf[1:], db, out, M, N, K, stream=st)
+    for _ in range(3):
+        out.fill_(float("nan"))
+        g.replay()
+        torch.cuda.synchronize()
+        assert_bitexact(to_host(out), to_host(eager), "replay vs eager")
+    assert capi.workspace_info(st) == (0, 0, 0)
+
+
 @pytest.mark.parametrize("M,N,K", [(3, 96, 512), (8, 1024, 4096), (20, 160, 96), (40, 64, 1056)])
 def test_matmul_mfma_tiny_activations(dev, M, N, K):
     """Rows of A down to the smallest normal magnitudes keep fp32 accuracy (products with
