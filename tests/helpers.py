@@ -165,4 +165,5 @@ def slower_by(fn, than, rounds: int = 9) -> float:
             b.record()
             b.synchronize()
             best[i] = min(best[i], a.elapsed_time(b))
+    note(f"time ratio {best[0] / best[1]:.3f}")
     return best[0] / best[1]
